@@ -99,7 +99,7 @@ __device__ __forceinline__ void load8_any(const void* base, int dt, int64_t i, i
 // target count of label `act` for 8 cells starting at cell0
 __device__ __forceinline__ void target8(const BwdArgs& a, int64_t b, int64_t act, int64_t cell0,
                                         float t[8]) {
-  if (a.counts == nullptr) {
+  if (a.counts.p == nullptr) {
     const uint4 lv = *(const uint4*)(a.lab16 + b * a.HWp + cell0);
     const uint32_t w[4] = {lv.x, lv.y, lv.z, lv.w};
 #pragma unroll
@@ -108,7 +108,7 @@ __device__ __forceinline__ void target8(const BwdArgs& a, int64_t b, int64_t act
       t[2 * k + 1] = (int64_t)(w[k] >> 16) == act ? 1.f : 0.f;
     }
   } else {
-    counts8_f(a.counts, a.cw, (b * a.GT_total + act) * a.HWp + cell0, t);
+    counts8_f(a.counts.p, a.counts.cw, a.counts.at(b, act, cell0), t);
   }
 }
 
@@ -613,12 +613,12 @@ __device__ __forceinline__ void lut_load(const BwdArgs& a, int64_t it, int64_t n
         m.z[u] = make_uint4(w[0], w[1], w[2], w[3]);
       }
       if constexpr (CNT) {
-        const int64_t e = (b * a.GT_total + actc) * a.HWp + c;
-        if (a.cw == 1) {
-          const uint2 cv = *(const uint2*)(a.counts + e);
+        const int64_t e = a.counts.at(b, actc, c);
+        if (a.counts.cw == 1) {
+          const uint2 cv = *(const uint2*)(a.counts.p + e);
           m.lab[u] = make_uint4(cv.x, cv.y, 0, 0);
         } else {
-          m.lab[u] = *(const uint4*)(a.counts + 2 * e);
+          m.lab[u] = *(const uint4*)(a.counts.p + 2 * e);
         }
       } else {
         m.lab[u] = *(const uint4*)(a.lab16 + b * a.HWp + c);
@@ -658,7 +658,7 @@ __device__ __forceinline__ void lut_compute_store(const BwdArgs& a, const LutIte
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const uint32_t lw[4] = {m.lab[u].x, m.lab[u].y, m.lab[u].z, m.lab[u].w};
-        const uint32_t n = a.cw == 1 ? (lw[k >> 2] >> ((k & 3) * 8)) & 0xFFu
+        const uint32_t n = a.counts.cw == 1 ? (lw[k >> 2] >> ((k & 3) * 8)) & 0xFFu
                                      : (lw[k >> 1] >> ((k & 1) * 16)) & 0xFFFFu;
         t[k] = matched ? (float)n : 0.f;
       }

@@ -135,6 +135,7 @@ bool make_dims(const ml_shape* s, int64_t background_index, int dtype, Dims& d,
   d.ks_max = nsteps / 4 > 1 ? nsteps / 4 : 1;
   d.counts_mode = d.s > 1;
   d.cw = d.s >= 16 ? 2 : 1;  // u8 counts overflow at s*s >= 256
+  d.crows = d.GT_total + 1;  // every label, and the pixels of no column
   // row-tile pairs stream 16-byte aligned rows (HW % 8 == 0) with 32-bit
   // element offsets within a pair's 32 rows
   d.pair_ok = dtype == ML_BF16 && !d.counts_mode && d.rows == 16 && d.HW % 8 == 0 && d.HW >= 8 &&
@@ -218,8 +219,7 @@ Layout make_layout(const Dims& d, bool force_masks, const CostPlan& pl) {
     o = align256(o + bytes);
     return r;
   };
-  L.lab16 = take(d.counts_mode ? 0 : (size_t)d.B * d.HWp * 2);
-  L.counts = take(d.counts_mode ? (size_t)d.B * d.GT_total * d.HWp * d.cw : 0);
+  L.targets = take(target_bytes(d));
   L.pbits = take((size_t)d.B * prep_blocks(d) * kPresWords * 4);
   L.ncols = take((size_t)d.B * 4);
   L.colmap = take((size_t)d.B * d.nslot * 4);
@@ -377,6 +377,13 @@ static void side_release(const SideStream& ss) {
   g_side_free.push_back(ss);
 }
 
+// The preparation's compact targets at `p` (target_bytes(d)).
+static void set_targets(PrepArgs& pa, const Dims& d, void* p) {
+  pa.lab16 = d.counts_mode ? nullptr : (uint16_t*)p;
+  pa.counts = CountTiles{d.counts_mode ? (const uint8_t*)p : nullptr, d.cw, count_blocks(d.HW), d.crows};
+  pa.rest = d.GT_total;
+}
+
 // Shared forward: prep -> cost -> assign (-> layer).
 int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
                  const void* mask_logits, const int64_t* mask_targets, int cls_dtype,
@@ -441,10 +448,8 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   PrepArgs pa;
   pa.fill = prep_fill;
   pa.targets = mask_targets;
-  // with a saved state the compact labels go straight into it (the backward reuses them)
-  pa.lab16 = (uint16_t*)(saved && !d.counts_mode ? sv + SL.lab16 : w + L.lab16);
-  pa.counts = (uint8_t*)(w + L.counts);
-  pa.cw = d.cw;
+  // with a saved state the compact targets go straight into it (the backward reuses them)
+  set_targets(pa, d, saved ? sv + SL.targets : w + L.targets);
   pa.pbits = (uint32_t*)(w + L.pbits);
   pa.nblk = prep_blocks(d);
   const int64_t void_idx =
@@ -485,8 +490,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   CostArgs ca;
   ca.logits = mask_logits;
   ca.lab16 = pa.lab16;
-  ca.counts = d.counts_mode ? pa.counts : nullptr;
-  ca.cw = d.cw;
+  ca.counts = pa.counts;
   ca.ncols = pa.ncols;
   ca.colmap = pa.colmap;
   ca.sched = pa.sched;
@@ -918,8 +922,7 @@ size_t ml_mask_matching_backward_workspace_size(const ml_shape* s, const ml_para
   std::string err;
   if (!make_dims(s, p->background_index, mask_dtype, d, err)) return 0;
   size_t o = 0;
-  o = align256(o + (d.counts_mode ? 0 : (size_t)d.B * d.HWp * 2));
-  o = align256(o + (d.counts_mode ? (size_t)d.B * d.GT_total * d.HWp * d.cw : 0));
+  o = align256(o + target_bytes(d));
   o = align256(o + (size_t)d.B * 4);                // ncols
   o = align256(o + (size_t)d.B * d.nslot * 4);      // colmap
   o = align256(o + (size_t)d.B * d.GT_out * 4);     // slot_of_col
@@ -956,9 +959,7 @@ int ml_mask_matching_backward(const ml_shape* s, const ml_params* p, const float
     return r;
   };
   PrepArgs pa;
-  pa.lab16 = (uint16_t*)(w + take(d.counts_mode ? 0 : (size_t)d.B * d.HWp * 2));
-  pa.counts = (uint8_t*)(w + take(d.counts_mode ? (size_t)d.B * d.GT_total * d.HWp * d.cw : 0));
-  pa.cw = d.cw;
+  set_targets(pa, d, w + take(target_bytes(d)));
   pa.pbits = nullptr;  // labels only
   pa.ncols = (int*)(w + take((size_t)d.B * 4));
   pa.colmap = (int*)(w + take((size_t)d.B * d.nslot * 4));
@@ -969,9 +970,8 @@ int ml_mask_matching_backward(const ml_shape* s, const ml_params* p, const float
   pa.GT_total = d.GT_total; pa.GT_out = d.GT_out; pa.bg = d.bg; pa.nslot = d.nslot;
   pa.sched = nullptr;
   pa.L = d.L; pa.rtiles = d.rtiles; pa.plan = CostPlan{};
-  // the forward's saved state holds the compact label map for s == 1
-  const bool saved_labels = saved && !d.counts_mode;
-  if (saved_labels) pa.lab16 = (uint16_t*)(sv + SL.lab16);
+  // the forward's saved state holds the compact targets
+  if (saved) set_targets(pa, d, (void*)(sv + SL.targets));
   else if (d.B > 0 && (rc = launch_prep(pa, d, st))) return rc;
 
   const int64_t void_idx =
@@ -990,9 +990,8 @@ int ml_mask_matching_backward(const ml_shape* s, const ml_params* p, const float
   BwdArgs ba;
   ba.logits = mask_logits;
   ba.dtype = mask_dtype;
-  ba.lab16 = d.counts_mode ? nullptr : pa.lab16;
-  ba.counts = d.counts_mode ? pa.counts : nullptr;
-  ba.cw = d.cw;
+  ba.lab16 = pa.lab16;
+  ba.counts = pa.counts;
   ba.pred_to_gt = pred_to_gt;
   ba.stats = stats;
   ba.list = grad_prefilled ? (const int*)(sv + SL.list) : nullptr;
@@ -1058,7 +1057,8 @@ bool dense_plan(const ml_dense_shape* s, bool dice, bool backward, DensePlan& P,
   d.HWp = ceil_div(d.HW, kStep) * kStep;
   d.counts_mode = d.s > 1;
   d.cw = d.s >= 16 ? 2 : 1;
-  P.tgt_bytes = align256(d.counts_mode ? (size_t)d.B * d.C * d.HWp * d.cw : (size_t)d.B * d.HWp * 2);
+  d.crows = d.C;
+  P.tgt_bytes = align256(target_bytes(d));
   P.partial_off = P.tgt_bytes;
   P.total = P.tgt_bytes + (backward ? 0 : align256(dense_partials_bytes(d.L, d.B, d.C, d.HW, dice)));
   return true;
@@ -1069,15 +1069,13 @@ int dense_prep(const DensePlan& P, const int64_t* targets, unsigned char* w, Den
   const Dims& d = P.d;
   PrepArgs pa{};
   pa.targets = targets;
-  pa.lab16 = d.counts_mode ? nullptr : (uint16_t*)w;
-  pa.counts = d.counts_mode ? (uint8_t*)w : nullptr;
-  pa.cw = d.cw;
+  set_targets(pa, d, w);
+  pa.rest = -1;  // one row per class
   pa.pbits = nullptr;
   pa.B = d.B; pa.H = d.H; pa.W = d.W; pa.Ht = d.Ht; pa.Wt = d.Wt; pa.s = d.s; pa.HWp = d.HWp;
   pa.GT_total = d.C; pa.GT_out = d.C; pa.bg = d.C;
   a.lab16 = pa.lab16;
   a.counts = pa.counts;
-  a.cw = d.cw;
   a.L = d.L; a.B = d.B; a.C = d.C; a.HW = d.HW; a.HWp = d.HWp; a.HtWt = d.Ht * d.Wt;
   a.N2 = (float)d.N2;
   if (d.B == 0) return ML_OK;

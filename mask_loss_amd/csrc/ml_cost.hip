@@ -426,7 +426,7 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
         const uint32_t N2i = (uint32_t)a.N2;
         const uint32_t act = colL[nt] & 0xFFFFu;
         uint32_t n[8];
-        counts8_u32(a.counts, CNT == 2 ? 2 : 1, (b * a.GT_total + act) * a.HWp + cell0, n);
+        counts8_u32(a.counts.p, CNT == 2 ? 2 : 1, a.counts.at(b, act, cell0), n);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           uint32_t v[2], p[2];

@@ -100,7 +100,7 @@ __device__ __forceinline__ void dense_store8(void* base, int dt, int64_t i, cons
 // counts of class c for 8 cells starting at cell0
 __device__ __forceinline__ void dense_count8(const DenseArgs& a, int64_t b, int64_t c,
                                              int64_t cell0, float n[8]) {
-  if (a.counts == nullptr) {
+  if (a.counts.p == nullptr) {
     const uint4 lv = *(const uint4*)(a.lab16 + b * a.HWp + cell0);
     const uint32_t w[4] = {lv.x, lv.y, lv.z, lv.w};
     const uint32_t c32 = (uint32_t)c;
@@ -110,7 +110,7 @@ __device__ __forceinline__ void dense_count8(const DenseArgs& a, int64_t b, int6
       n[2 * k + 1] = (w[k] >> 16) == c32 ? 1.f : 0.f;
     }
   } else {
-    counts8_f(a.counts, a.cw, (b * a.C + c) * a.HWp + cell0, n);
+    counts8_f(a.counts.p, a.counts.cw, a.counts.at(b, c, cell0), n);
   }
 }
 

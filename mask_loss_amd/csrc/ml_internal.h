@@ -172,32 +172,59 @@ struct Dims {
   int nslot;                 // 16 * NT
   bool counts_mode;          // s > 1: per-cell count operands
   int cw;                    // bytes per count: 1 (u8, s <= 15) or 2 (u16, s >= 16)
+  int64_t crows;             // count rows per 64-cell block (see CountTiles)
   bool pair_ok;              // bf16 label maps whose rows suit the row-tile pair kernel
 };
+
+// Per-cell label counts of s > 1 targets (the reference's count tensor,
+// src/cuda/utils.cuh:6-36) in blocks of 64 cells: [B][ceil(HW / 64)][rows][64]
+// of cw bytes, row r < GT_total holding label r and, on the matching path, row
+// GT_total the pixels of no output column (labels outside [0, GT_total) and
+// the background slot; that slot's own row then stays zero).  A block holds
+// every label of 64 cells side by side, so the contraction reads its operand
+// tile (many labels, the same cells) as one run, and one label's counts along
+// the cells (the backward) come in runs of 64.
+constexpr int kCountCells = 64;
+__host__ __device__ inline int64_t count_blocks(int64_t HW) { return (HW + kCountCells - 1) / kCountCells; }
+struct CountTiles {
+  const uint8_t* p;   // null: label map targets (s == 1)
+  int cw;             // bytes per count
+  int64_t nb, rows;   // blocks per image, rows per block
+  // element index of (image b, row r, cell)
+  __host__ __device__ int64_t at(int64_t b, int64_t r, int64_t cell) const {
+    return ((b * nb + (cell >> 6)) * rows + r) * kCountCells + (cell & (kCountCells - 1));
+  }
+};
+inline size_t count_bytes(int64_t B, int64_t HW, int64_t rows, int cw) {
+  return (size_t)(B * count_blocks(HW) * rows) * kCountCells * cw;
+}
 
 bool make_dims(const ml_shape* s, int64_t background_index, int dtype, Dims& d, std::string& err);
 int cost_rt_for(int dtype, int NT);
 
 // Byte offsets inside the forward's saved state (see ml_saved_bytes): the
 // float head (per-query stats, then the per-layer block), the matched-row list
-// (int32 count, then (l*B+b)*Q+q of every matched row, ascending), and for
-// s == 1 the compact label map lab16 [B][HWp].
+// (int32 count, then (l*B+b)*Q+q of every matched row, ascending), and the
+// compact targets: for s == 1 the label map lab16 [B][HWp], else the counts.
 struct SavedLayout {
-  size_t stats, layer, list, lab16, total;
+  size_t stats, layer, list, targets, total;
 };
+inline size_t target_bytes(const Dims& d) {
+  return d.counts_mode ? count_bytes(d.B, d.HW, d.crows, d.cw) : (size_t)d.B * d.HWp * 2;
+}
 inline SavedLayout saved_layout(const Dims& d) {
   SavedLayout S;
   S.stats = 0;
   S.layer = (size_t)d.LB * d.Q * ML_STATS * 4;
   S.list = align256(S.layer + (size_t)d.L * ML_LAYERS * 4);
-  S.lab16 = align256(S.list + (size_t)(1 + d.LB * d.Q) * 4);
-  S.total = align256(S.lab16 + (d.counts_mode ? 0 : (size_t)d.B * d.HWp * 2));
+  S.targets = align256(S.list + (size_t)(1 + d.LB * d.Q) * 4);
+  S.total = align256(S.targets + target_bytes(d));
   return S;
 }
 
 // Byte offsets inside the caller's workspace.
 struct Layout {
-  size_t lab16, counts, pbits, ncols, colmap, slot_of_col, sched, partials, rowsum,
+  size_t targets, pbits, ncols, colmap, slot_of_col, sched, partials, rowsum,
       sep, tot, tot64, rowIT, rowstat, img, mrows, layer, done, total;
 };
 // Workspace layout for the cost plan `pl` (its float_total / slot_total size
@@ -227,10 +254,10 @@ struct FillSlice {
 
 struct PrepArgs {
   const int64_t* targets;
-  uint16_t* lab16;
-  uint8_t* counts;       // s > 1: [B][GT_total][HWp] counts of cw bytes each
+  uint16_t* lab16;       // s == 1
+  CountTiles counts{};   // s > 1 (its p is written)
+  int64_t rest = -1;     // count row of the pixels of no column, or -1: none kept
   FillSlice fill;        // done by extra workgroups of the column pass
-  int cw = 1;
   // forward only (else null): per preparation workgroup, kPresWords words of
   // presence bits of its GT labels, [B][nblk][kPresWords]; every word is
   // rewritten on each call, so nothing needs clearing first
@@ -262,8 +289,7 @@ struct PrepArgs {
 struct CostArgs {
   const void* logits;
   const uint16_t* lab16;
-  const uint8_t* counts;  // s > 1: [B][GT_total][HWp] counts of cw bytes each
-  int cw;
+  CountTiles counts;      // s > 1
   const int* ncols;
   const int* colmap;
   const int* sched;  // device schedule (see CostPlan)
@@ -362,8 +388,7 @@ struct BwdArgs {
   const void* logits;
   int dtype;
   const uint16_t* lab16;
-  const uint8_t* counts;  // s > 1: [B][GT_total][HWp] counts of cw bytes each
-  int cw;
+  CountTiles counts;      // s > 1
   const int64_t* pred_to_gt;
   const float* stats;     // per-query stats or null
   const int* list;        // matched-row list (count, rows): only these rows are written
@@ -392,8 +417,7 @@ struct DenseArgs {
   const void* logits;
   int dtype;
   const uint16_t* lab16;   // s == 1: label per cell (0xFFFF outside [0, C))
-  const uint8_t* counts;   // s > 1: [B][C][HWp] per-cell counts of cw bytes each
-  int cw;
+  CountTiles counts;       // s > 1, one row per class
   int64_t L, B, C, HW, HWp, HtWt;
   float N2;
   ElemParams ep;           // focal terms (sigmoid CE)
@@ -509,9 +533,9 @@ __device__ inline void fill_slice(const FillSlice& f, int64_t blk) {
 int launch_any_equal(const int64_t* x, int64_t n, int64_t value, int32_t* flag, hipStream_t st);
 int launch_stream_read(const void* p, int64_t n16, uint32_t* out, int grid, hipStream_t st);
 
-// Counts of one label at 8 consecutive cells starting at element `idx` of the
-// count tensor: u8 (cw == 1) or u16 (cw == 2).  idx is a multiple of 8, so the
-// run is one aligned 8- or 16-byte load.  The reference's uint8 counts
+// Counts of one label at 8 consecutive cells from element `idx` of the count
+// tiles (CountTiles::at): u8 (cw == 1) or u16 (cw == 2).  The first cell is a
+// multiple of 8, so the run is one aligned 8- or 16-byte load.  The reference's uint8 counts
 // (src/cuda/utils.cuh:9) overflow for s >= 16; u16 holds up to s = 255.
 __device__ __forceinline__ void counts8_u32(const uint8_t* base, int cw, int64_t idx, uint32_t n[8]) {
   if (cw == 1) {

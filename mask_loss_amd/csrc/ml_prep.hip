@@ -2,13 +2,15 @@
 //
 //   s == 1 : u16 label per cell (labels outside [0, GT_total) -> 0xFFFF)
 //   s  > 1 : count of each label inside the s x s block of every cell
-//            (B, GT_total, HWp), the reference's count tensor
+//            (CountTiles), the reference's count tensor
 //            (src/cuda/utils.cuh:6-36); u8 for s <= 15, u16 for s >= 16
 //            (where the reference's uint8 counts overflow, utils.cuh:9)
 // plus, for the forward, which GTs have pixels (the reference's per-GT areas
 // of src/cuda/pw_mask.cu:391 are only ever tested against zero) and, per
 // image, the compacted list of output columns whose GT is non-empty, and the
 // cost schedule.
+#include <algorithm>
+
 #include "ml_internal.h"
 
 namespace ml {
@@ -304,10 +306,26 @@ __global__ __launch_bounds__(256) void prep_labels_kernel(PrepArgs a) {
   }
 }
 
-// s > 1: one thread per low-res cell, counts[b][lab][cell] (single writer).
-// grid (nblk, B)
-__global__ __launch_bounds__(256) void prep_counts_kernel(PrepArgs a) {
+// s > 1: the count tiles of 256 cells (four blocks), four threads per cell,
+// each taking every fourth target row of the cell's s x s block (S = s for the
+// unrolled forms 2 and 4, else 0).  grid (nblk, B)
+//
+// Bound by reading the labels (8 s^2 bytes per cell).  The counts of a block
+// are built in LDS (rc rows of 256 cells at a time; every row at once for up
+// to 160 rows of u8) and leave as one run of 16-byte words, zeros included,
+// so nothing is cleared first and no count is read back from memory.  A cell
+// whose pixels all carry one label, most of a natural label map, is one byte
+// store; other cells add their runs with LDS atomics.  8 maps of 1024 x 1024
+// at s = 4 with 61 rows: 22.6 us (67 MB read, 32 MB written, 4.4 TB/s; a copy
+// runs at 5.15), against 6.7 + 24.5 us for clearing the counts and adding to
+// them in memory pixel by pixel.
+constexpr int kCntCells = 256;
+constexpr int kCntThreads = 4 * kCntCells;
+constexpr size_t kCntLds = 40 * 1024;  // of the rows in LDS: three workgroups per CU
+template <int CW, int S>
+__global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, int rc, int vec) {
   __shared__ uint32_t pres[kPresWords];
+  extern __shared__ __align__(16) unsigned char tile[];  // [4 blocks][rc][64] of CW bytes
   const int64_t b = blockIdx.y;
   if (a.void_found && blockIdx.x == (unsigned)a.nblk) {  // the void check's own column
     if (b == 0) void_check(a);
@@ -315,37 +333,111 @@ __global__ __launch_bounds__(256) void prep_counts_kernel(PrepArgs a) {
   }
   const int64_t HW = a.H * a.W;
   const bool mark = a.pbits != nullptr;
-  if (mark) {
-    pres_clear(pres);
-    __syncthreads();
-  }
-  const int64_t cell = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cell < HW) {
-    const int64_t i = cell / a.W, j = cell % a.W;
-    int64_t prev = -1;
-    for (int64_t dy = 0; dy < a.s; ++dy) {
-      const int64_t* row = a.targets + (b * a.Ht + i * a.s + dy) * a.Wt + j * a.s;
-      for (int64_t dx = 0; dx < a.s; ++dx) {
-        const int64_t lab = row[dx];
-        if ((uint64_t)lab < (uint64_t)a.GT_total) {
-          const int64_t e = (b * a.GT_total + lab) * a.HWp + cell;
-          if (a.cw == 1) {
-            uint8_t* c = a.counts + e;
-            *c = (uint8_t)(*c + 1);
-          } else {
-            uint16_t* c = (uint16_t*)a.counts + e;
-            *c = (uint16_t)(*c + 1);
-          }
-          if (mark && lab != prev) pres_mark(pres, lab);
+  if (mark) pres_clear(pres);
+  const int tid = threadIdx.x, cl = tid >> 2, sub = tid & 3;
+  const int64_t cell = (int64_t)blockIdx.x * kCntCells + cl;
+  const bool in = cell < HW;
+  const int64_t s = S ? S : a.s;
+  const int64_t ci = in ? cell / a.W : 0, cj = in ? cell - ci * a.W : 0;
+  const int64_t* src = a.targets + (b * a.Ht + ci * s) * a.Wt + cj * s;
+  // row of a label in the tiles, -1 for none
+  auto row_of = [&](int64_t lab) -> int {
+    return (uint64_t)lab < (uint64_t)a.GT_total && (a.rest < 0 || lab != a.bg) ? (int)lab : (int)a.rest;
+  };
+  int64_t lab[S ? S : 1];
+  bool whole = false;  // every pixel of the cell carries lab[0]
+  bool first = true;   // ... and the wave's first cell does not already mark that label
+  if constexpr (S != 0) {
+    const bool act = in && sub < S;
+    if (act) {
+      const int64_t* p = src + sub * a.Wt;
+      if (vec) {
+#pragma unroll
+        for (int k = 0; k < S; k += 2) {
+          const longlong2 v = *(const longlong2*)(p + k);
+          lab[k] = v.x;
+          lab[k + 1] = v.y;
         }
-        prev = lab;
+      } else {
+#pragma unroll
+        for (int k = 0; k < S; ++k) lab[k] = p[k];
       }
     }
+    const int64_t l0 = __shfl(act ? lab[0] : 0, (tid & 63) & ~3, 64);
+    bool same = !act || lab[0] == l0;
+#pragma unroll
+    for (int k = 1; k < S; ++k) same = same && (!act || lab[k] == l0);
+    const uint64_t m = __ballot(same);
+    whole = in && ((m >> ((tid & 63) & ~3)) & 0xFull) == 0xFull;
+    const int64_t lw = __shfl(lab[0], 0, 64);
+    first = (tid & 63) == 0 || (m & 0xFull) != 0xFull || lab[0] != lw;
   }
-  if (mark) {
+  uint8_t* const out0 = (uint8_t*)a.counts.p;
+  for (int64_t r0 = 0; r0 < a.counts.rows; r0 += rc) {  // one round unless there are many rows
+    const int64_t nr = min((int64_t)rc, a.counts.rows - r0);
+    for (int i = tid; i < (int)(nr * kCntCells * CW / 16); i += kCntThreads)
+      ((uint4*)tile)[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
-    pres_store(a, pres, b);
+    // n pixels of one label in this thread's cell
+    auto add = [&](int64_t lb, uint32_t n, bool single) {
+      const bool valid = (uint64_t)lb < (uint64_t)a.GT_total;
+      if (mark && valid && r0 == 0 && !(single && !first)) pres_mark(pres, lb);
+      const int64_t r = (int64_t)row_of(lb) - r0;
+      if (r < 0 || r >= nr) return;
+      const uint32_t e = (uint32_t)(((cl >> 6) * nr + r) * kCountCells + (cl & (kCountCells - 1)));
+      if (single) {
+        if constexpr (CW == 1) tile[e] = (unsigned char)n;
+        else ((uint16_t*)tile)[e] = (uint16_t)n;
+      } else if constexpr (CW == 1) {
+        atomicAdd((uint32_t*)tile + (e >> 2), n << ((e & 3u) * 8u));
+      } else {
+        atomicAdd((uint32_t*)tile + (e >> 1), n << ((e & 1u) * 16u));
+      }
+    };
+    if constexpr (S != 0) {
+      if (whole) {
+        if (sub == 0) add(lab[0], S * S, true);
+      } else if (in && sub < S) {
+        uint32_t n = 1;
+#pragma unroll
+        for (int k = 1; k < S; ++k) {
+          if (lab[k] != lab[k - 1]) {
+            add(lab[k - 1], n, false);
+            n = 0;
+          }
+          ++n;
+        }
+        add(lab[S - 1], n, false);
+      }
+    } else if (in) {
+      for (int64_t dy = sub; dy < s; dy += 4) {
+        const int64_t* p = src + dy * a.Wt;
+        int64_t run = p[0];
+        uint32_t n = 1;
+        for (int64_t dx = 1; dx < s; ++dx) {
+          const int64_t v = p[dx];
+          if (v != run) {
+            add(run, n, false);
+            run = v;
+            n = 0;
+          }
+          ++n;
+        }
+        add(run, n, false);
+      }
+    }
+    __syncthreads();
+    // block k of this workgroup: rows [r0, r0 + nr) are one run of the tiles
+    const int per = (int)(nr * kCountCells * CW / 16);  // 16-byte words
+    const int64_t blk0 = (int64_t)blockIdx.x * (kCntCells / kCountCells);
+    for (int k = 0; k < kCntCells / kCountCells; ++k) {
+      if (blk0 + k >= a.counts.nb) break;
+      uint4* dst = (uint4*)(out0 + ((b * a.counts.nb + blk0 + k) * a.counts.rows + r0) * kCountCells * CW);
+      for (int i = tid; i < per; i += kCntThreads) dst[i] = ((const uint4*)tile)[k * per + i];
+    }
+    __syncthreads();
   }
+  if (mark) pres_store(a, pres, b);
 }
 
 // Workgroup 0: runs once every presence record of the preparation grid is
@@ -362,7 +454,7 @@ __global__ __launch_bounds__(1024) void prep_columns_kernel(PrepArgs a) {
 
 // Preparation workgroups per image (the presence records' count).
 int prep_blocks(const Dims& d) {
-  return (int)(d.counts_mode ? ceil_div(d.HW, 256) : ceil_div(d.HWp, 256 * 8));
+  return (int)(d.counts_mode ? ceil_div(d.HW, kCntCells) : ceil_div(d.HWp, 256 * 8));
 }
 
 int launch_prep(const PrepArgs& a, const Dims& d, hipStream_t st) {
@@ -376,9 +468,16 @@ int launch_prep(const PrepArgs& a, const Dims& d, hipStream_t st) {
   if (!d.counts_mode) {
     hipLaunchKernelGGL(prep_labels_kernel, grid, dim3(256), 0, st, a);
   } else {
-    rc = launch_fill_i32((int*)a.counts, 0, d.B * d.GT_total * d.HWp * d.cw / 4, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(prep_counts_kernel, grid, dim3(256), 0, st, a);
+    const size_t row = (size_t)kCntCells * d.cw;
+    const int rows = (int)std::max<int64_t>(1, std::min<int64_t>(a.counts.rows, (int64_t)(kCntLds / row)));
+    const size_t lds = rows * row;
+    // pairs of labels by one 16-byte load: even s keeps every row 16-byte aligned
+    const int vec = ((uintptr_t)a.targets & 15) == 0 ? 1 : 0;
+    const int S = d.s == 4 ? 4 : d.s == 2 ? 2 : 0;
+    if (d.cw == 2) hipLaunchKernelGGL((prep_counts_kernel<2, 0>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
+    else if (S == 4) hipLaunchKernelGGL((prep_counts_kernel<1, 4>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
+    else if (S == 2) hipLaunchKernelGGL((prep_counts_kernel<1, 2>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
+    else hipLaunchKernelGGL((prep_counts_kernel<1, 0>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
   }
   if ((rc = check_launch("prep"))) return rc;
   if (a.pbits) {
