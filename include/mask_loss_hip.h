@@ -91,8 +91,8 @@ typedef struct ml_params {
  * bytes, 256-byte aligned, written by ml_mask_matching_forward, read by
  * ml_mask_matching_backward).  Its head is float: per-query statistics
  * stats[(l*B+b)*Q+q][ML_STAT_*], then the per-layer block layer[l][ML_LAYER_*];
- * after them (internal layout) the list of matched query rows and, when the
- * targets are at the logit resolution, the compact label map, so the backward
+ * after them (internal layout) the list of matched query rows and the compact
+ * targets (label map, or per-cell counts of larger targets), so the backward
  * neither recomputes statistics nor re-reads the int64 label map. */
 enum {
   ML_STAT_S = 0,    /* uncertainty normaliser after normalise/clamp */
@@ -185,14 +185,14 @@ int ml_mask_matching_forward_polled(const ml_shape* s, const ml_params* p, int m
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  ml_mask_matching_forward with the same arguments and
  * results, minus workspace / workspace_bytes: its scratch is a static device
- * array of ML_NOALLOC_SCRATCH_BYTES (128 MiB) on each device it runs on, held
+ * array of ML_NOALLOC_SCRATCH_BYTES (256 MiB) on each device it runs on, held
  * until the process ends; the call itself allocates and frees nothing.
  * Shapes that need more scratch than that fail with ML_EUNSUPPORTED (the
  * headline shape, B=16, Q=200, 256x256, up to 100 GT columns, fits).  Calls
  * that overlap on one device share the array and race: serialise them (one
  * stream, or wait between calls).  The array's contents need no clearing
  * between calls. */
-#define ML_NOALLOC_SCRATCH_BYTES ((size_t)128 << 20)
+#define ML_NOALLOC_SCRATCH_BYTES ((size_t)256 << 20)
 int ml_mask_matching_forward_noalloc(const ml_shape* s, const ml_params* p, int mask_dtype,
                                      const void* mask_logits, const int64_t* mask_targets,
                                      int cls_dtype, const void* cls_logits,

@@ -114,68 +114,35 @@ constexpr int kFinCols = 2;      // GT_out <= 128
 constexpr int kFinColsWide = 4;  // GT_out <= 256, class logits streamed (NC = 0)
 constexpr int kFinClsBatch = 8;  // streamed class logits loaded per lane and batch
 constexpr int kFinClsWide = 20;  // C <= 1280 in registers with up to 64 kFinColsWide output columns
-constexpr int kFinSplits = 12;  // K-splits loaded per lane and batch
-constexpr int kFinSplits4 = 9;  // the same for four-plane partials (same registers)
+// K-splits loaded per lane and batch, by the planes of a partial (3 or 4)
+template <int NP>
+constexpr int kFinSplits = NP == 3 ? 12 : 9;
 
-// Sum the K-split partials k0, k0 + step, ... of slot s in split order.  The
-// loads of a batch are unconditional (indices clamped to the last split) so
-// all of them are in flight together.
-__device__ __forceinline__ void sum_splits(const RowPartials& rp, int s, int k0, int step,
-                                           float& v0, float& v1, float& v2) {
-  float a0 = 0.f, a1 = 0.f, a2 = 0.f;
-  for (int base = k0; base < rp.KS; base += kFinSplits * step) {
-    float x0[kFinSplits], x1[kFinSplits], x2[kFinSplits];
+// Sum the K-split partials k0, k0 + step, ... of slot s (NP planes) in split
+// order.  The loads of a batch are unconditional (indices clamped to the last
+// split) so all of them are in flight together.
+template <int NP>
+__device__ __forceinline__ void sum_splits(const RowPartials& rp, int s, int k0, int step, float (&v)[NP]) {
+  constexpr int NU = kFinSplits<NP>;
 #pragma unroll
-    for (int u = 0; u < kFinSplits; ++u) {
+  for (int i = 0; i < NP; ++i) v[i] = 0.f;
+  for (int base = k0; base < rp.KS; base += NU * step) {
+    float x[NP][NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
       const int ks = min(base + u * step, rp.KS - 1);
       const float* P = rp.p0 + (int64_t)ks * rp.ks_stride + s;
-      x0[u] = P[0];
-      x1[u] = P[rp.plane];
-      x2[u] = P[2 * rp.plane];
+#pragma unroll
+      for (int i = 0; i < NP; ++i) x[i][u] = P[i * rp.plane];
     }
 #pragma unroll
-    for (int u = 0; u < kFinSplits; ++u) {
+    for (int u = 0; u < NU; ++u) {
       if (base + u * step < rp.KS) {
-        a0 += x0[u];
-        a1 += x1[u];
-        a2 += x2[u];
+#pragma unroll
+        for (int i = 0; i < NP; ++i) v[i] += x[i][u];
       }
     }
   }
-  v0 = a0;
-  v1 = a1;
-  v2 = a2;
-}
-
-// The same for four-plane partials (slot sums of A_neg, A_pos, A_p, A_w).
-__device__ __forceinline__ void sum_splits4(const RowPartials& rp, int s, float& v0, float& v1,
-                                            float& v2, float& v3) {
-  float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-  for (int base = 0; base < rp.KS; base += kFinSplits4) {
-    float x0[kFinSplits4], x1[kFinSplits4], x2[kFinSplits4], x3[kFinSplits4];
-#pragma unroll
-    for (int u = 0; u < kFinSplits4; ++u) {
-      const int ks = min(base + u, rp.KS - 1);
-      const float* P = rp.p0 + (int64_t)ks * rp.ks_stride + s;
-      x0[u] = P[0];
-      x1[u] = P[rp.plane];
-      x2[u] = P[2 * rp.plane];
-      x3[u] = P[3 * rp.plane];
-    }
-#pragma unroll
-    for (int u = 0; u < kFinSplits4; ++u) {
-      if (base + u < rp.KS) {
-        a0 += x0[u];
-        a1 += x1[u];
-        a2 += x2[u];
-        a3 += x3[u];
-      }
-    }
-  }
-  v0 = a0;
-  v1 = a1;
-  v2 = a2;
-  v3 = a3;
 }
 
 // Exclusive prefix (UP) or suffix sum of v over the wave's lanes, in a fixed
@@ -274,37 +241,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC > 8 ? 3 
 #pragma unroll
     for (int j = 0; j < NG; ++j) zy[j] = cls_at<CDT>(a.cls_logits, zb + min(max(oy[j], (int64_t)0), C - 1));
   }
-  const int nsl = G + 1;  // GT columns + the ones column
+  const int nsl = G + 1;  // GT columns + slot G
   if (nsl <= 32) {
-    // two lanes per slot, each summing every other K-split; fixed-order combine
+    // bce numerator, I, T; slot G: the ones column.  Two lanes per slot, each
+    // summing every other K-split; fixed-order combine
     const int s = lane & 31, half = lane >> 5;
-    float v0 = 0.f, v1 = 0.f, v2 = 0.f;
-    if (s < nsl) sum_splits(rp, s, half, 2, v0, v1, v2);
-    v0 += __shfl_xor(v0, 32, 64);
-    v1 += __shfl_xor(v1, 32, 64);
-    v2 += __shfl_xor(v2, 32, 64);
+    float v[3] = {0.f, 0.f, 0.f};
+    if (s < nsl) sum_splits<3>(rp, s, half, 2, v);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] += __shfl_xor(v[i], 32, 64);
     if (half == 0 && s < nsl) {
-      sl[wave][0][s] = v0;
-      sl[wave][1][s] = v1;
-      sl[wave][2][s] = v2;
-    }
-  } else if (a.plan.planes[ci] == 3) {
-    for (int s = lane; s < nsl; s += 64) {
-      float v0 = 0.f, v1 = 0.f, v2 = 0.f;
-      sum_splits(rp, s, 0, 1, v0, v1, v2);
-      sl[wave][0][s] = v0;
-      sl[wave][1][s] = v1;
-      sl[wave][2][s] = v2;
+      sl[wave][0][s] = v[0];
+      sl[wave][1][s] = v[1];
+      sl[wave][2][s] = v[2];
     }
   } else {
-    // slot sums N, Pos, I, T of slots 0..G (slot G: cells of no column)
+    // slot sums N, Pos, I, T of slots 0..G (slot G: the pixels of no column)
     for (int s = lane; s < nsl; s += 64) {
-      float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
-      sum_splits4(rp, s, v0, v1, v2, v3);
-      sl[wave][0][s] = v0;
-      sl[wave][3][s] = v1;
-      sl[wave][1][s] = v2;
-      sl[wave][2][s] = v3;
+      float v[4];
+      sum_splits<4>(rp, s, 0, 1, v);
+      sl[wave][0][s] = v[0];
+      sl[wave][3][s] = v[1];
+      sl[wave][1][s] = v[2];
+      sl[wave][2][s] = v[3];
     }
     wave_sync();
     // bce numerator of slot g: the A_neg sums of every other slot (cells

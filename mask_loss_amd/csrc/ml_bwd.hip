@@ -101,11 +101,11 @@ __device__ __forceinline__ void target8(const BwdArgs& a, int64_t b, int64_t act
                                         float t[8]) {
   if (a.counts.p == nullptr) {
     const uint4 lv = *(const uint4*)(a.lab16 + b * a.HWp + cell0);
-    const uint32_t w[4] = {lv.x, lv.y, lv.z, lv.w};
+    const uint32_t w[4] = {lv.x, lv.y, lv.z, lv.w}, code = label_code(act);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      t[2 * k] = (int64_t)(w[k] & 0xFFFF) == act ? 1.f : 0.f;
-      t[2 * k + 1] = (int64_t)(w[k] >> 16) == act ? 1.f : 0.f;
+      t[2 * k] = (w[k] & 0xFFFF) == code ? 1.f : 0.f;
+      t[2 * k + 1] = (w[k] >> 16) == code ? 1.f : 0.f;
     }
   } else {
     counts8_f(a.counts.p, a.counts.cw, a.counts.at(b, act, cell0), t);
@@ -647,7 +647,7 @@ __device__ __forceinline__ void lut_compute_store(const BwdArgs& a, const LutIte
   const float cs = rc.mc * rc.sf;
   const float c2 = rc.dc * rc.kd * rc.num * a.N2;
   const float c3 = rc.dc * rc.kd * 2.f * rc.D;
-  const uint32_t act32 = matched ? (uint32_t)act : 0xFFFFFFFFu;
+  const uint32_t act32 = matched ? label_code(act) : 0xFFFFFFFFu;
 #pragma unroll
   for (int u = 0; u < kLutU; ++u) {
     const int64_t c = m.cell0 + u * kLutThreads * 8;

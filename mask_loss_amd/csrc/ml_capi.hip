@@ -115,7 +115,7 @@ bool make_dims(const ml_shape* s, int64_t background_index, int dtype, Dims& d,
   d.bg = background_index >= 0 ? background_index : d.GT_total;
   d.GT_out = d.GT_total - (skip ? 1 : 0);
   d.HWp = ceil_div(d.HW, kStep) * kStep;
-  const int64_t need = ceil_div(d.GT_out + 1, 16);  // + ones column
+  const int64_t need = ceil_div(d.GT_out + 1, 16);  // + slot G
   if (need <= 2) d.NT = 2;
   else if (need <= 7) d.NT = 7;
   else if (need <= 16) d.NT = 16;
@@ -123,8 +123,7 @@ bool make_dims(const ml_shape* s, int64_t background_index, int dtype, Dims& d,
     err = "more than 255 GT columns per image are not supported";
     return false;
   }
-  d.RT = cost_rt_for(dtype, d.NT);
-  d.rows = 16 * d.RT;
+  d.rows = 16;
   d.nslot = 16 * d.NT;
   d.rtiles = ceil_div(d.Q, d.rows);
   // a wave covers at least 4 K-steps of its task (small maps then split
@@ -135,10 +134,10 @@ bool make_dims(const ml_shape* s, int64_t background_index, int dtype, Dims& d,
   d.ks_max = nsteps / 4 > 1 ? nsteps / 4 : 1;
   d.counts_mode = d.s > 1;
   d.cw = d.s >= 16 ? 2 : 1;  // u8 counts overflow at s*s >= 256
-  d.crows = d.GT_total + 1;  // every label, and the pixels of no column
+  d.crows = d.GT_total + 2;  // every label, the pixels of no column, the ones column
   // row-tile pairs stream 16-byte aligned rows (HW % 8 == 0) with 32-bit
   // element offsets within a pair's 32 rows
-  d.pair_ok = dtype == ML_BF16 && !d.counts_mode && d.rows == 16 && d.HW % 8 == 0 && d.HW >= 8 &&
+  d.pair_ok = dtype == ML_BF16 && d.cw == 1 && d.rows == 16 && d.HW % 8 == 0 && d.HW >= 8 &&
               d.HW * 32 < ((int64_t)1 << 31);
   return true;
 }
@@ -161,8 +160,7 @@ CostPlan bound_cost_plan(const Dims& d) {
     p.float_base[c] = f;
     // row-tile pairs: up to max(slots, pairs) items of two row tiles each
     const int64_t items = c == 0 && d.pair_ok ? 2 * cap : cap;
-    p.planes[c] = c == 0 ? 3 : 4;  // the most any plan of this shape uses
-    if (c < p.nclass) f += items * p.planes[c] * d.rows * 16 * class_nt(c);
+    if (c < p.nclass) f += items * class_planes(c) * d.rows * 16 * class_nt(c);
   }
   p.float_total = f;
   p.slot_total = (int64_t)p.nclass * cap;
@@ -176,7 +174,7 @@ void pack_cost_plan(CostPlan& p, const Dims& d) {
     p.slot_base[c] = sl;
     p.float_base[c] = f;
     sl += cap;
-    f += (c == 0 && p.pair0 ? 2 * cap : cap) * p.planes[c] * d.rows * 16 * class_nt(c);
+    f += (c == 0 && p.pair0 ? 2 * cap : cap) * class_planes(c) * d.rows * 16 * class_nt(c);
   }
   p.float_total = f;
   p.slot_total = sl;
@@ -413,9 +411,9 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   const SavedLayout SL = saved_layout(d);
   unsigned char* sv = (unsigned char*)saved;
   float* stats = saved ? (float*)(sv + SL.stats) : nullptr;
-  const bool tab = mask_dtype == ML_BF16 && !d.counts_mode && g_use_lut && !force_masks;
+  const bool tab = mask_dtype == ML_BF16 && g_use_lut && !force_masks;
   CostPlan plan = make_cost_plan(d, mask_dtype, tab);
-  if (packed) fit_cost_plan(plan, d, force_masks, ws_bytes);
+  if (packed) fit_cost_plan(plan, d, force_masks, ws_bytes / 2);
   const Layout L = packed ? make_layout(d, force_masks, plan) : make_layout(d, force_masks);
   // point-sampling front end: presence records of the full label map after the layout
   const size_t pt_pbits = align256(L.total);
@@ -675,7 +673,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
 }
 
 // Workspace bytes of the matching forward with the packed cost plan fitted
-// to `budget` (what forward_impl with packed = true and ws_bytes = budget
+// to half of `budget` (what forward_impl with packed = true and ws_bytes = budget
 // needs) in `bytes`; the shape errors are
 // those of ml_mask_matching_forward (ML_EINVAL for malformed shapes,
 // ML_EUNSUPPORTED for shapes the assignment does not take).
@@ -687,9 +685,9 @@ int forward_packed_bytes(const ml_shape* s, const ml_params* p, int mask_dtype, 
   if (!make_dims(s, p->background_index, mask_dtype, d, err)) return fail(ML_EINVAL, err);
   if (!check_assign_dims(d, err)) return fail(ML_EUNSUPPORTED, err);
   const bool force_masks = p->force_unmatched_masks_to_empty != 0;
-  const bool tab = mask_dtype == ML_BF16 && !d.counts_mode && g_use_lut && !force_masks;
+  const bool tab = mask_dtype == ML_BF16 && g_use_lut && !force_masks;
   CostPlan plan = make_cost_plan(d, mask_dtype, tab);
-  fit_cost_plan(plan, d, force_masks, budget);
+  fit_cost_plan(plan, d, force_masks, budget / 2);
   bytes = make_layout(d, force_masks, plan).total;
   return ML_OK;
 }
@@ -878,7 +876,7 @@ int ml_point_sample_backward(int dtype, const void* grad_out, const float* coord
 int ml_point_labels(const int64_t* targets, const float* coords, int64_t B, int64_t Ht, int64_t Wt,
                     int64_t P, int64_t* labels, ml_stream_t stream) {
   if (B < 0 || Ht <= 0 || Wt <= 0 || P < 0) return fail(ML_EINVAL, "point labels: invalid shape");
-  return launch_point_labels(targets, coords, B, Ht, Wt, P, INT64_MAX, labels, nullptr, 0,
+  return launch_point_labels(targets, coords, B, Ht, Wt, P, INT64_MAX, -1, labels, nullptr, 0,
                              (hipStream_t)stream);
 }
 
@@ -1071,6 +1069,7 @@ int dense_prep(const DensePlan& P, const int64_t* targets, unsigned char* w, Den
   pa.targets = targets;
   set_targets(pa, d, w);
   pa.rest = -1;  // one row per class
+  pa.codes = 0;  // up to 65535 classes
   pa.pbits = nullptr;
   pa.B = d.B; pa.H = d.H; pa.W = d.W; pa.Ht = d.Ht; pa.Wt = d.Wt; pa.s = d.s; pa.HWp = d.HWp;
   pa.GT_total = d.C; pa.GT_out = d.C; pa.bg = d.C;

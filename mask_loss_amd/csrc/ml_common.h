@@ -20,7 +20,7 @@ typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kEps = 1e-12f;
-constexpr uint16_t kNoLabel = 0xFFFFu;
+constexpr uint16_t kNoLabel = 0xFFFFu;  // dense losses' label maps
 
 // ---------------------------------------------------------------------------
 // element type helpers

@@ -1,33 +1,54 @@
 // Pairwise sigmoid-BCE / dice cost as an MFMA contraction (gfx950).
 //
-// For one image b, query q and GT column g (label a, count n_g(cell)):
-//   bce_num[q,g] = sum_cell A_neg[q,cell] (N2 - n_g) + A_pos[q,cell] n_g
-//   I[q,g]       = sum_cell A_p[q,cell] n_g          (intersection)
-//   T[q,g]       = sum_cell A_w[q,cell] n_g          (weighted target mass)
-// with per-cell planes A_neg = w an mn cn, A_pos = w ap mp cp, A_p = w p, A_w = w.
-// An extra "ones" column (n = N2 everywhere) yields the row sums
-//   P = sum N2 w p (from the I plane) and S = sum N2 w (from the T plane).
+// For one image b and query q, with per-cell planes A_neg = w an mn cn, A_pos =
+// w ap mp cp, A_p = w p, A_w = w and the count n_g(cell) of GT column g:
+//   bce_num(g) = sum A_neg (N2 - n_g) + A_pos n_g, I(g) = sum A_p n_g, T(g) = sum A_w n_g
 // This is the reference's fused BCE+dice reduction (src/cuda/pw_mask.cu:52-308)
-// rewritten as (Q x K)(K x G) products: bce*S = base + Delta of pw_mask.cu:300
-// regrouped as sum_{cells} w cn (N2-n) + w cp n (both terms non-negative, so no
-// cancellation), I and T as pw_mask.cu:270-271, P and S as pw_mask.cu:140-141.
+// as (Q x K)(K x G) products, its base + Delta of :300 regrouped so that both
+// terms are non-negative (no cancellation); I and T as :270-271.  Class 0 (up to
+// 31 non-empty GTs) sums these three, and a ones column (slot G, n = N2
+// everywhere) gives the row sums P = sum N2 w p and S = sum N2 w (:140-141).
+// The wide classes sum the four planes per slot instead,
+//   N(s) = sum A_neg n_s, Pos(s) = sum A_pos n_s, I(s), T(s),
+// slot G holding the pixels of no column, and finalize rebuilds the bce numerator of
+// slot g as sum_{s != g} N(s) + Pos(g) and P, S as the sums of I and T over all
+// slots: their right operands are zero outside the tiles that a K-step's cells
+// touch, so those tiles' MFMAs are skipped.
 //
-// Work decomposition: one wave = 16*RT query rows of one image over a
-// contiguous range of 32-cell K-steps (K-split index = blockIdx.x); the four
-// waves of a workgroup take four consecutive (image, row-tile) tasks.  Each
-// image is handled by the kernel instance whose column-tile count NT matches
-// its number of non-empty GTs (+1 ones column), so accumulator registers are
-// sized to the image, not to the padded GT width.  Every wave writes its own
-// partial sums: partials[ks][lb][rtile][3][rows][nslot].
+// Operands are float16.  The planes are scaled by 2^9, split into two float16
+// terms for float32 and float16 logits (22 bits) and one for bf16 ones (11
+// bits).  The right operand is made of 16-bit integer ops: label codes of two
+// labels differ by at least 0x100 under xor, so a saturating subtraction of the
+// xor from 0x100 gives 0x100 (as a float16: 2^-16) where they agree and 0 elsewhere;
+// times 0x3C it is 1.0, which the two-term operands take (the matrix cores align a
+// subnormal factor's product without normalising it: with 2^-24, ten places
+// down, float32 sums were 1e-5 off; 2^-16 costs two places of a bf16 logit's
+// plane).  A u8 count n becomes 0x6400 + n = 1024 + n by one byte permute, then n.
+// The sums leave with all scales undone (powers of two).  A plane above
+// 127 (|z| > 127, or > 2558 at the smallest weight), inf or nan makes the wave's
+// sums non-finite; such a wave redoes its K-range with bf16 operands (3, 2 or 1
+// terms), which hold any float32.
+//
+// Bounds and measurements (MI355X; before: bf16 operands, 3 terms for float32
+// and 2 for float16, counts evaluated by formula from planes of u8 counts).  The
+// float32 kernels are bound by vector-ALU issue (~25 ops and 3 transcendental per
+// logit, a third of them the split): 10 M logits in 32 columns 28.1 -> 21.8 us, 33.6 M
+// against 4x targets 96 -> 58.6 us, the 16- and 7-tile launches of 39 M logits
+// 113 + 49 -> 88 + 39 us.  float32 sums are as far from 64 bits as before (4e-8 to
+// 1e-7), float16 and bf16 ones 3 to 10 times closer.
+//
+// Work decomposition: one wave = 16 query rows of one image over a
+// contiguous range of 32-cell K-steps; each image is handled by the kernel
+// instance whose column-tile count NT matches its number of non-empty GTs (+1
+// slot), so accumulator registers are sized to the image, not to the padded
+// GT width.
 //
 // Per-cell planes: bf16 logits take only 65536 values, so for them the four
 // planes are read from a per-workgroup LDS table built with the same float32
 // formulas (|z| in [2^-9, 64): one entry per bf16 value; |z| < 2^-9: the
-// z = 0 entry, which the bf16 planes of such z match to within one rounding
-// step; |z| >= 64, inf and nan read a NaN marker, and a wave whose sums come
-// out NaN redoes its K-range with the formulas).  Other dtypes
-// evaluate the formulas directly and split each plane into NS bf16 terms so
-// products keep float32 accuracy.
+// z = 0 entry, within 2^-9.5 of those; |z| >= 64, inf and nan read a NaN
+// marker, and a wave whose sums come out NaN redoes its K-range with the
+// formulas).  Other dtypes evaluate the formulas directly.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -36,19 +57,28 @@
 
 namespace ml {
 
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2_t as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2_t, v); }
+__device__ __forceinline__ uint32_t as_u32(u16x2_t v) { return __builtin_bit_cast(uint32_t, v); }
+
+constexpr float kPlaneScale = 512.f;  // of the float16 planes
+
+// terms per plane: float16 operands, and the bf16 operands of a redone range
 template <int DT>
 struct InTraits;
 template <>
 struct InTraits<ML_F32> {
-  static constexpr int kSplit = 3;  // hi/mid/lo bf16 terms: fp32-equivalent products
+  static constexpr int kTerms = 2, kRedo = 3;
 };
 template <>
 struct InTraits<ML_BF16> {
-  static constexpr int kSplit = 1;
+  static constexpr int kTerms = 1, kRedo = 1;
 };
 template <>
 struct InTraits<ML_F16> {
-  static constexpr int kSplit = 2;
+  static constexpr int kTerms = 2, kRedo = 2;
 };
 
 // ---- LUT geometry (bytes): positive block at 0, negative block at 32768 ----
@@ -61,30 +91,31 @@ constexpr uint32_t kLutNegOff = 32768;
 constexpr uint32_t kLutBytes = kLutNegOff + kLutBlock * 8;
 constexpr int kDepth = 4;  // K-steps of logits in flight per wave
 
-__device__ __forceinline__ uint32_t pk_lshl3_u16(uint32_t a) {
-  uint32_t r;
-  asm("v_pk_lshlrev_b16 %0, %1, %2" : "=v"(r) : "s"(0x00030003u), "v"(a));
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+  f32x2_t f = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2_t));
+}
+// v minus the low / high float16 of w, exactly rounded (one mixed-precision fma)
+__device__ __forceinline__ float rem_lo(float v, uint32_t w) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(v));
+  return r;
+}
+__device__ __forceinline__ float rem_hi(float v, uint32_t w) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(v));
   return r;
 }
 
-// (a & m) | (b & ~m) in one v_bfi_b32 (written out, the compiler splits it
-// into and / or / bitop3); m wave-uniform (a scalar register)
-__device__ __forceinline__ uint32_t bfi32(uint32_t m, uint32_t a, uint32_t b) {
-  uint32_t r;
-  asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(m), "v"(a), "v"(b));
-  return r;
-}
-
-// The four planes of one logit from the float32 formulas (+ the unweighted
-// terms of the unmatched-mask penalty).
-template <int EM = 0>
-__device__ __forceinline__ void planes_formula(float z, const ElemParams& ep, float& neg,
-                                               float& pos, float& wp, float& w, float& negu,
-                                               float& pu) {
+// ---- planes of one logit ---------------------------------------------------
+// The four planes from the float32 formulas, unscaled, and the unweighted terms
+// of the unmatched-mask penalty.
+__device__ __forceinline__ void planes_formula(float z, const ElemParams& ep, float& neg, float& pos,
+                                               float& wp, float& w, float& negu, float& pu) {
   const Sig s = sig_terms(z);
-  w = unc_weight_m<EM>(s, ep);
+  w = unc_weight(s, ep);
   float mn, mp;
-  focal_mods_m<EM>(s, ep, mn, mp);
+  focal_mods(s, ep, mn, mp);
   negu = ep.an * mn * s.cn;
   pu = s.p;
   neg = w * negu;
@@ -92,10 +123,62 @@ __device__ __forceinline__ void planes_formula(float z, const ElemParams& ep, fl
   wp = w * s.p;
 }
 
+// Which of the per-logit forms a call takes (chosen once per 8 logits, wave-uniform):
+// 0 general; 1 no focal terms, weight H^1 (the operator's defaults); 2 no
+// focal terms, no weights; 3 focal gamma 2 with or without weights H^1.
+__device__ __forceinline__ int elem_mode(const ElemParams& ep) {
+  const bool plain = ep.gamma_mode == 0 && ep.an == 1.f && ep.ap == 1.f;
+  if (plain && ep.ug_mode == 1) return 1;
+  if (plain && ep.ug_mode == 0 && ep.ug_min <= 1.f) return 2;
+  if (ep.gamma_mode == 2 && ep.ug_mode != 2) return 3;
+  return 0;
+}
+
+// The planes scaled by kPlaneScale.  With t = -|z| log2 e, e = 2^t, d = 1 + e:
+// the entropy -(p ln p + q ln q) / ln 2 is log2 d + (e / d) |t| (both terms
+// non-negative) and softplus(+-z) = ln 2 log2 d + max(+-z, 0), so the default
+// form takes 3 transcendental and 15 other ops per logit.
+template <int EM>
+__device__ __forceinline__ void planes_scaled(float z, const ElemParams& ep, float& neg, float& pos, float& wp,
+                                              float& w, float& negu, float& pu) {
+  if constexpr (EM == 0) {
+    planes_formula(z, ep, neg, pos, wp, w, negu, pu);
+    neg *= kPlaneScale;
+    pos *= kPlaneScale;
+    wp *= kPlaneScale;
+    w *= kPlaneScale;
+    return;
+  }
+  const float t = -fabsf(z) * kLog2e;
+  const float e = __builtin_amdgcn_exp2f(t);
+  const float d = 1.f + e;
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float l2 = __builtin_amdgcn_logf(d);  // log2
+  const float er = e * r;
+  const bool up = z >= 0.f;
+  const float p = up ? r : er;
+  float cn = __builtin_fmaf(l2, kLn2, fmaxf(z, 0.f)), cp = __builtin_fmaf(l2, kLn2, fmaxf(-z, 0.f));
+  if constexpr (EM == 3) {
+    const float q = up ? er : r;
+    cn *= ep.an * (p * p);
+    cp *= ep.ap * (q * q);
+  }
+  if (EM == 1 || (EM == 3 && ep.ug_mode == 1)) {
+    const float h = __builtin_fmaf(-er, t, l2);
+    w = __builtin_amdgcn_fmed3f(h * kPlaneScale, ep.ug_min * kPlaneScale, kPlaneScale);
+  } else {
+    w = kPlaneScale;
+  }
+  negu = cn;
+  pu = p;
+  neg = w * cn;
+  pos = w * cp;
+  wp = w * p;
+}
+
 // Build the LUT in LDS (all threads of the workgroup).  The overflow slot
 // holds NaN so that a wave whose sums come out NaN knows it met |z| >= 64,
-// inf or nan (finite table entries cannot produce NaN) and redoes its K-range
-// with the formulas.
+// inf or nan (finite table entries stay below 2^15 and cannot produce NaN).
 __device__ void build_lut(unsigned char* lut, const ElemParams& ep) {
   for (uint32_t e = threadIdx.x; e < 2 * kLutBlock; e += blockDim.x) {
     const uint32_t sgn = e >= kLutBlock ? 1u : 0u;
@@ -105,12 +188,12 @@ __device__ void build_lut(unsigned char* lut, const ElemParams& ep) {
       const uint32_t mag = j == 0 ? 0u : kLutSub + j;  // j == 0: |z| < 2^-9 -> z = 0
       const float z = __uint_as_float(((sgn << 15) | mag) << 16);
       float neg, pos, wp, w, nu, pu;
-      planes_formula(z, ep, neg, pos, wp, w, nu, pu);
-      v.x = pack_bf16x2(neg, pos);
-      v.y = pack_bf16x2(wp, w);
+      planes_scaled<0>(z, ep, neg, pos, wp, w, nu, pu);
+      v.x = pack_f16x2(neg, pos);
+      v.y = pack_f16x2(wp, w);
     } else {
-      v.x = 0x7FC07FC0u;  // NaN marker
-      v.y = 0x7FC07FC0u;
+      v.x = 0x7E007E00u;  // NaN marker
+      v.y = 0x7E007E00u;
     }
     *(uint2*)(lut + sgn * kLutNegOff + j * 8) = v;
   }
@@ -122,29 +205,28 @@ struct Raw8 {
   uint4 w[DT == ML_F32 ? 2 : 1];
 };
 
-// `vec`: rows start 16-byte aligned (HW % 4 == 0 for float32, HW % 8 == 0
-// otherwise); else the 8 values are read one by one.
+// Rows of odd sizes start on element boundaries only: 16-byte loads all the
+// same (global memory takes them at any alignment).
 template <int DT>
-__device__ __forceinline__ void load_raw8(const void* base, int64_t i, Raw8<DT>& r, bool vec) {
+__device__ __forceinline__ void load_raw8(const void* base, int64_t i, Raw8<DT>& r) {
+  if constexpr (DT == ML_F32) __builtin_memcpy(&r, (const float*)base + i, 32);
+  else __builtin_memcpy(&r, (const uint16_t*)base + i, 16);
+}
+// The first nvalid (any int64: <= 0 none, >= 8 all) of the 8 logits, the rest zero.
+template <int DT>
+__device__ __forceinline__ void load_raw8_part(const void* base, int64_t i, int64_t nvalid, Raw8<DT>& r) {
   if constexpr (DT == ML_F32) {
-    const float* f = (const float*)base + i;
-    if (vec) {
-      r.w[0] = ((const uint4*)f)[0];
-      r.w[1] = ((const uint4*)f)[1];
-    } else {
-      r.w[0] = make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]),
-                          __float_as_uint(f[3]));
-      r.w[1] = make_uint4(__float_as_uint(f[4]), __float_as_uint(f[5]), __float_as_uint(f[6]),
-                          __float_as_uint(f[7]));
-    }
+    uint32_t u[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) u[k] = k < nvalid ? __float_as_uint(((const float*)base)[i + k]) : 0u;
+    r.w[0] = make_uint4(u[0], u[1], u[2], u[3]);
+    r.w[1] = make_uint4(u[4], u[5], u[6], u[7]);
   } else {
-    const uint16_t* h = (const uint16_t*)base + i;
-    if (vec) {
-      r.w[0] = *(const uint4*)h;
-    } else {
-      r.w[0] = make_uint4((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
-                          (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16));
-    }
+    uint32_t u[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k < nvalid) u[k >> 1] |= (uint32_t)((const uint16_t*)base)[i + k] << ((k & 1) * 16);
+    r.w[0] = make_uint4(u[0], u[1], u[2], u[3]);
   }
 }
 
@@ -170,9 +252,23 @@ __device__ __forceinline__ void raw_to_f32(const Raw8<DT>& r, float z[8]) {
   }
 }
 
-// Split 8 fp32 values into NS bf16 terms whose sum reproduces them.
+// 8 float32 values as NT float16 terms (1 or 2) whose sum reproduces them.
+template <int NT>
+__device__ __forceinline__ void split_f16(const float v[8], f16x8_t out[NT]) {
+  u32x4_t hi;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) hi[k] = pack_f16x2(v[2 * k], v[2 * k + 1]);
+  out[0] = __builtin_bit_cast(f16x8_t, hi);
+  if constexpr (NT == 2) {
+    u32x4_t lo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) lo[k] = pack_f16x2(rem_lo(v[2 * k], hi[k]), rem_hi(v[2 * k + 1], hi[k]));
+    out[1] = __builtin_bit_cast(f16x8_t, lo);
+  }
+}
+// ... and as NS bf16 terms (redone ranges).
 template <int NS>
-__device__ __forceinline__ void split_pack(const float v[8], bf16x8_t out[NS]) {
+__device__ __forceinline__ void split_bf16(const float v[8], bf16x8_t out[NS]) {
   float rem[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) rem[k] = v[k];
@@ -192,37 +288,73 @@ __device__ __forceinline__ void split_pack(const float v[8], bf16x8_t out[NS]) {
   }
 }
 
-// A planes of one row's 8 cells by formula; with MASK, cells >= nvalid are zero.
-template <int DT, int NS, bool MASK>
-__device__ __forceinline__ void planes8_formula(const Raw8<DT>& r, const ElemParams& ep,
-                                                int64_t nvalid, bool unw, bf16x8_t A[4][NS],
-                                                float& ub, float& up) {
+// A planes of one row's 8 cells by formula, float16 terms; with MASK, cells >=
+// nvalid are zero.  ub, up: sums of the unweighted terms (unw).
+template <int DT, int NT, bool MASK>
+__device__ __forceinline__ void planes8_formula(const Raw8<DT>& r, const ElemParams& ep, int64_t nvalid, bool unw,
+                                                f16x8_t A[4][NT], float& ub, float& up) {
   float z[8];
   raw_to_f32<DT>(r, z);
   float v[4][8];
-  auto cell = [&](auto em, int k) {
+  auto cells = [&](auto em) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      float neg, pos, wp, w, nu, pu;
+      planes_scaled<decltype(em)::value>(z[k], ep, neg, pos, wp, w, nu, pu);
+      const bool ok = !MASK || k < nvalid;
+      v[0][k] = ok ? neg : 0.f;
+      v[1][k] = ok ? pos : 0.f;
+      v[2][k] = ok ? wp : 0.f;
+      v[3][k] = ok ? w : 0.f;
+      if (unw) {
+        ub += ok ? nu : 0.f;
+        up += ok ? pu : 0.f;
+      }
+    }
+  };
+  switch (elem_mode(ep)) {
+    case 1: cells(std::integral_constant<int, 1>()); break;
+    case 2: cells(std::integral_constant<int, 2>()); break;
+    case 3: cells(std::integral_constant<int, 3>()); break;
+    default: cells(std::integral_constant<int, 0>()); break;
+  }
+#pragma unroll
+  for (int pl = 0; pl < 4; ++pl) split_f16<NT>(v[pl], A[pl]);
+}
+// The same as unscaled bf16 terms, for a redone range.
+template <int DT>
+__device__ __forceinline__ void planes8_redo(const Raw8<DT>& r, const ElemParams& ep, int64_t nvalid,
+                                             bf16x8_t A[4][InTraits<DT>::kRedo]) {
+  float z[8];
+  raw_to_f32<DT>(r, z);
+  float v[4][8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
     float neg, pos, wp, w, nu, pu;
-    planes_formula<decltype(em)::value>(z[k], ep, neg, pos, wp, w, nu, pu);
-    const bool ok = !MASK || k < nvalid;
+    planes_formula(z[k], ep, neg, pos, wp, w, nu, pu);
+    const bool ok = k < nvalid;
     v[0][k] = ok ? neg : 0.f;
     v[1][k] = ok ? pos : 0.f;
     v[2][k] = ok ? wp : 0.f;
     v[3][k] = ok ? w : 0.f;
-    if (unw) {
-      ub += ok ? nu : 0.f;
-      up += ok ? pu : 0.f;
-    }
-  };
-  // one branch on the modes per 8 logits (wave-uniform), not per logit
-  if (default_modes(ep)) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) cell(std::integral_constant<int, 1>(), k);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) cell(std::integral_constant<int, 0>(), k);
   }
 #pragma unroll
-  for (int pl = 0; pl < 4; ++pl) split_pack<NS>(v[pl], A[pl]);
+  for (int pl = 0; pl < 4; ++pl) split_bf16<InTraits<DT>::kRedo>(v[pl], A[pl]);
+}
+
+// Table byte offsets (sign block included) of the two bf16 logits packed in
+// u, in compiler-visible packed 16-bit ops (no inline assembly, so no hazard
+// padding after each one): the clamped index times 8 stays below 2^15, so the
+// sign bit ORs in without carry.
+__device__ __forceinline__ uint32_t lut_addr_pair(uint32_t u) {
+  const u16x2_t m = as_u16x2(u & 0x7FFF7FFFu);
+  const u16x2_t idx = __builtin_elementwise_min(
+      __builtin_elementwise_sub_sat(m, (u16x2_t){(unsigned short)kLutSub, (unsigned short)kLutSub}),
+      (u16x2_t){(unsigned short)(kLutN + 1), (unsigned short)(kLutN + 1)});
+  uint32_t addr = (u & 0x80008000u) | as_u32(idx << (u16x2_t){3, 3});
+  // kept whole, so its two halves are one mask and one shift of it
+  asm("" : "+v"(addr));
+  return addr;
 }
 
 // Table entries of one row's 8 bf16 cells (LDS reads only; see lut_planes).
@@ -230,11 +362,7 @@ __device__ __forceinline__ void lut_lookup8(const uint4& x, const unsigned char*
   const uint32_t u[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t m = u[i] & 0x7FFF7FFFu;
-    const uint32_t idx =
-        pk_min_u16(pk_sub_sat_u16(m, kLutSub * 0x10001u), (kLutN + 1) * 0x10001u);
-    // sign bits (the negative block's 32 KB offset) merged in with one bitfield insert
-    const uint32_t addr = bfi32(0x80008000u, u[i], pk_lshl3_u16(idx));
+    const uint32_t addr = lut_addr_pair(u[i]);
     E[2 * i] = *(const uint2*)(lut + (addr & 0xFFFFu));
     E[2 * i + 1] = *(const uint2*)(lut + (addr >> 16));
   }
@@ -242,7 +370,7 @@ __device__ __forceinline__ void lut_lookup8(const uint4& x, const unsigned char*
 
 // The four A planes from the entries of 8 cells: (neg, pos) and (wp, w) of
 // each cell regrouped into per-plane pairs of consecutive cells.
-__device__ __forceinline__ void lut_planes(const uint2 E[8], bf16x8_t A[4]) {
+__device__ __forceinline__ void lut_planes(const uint2 E[8], f16x8_t A[4]) {
   u32x4_t a0, a1, a2, a3;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -252,18 +380,98 @@ __device__ __forceinline__ void lut_planes(const uint2 E[8], bf16x8_t A[4]) {
     a2[i] = __builtin_amdgcn_perm(e1.y, e0.y, 0x05040100u);
     a3[i] = __builtin_amdgcn_perm(e1.y, e0.y, 0x07060302u);
   }
-  A[0] = __builtin_bit_cast(bf16x8_t, a0);
-  A[1] = __builtin_bit_cast(bf16x8_t, a1);
-  A[2] = __builtin_bit_cast(bf16x8_t, a2);
-  A[3] = __builtin_bit_cast(bf16x8_t, a3);
+  A[0] = __builtin_bit_cast(f16x8_t, a0);
+  A[1] = __builtin_bit_cast(f16x8_t, a1);
+  A[2] = __builtin_bit_cast(f16x8_t, a2);
+  A[3] = __builtin_bit_cast(f16x8_t, a3);
 }
 
-// A planes of one row's 8 bf16 cells from the LDS table.
-__device__ __forceinline__ void planes8_lut(const uint4& x, const unsigned char* lut,
-                                            bf16x8_t A[4]) {
-  uint2 E[8];
-  lut_lookup8(x, lut, E);
-  lut_planes(E, A);
+// ---- right operands ---------------------------------------------------------
+// Counts of 8 cells: kHot where a label code equals the column's (a zero mask
+// makes it the ones column), 0 elsewhere.
+__device__ __forceinline__ u32x4_t hot8(const uint32_t (&L2)[4], uint32_t col, uint32_t mask = 0xFFFFFFFFu) {
+  u32x4_t b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    // (L ^ col) & mask in one three-input boolean op
+    b[i] = as_u32(__builtin_elementwise_sub_sat((u16x2_t){kHot, kHot},
+                                                as_u16x2(__builtin_amdgcn_bitop3_b32(L2[i], col, mask, 0x28))));
+  return b;
+}
+// pair - n for 8 16-bit integers.
+__device__ __forceinline__ u32x4_t isub8(uint32_t pair, const u32x4_t& n) {
+  u32x4_t b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = as_u32(as_u16x2(pair) - as_u16x2(n[i]));
+  return b;
+}
+// 8 integers times a constant.
+__device__ __forceinline__ u32x4_t imul8(const u32x4_t& n, unsigned short c) {
+  u32x4_t b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = as_u32(as_u16x2(n[i]) * (u16x2_t){c, c});
+  return b;
+}
+// 8 u8 counts with `hi` as every high byte: 0 for integers, 0x64 for 1024 + n in float16.
+template <uint32_t HI>
+__device__ __forceinline__ u32x4_t widen8(uint32_t x, uint32_t y) {
+  constexpr uint32_t h = HI * 0x01010101u;
+  constexpr uint32_t s0 = HI ? 0x04010400u : 0x0C010C00u, s1 = HI ? 0x04030402u : 0x0C030C02u;
+  return u32x4_t{__builtin_amdgcn_perm(h, x, s0), __builtin_amdgcn_perm(h, x, s1), __builtin_amdgcn_perm(h, y, s0),
+                 __builtin_amdgcn_perm(h, y, s1)};
+}
+// c + t and c - t for 8 float16 values, two per op (exact here: integers below
+// 2048); c: the value twice.
+template <bool NEG>
+__device__ __forceinline__ u32x4_t hadd8(uint32_t c, const u32x4_t& t) {
+  u32x4_t b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (NEG) asm("v_pk_add_f16 %0, %1, %2 neg_lo:[0,1] neg_hi:[0,1]" : "=v"(b[i]) : "s"(c), "v"(t[i]));
+    else asm("v_pk_add_f16 %0, %1, %2" : "=v"(b[i]) : "s"(c), "v"(t[i]));
+  }
+  return b;
+}
+// The operands n and N2 - n of one column tile.
+struct Opnd {
+  f16x8_t n, rest;
+};
+// u8 counts; top: 1024 + N2 as a float16 pair (wave-uniform).
+template <bool REST>
+__device__ __forceinline__ Opnd opnd_u8(uint32_t x, uint32_t y, uint32_t top) {
+  const u32x4_t t = widen8<0x64>(x, y);  // 1024 + n
+  Opnd o;
+  o.n = __builtin_bit_cast(f16x8_t, hadd8<false>(0xE400E400u, t));  // -1024
+  if (REST) o.rest = __builtin_bit_cast(f16x8_t, hadd8<true>(top, t));
+  return o;
+}
+__device__ __forceinline__ uint32_t opnd_top(float N2) { return (0x6400u + (uint32_t)N2) * 0x10001u; }
+// Label compare: ONE is the value of a hit, kHot (2^-16) or 0x3C00 (1.0).
+template <uint32_t ONE, bool REST>
+__device__ __forceinline__ Opnd opnd_hot(const u32x4_t& hot) {
+  const u32x4_t v = ONE == kHot ? hot : imul8(hot, (unsigned short)(ONE / kHot));
+  Opnd o;
+  o.n = __builtin_bit_cast(f16x8_t, v);
+  if (REST) o.rest = __builtin_bit_cast(f16x8_t, isub8(ONE * 0x10001u, v));
+  return o;
+}
+// Bits 0..10 (HIGH = 0) or 11..15 of 8 16-bit integers as float16.
+template <bool HIGH>
+__device__ __forceinline__ f16x8_t part8(const u32x4_t& w) {
+  constexpr uint32_t m = HIGH ? 0xF800u : 0x07FFu;
+  u32x4_t b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = pack_f16x2((float)(w[i] & m), (float)((w[i] >> 16) & m));
+  return __builtin_bit_cast(f16x8_t, b);
+}
+// bf16 operands of a redone range from 16-bit integers: the bits of `mask`,
+// shifted down.
+__device__ __forceinline__ bf16x8_t redo8(const u32x4_t& w, uint32_t mask, int shift = 0) {
+  u32x4_t b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    b[i] = pack_bf16x2((float)((w[i] & mask) >> shift), (float)(((w[i] >> 16) & mask) >> shift));
+  return __builtin_bit_cast(bf16x8_t, b);
 }
 
 // Pacing of the waves of one workgroup that share a CU: the SIMD arbiter
@@ -295,39 +503,42 @@ __device__ __forceinline__ void pace(int* prog, int k) {
 
 // In-workgroup sum of R consecutive K-splits of one task (R a power of two):
 // this wave is split r of its group grp of R waves.  buf: the workgroup's LDS
-// exchange area for its writers, 3*RT*NT float4 per lane each; rsbuf: their
-// row sums.  buf == null: no reduction.
+// exchange area for its writers, 2*NT float4 per lane each (two planes at a
+// time); rsbuf: their row sums.  buf == null: no reduction.
 struct SplitRed {
   f32x4_t* buf = nullptr;
   float2* rsbuf = nullptr;
   int R = 1, r = 0, grp = 0;
 };
+constexpr int kRedBarriers = 4;  // per level of the tree
 
-// One wave's work: 16*RT query rows of task (lb, rtile) over the K-steps of
-// split ks of KS; writes the partial sums to `out` ([3][16*RT][16*NT]) and,
-// for unweighted penalties, the row sums to `rs` ([16*RT][2]).  TAB:
-// per-cell planes from the LDS table (bf16 only); if the sums come out NaN,
-// some cell of the K-range hit the table's overflow marker, and the wave
-// redoes the range with the formulas before writing.  `setup` (the
+// One wave's work: 16 query rows of task (lb, rtile) over the K-steps of
+// split ks of KS; writes the partial sums to `out` ([NP][16][16*NT]) and,
+// for unweighted penalties, the row sums to `rs` ([16][2]).  TAB:
+// per-cell planes from the LDS table (bf16 only).  If the sums come out
+// non-finite (the table's marker, or a plane beyond float16), the wave redoes
+// the range with bf16 operands before writing.  `setup` (the
 // workgroup's table build and barrier) is called exactly once on every path,
 // after the first D K-steps of loads are issued, so their latency overlaps it.
 // With red.buf, the R waves of the group add their sums in a fixed tree order
-// (wave r takes wave r + h for h = R/2, ..., 1; 2 log2(R) barriers for every
-// wave of the workgroup) and only wave 0 of the group writes.
-template <int DT, int RT, int NT, int CNT, bool TAB, class Setup>
-__device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t rtile,
-                                          int64_t ks, int64_t KS, const unsigned char* lut,
-                                          float* out, float* rs_out, int* prog, Setup&& setup,
-                                          const SplitRed& red = SplitRed(), uint32_t* klut = nullptr) {
-  constexpr int NS = InTraits<DT>::kSplit;
-  // slot-sum form (classes 1 and 2 on label maps without the table): four
-  // planes summed per slot over the cells whose key (the slot of their label's
-  // column, or G for cells of no column) is that slot, with one-hot operands
-  // only, so each K-step runs the MFMAs of just the column tiles its cells'
-  // keys fall in.  klut: this wave's LDS label -> (key | tile bit << 16) table.
-  constexpr bool SP = CNT == 0 && !TAB && NT >= 7;
-  constexpr int NP = SP ? 4 : 3;
+// (wave r takes wave r + h for h = R/2, ..., 1; kRedBarriers log2(R) barriers for
+// every wave of the workgroup) and only wave 0 of the group writes.
+// CNT: 0 label map, 1 u8 counts, 2 u16 counts.  In the wide classes (NT >= 7) a
+// K-step's MFMAs run only for the column tiles its 32 cells touch (a coherent
+// label map touches few of them).
+template <int DT, int NT, int CNT, bool TAB, class Setup>
+__device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t rtile, int64_t ks, int64_t KS,
+                                          const unsigned char* lut, float* out, float* rs_out, int* prog,
+                                          Setup&& setup, const SplitRed& red = SplitRed(),
+                                          uint32_t* klut = nullptr) {
+  constexpr int NS = TAB ? 1 : InTraits<DT>::kTerms;
+  // label maps in the wide classes: the label -> (slot | tile bit << 16) table
+  // klut (this wave's, in LDS) gives each K-step's slots and touched tiles
+  constexpr bool KEYS = CNT == 0 && NT >= 7;
+  constexpr bool SUMS = NT >= 7;  // slot sums
+  constexpr int NP = class_planes(SUMS ? 1 : 0);
   constexpr int D = TAB ? kDepth : 2;  // K-steps of logits and labels in flight
+  constexpr uint32_t kOne = TAB ? kHot : 0x3C00u;  // a label hit's operand
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g4 = lane >> 4;
   const ElemParams ep = a.ep;
@@ -335,56 +546,60 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
   const int64_t b = lb % a.B;
   const int G = __builtin_amdgcn_readfirstlane(a.ncols[b]);
   const int nt_used = (G + 1 + 15) >> 4;
-  const int64_t q0 = rtile * (16 * RT);
+  const int64_t q0 = rtile * 16;
 
-  // per-lane column operands: label pair, and the coefficients that turn the
-  // match bit into the one-hot (B) and complement (B') bf16 operands.  Real
-  // columns: B = 1 on match, B' = 1 elsewhere; ones column (slot G): B = N2,
-  // B' = 0; padding: both 0.
-  uint32_t colL[NT], coefB[NT], baseB[NT];
-  const uint32_t n2pair = pack_bf16x2(a.N2, a.N2);
-  if constexpr (!SP) {
+  // Per tile: the lane's column code pair and compare mask (slot G: the ones
+  // column; padding compares with label 0, its sums are never used), or its row
+  // of the count tiles (slot G: the ones column or the pixels of no column;
+  // padding reads that row too).
+  uint32_t colL[KEYS ? 1 : NT], colM[KEYS ? 1 : NT];
+  const uint8_t* cbase = nullptr;
+  uint32_t crow[CNT ? NT : 1];
+  const int64_t cstep = (int64_t)a.counts.rows * kCountCells * (CNT == 2 ? 2 : 1);  // bytes per block
+  if constexpr (!KEYS) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const int slot = nt * 16 + r;
-      colL[nt] = 0;
-      coefB[nt] = slot < G ? 0x3F803F80u : 0u;
-      baseB[nt] = slot < G ? 0x3F803F80u : (slot == G ? n2pair : 0u);
+      int act = -1;
       if (slot < G) {
         const int c = a.colmap[b * a.nslot + slot];
-        const int act = c + (c >= a.bg ? 1 : 0);
-        colL[nt] = (uint32_t)act * 0x10001u;
+        act = c + (c >= a.bg ? 1 : 0);
+      }
+      if constexpr (CNT == 0) {
+        colL[nt] = act >= 0 ? label_code(act) * 0x10001u : 0u;
+        colM[nt] = slot == G ? 0u : 0xFFFFFFFFu;
+        asm("" : "+v"(colM[nt]));  // a register, not a select at every use
+      } else {
+        const int rest = (int)a.GT_total + (SUMS ? 0 : 1);
+        crow[nt] = ((uint32_t)(act >= 0 ? act : rest) * kCountCells + 8u * g4) * CNT;
       }
     }
+    if constexpr (CNT != 0) cbase = a.counts.p + b * a.counts.nb * cstep;
   } else {
-    // labels (u16, 0xFFFF for none; min(label, 256) indexes the table) ->
-    // key: every entry G first, then each column's label its slot (one
+    // label (the code's high byte) -> key: every entry G first, then each
+    // column's label its slot (one
     // wave's LDS writes land in issue order; the wait keeps the two rounds
     // apart all the same)
     const uint32_t eG = (uint32_t)G | (1u << (16 + (G >> 4)));
-    for (int l = lane; l < 257; l += 64) klut[l] = eG;
+    for (int l = lane; l < 256; l += 64) klut[l] = eG;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     for (int sl = lane; sl < G; sl += 64) {
       const int c = a.colmap[b * a.nslot + sl];
       const int act = c + (c >= a.bg ? 1 : 0);
-      if (act >= 0 && act < 256) klut[act] = (uint32_t)sl | (1u << (16 + (sl >> 4)));
+      klut[act & 255] = (uint32_t)sl | (1u << (16 + (sl >> 4)));
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 
-  f32x4_t acc[NP][RT][NT];
+  f32x4_t acc[NP][NT];
+  auto clear = [&]() {
 #pragma unroll
-  for (int i = 0; i < NP; ++i)
+    for (int i = 0; i < NP; ++i)
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[i][rt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float ub[RT], up[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    ub[rt] = 0.f;
-    up[rt] = 0.f;
-  }
+      for (int nt = 0; nt < NT; ++nt) acc[i][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+  float ub = 0.f, up = 0.f;
 
   // this wave's K-steps: [s0, s1) of the full steps, plus the tail step
   const int64_t full = a.HW / kStep;
@@ -392,202 +607,145 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
   const int64_t s0 = min(full, ks * per);
   const int64_t s1 = min(full, s0 + per);
   const bool has_tail = (a.HW % kStep) != 0 && ks == KS - 1;
+  const int64_t rowoff = (lb * a.Q + min(q0 + r, a.Q - 1)) * a.HW + g4 * 8;  // rows >= Q: unused outputs
+  const uint16_t* labp = a.lab16 + (CNT ? 0 : b * a.HWp + g4 * 8);
 
-  int64_t rowoff[RT];
+  // raw right operands of K-step st: labels, or the lane's 8 counts per tile
+  struct BRaw {
+    uint4 lab;
+    uint32_t w[CNT ? NT : 1][CNT == 2 ? 4 : 2];
+  };
+  auto fetch_b = [&](BRaw& x, int64_t st) {
+    if constexpr (CNT == 0) {
+      x.lab = *(const uint4*)(labp + st * kStep);
+    } else {
+      const uint8_t* p = cbase + (st >> 1) * cstep + (st & 1) * (kStep * CNT);
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int64_t q = min(q0 + rt * 16 + r, a.Q - 1);  // rows >= Q compute unused outputs
-    rowoff[rt] = (lb * a.Q + q) * a.HW + g4 * 8;
-  }
-  const uint16_t* labp = a.lab16 + b * a.HWp + g4 * 8;
-  const bool vec = DT == ML_F32 ? (a.HW % 4 == 0) : (a.HW % 8 == 0);
-
-  auto mma_step = [&](bf16x8_t (&A)[4][RT][NS], const uint4& lv, int64_t cell0) {
-    const uint32_t L2[4] = {lv.x, lv.y, lv.z, lv.w};
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      if (nt >= nt_used) continue;
-      // CNT == 2 (u16 counts): B = hi + lo with hi = v & 0xFF00 and lo =
-      // v & 0xFF, both exact in bf16 (counts and N2 - n reach s*s > 256,
-      // which bf16 does not hold exactly), so each product runs twice
-      constexpr int NB = CNT == 2 ? 2 : 1;
-      u32x4_t bp[NB], bv[NB];
-      if constexpr (CNT == 0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t m = pk_min_u16(L2[i] ^ colL[nt], 0x00010001u);
-          bp[0][i] = pk_mul_lo_u16(m, coefB[nt]);
-          bv[0][i] = pk_sub_u16(baseB[nt], bp[0][i]);
-        }
-      } else {
-        // real columns: B = n, B' = N2 - n; ones column: B = N2, B' = 0;
-        // padding: both 0 (integers: counts never exceed N2)
-        const int slot = nt * 16 + r;
-        const uint32_t N2i = (uint32_t)a.N2;
-        const uint32_t act = colL[nt] & 0xFFFFu;
-        uint32_t n[8];
-        counts8_u32(a.counts.p, CNT == 2 ? 2 : 1, a.counts.at(b, act, cell0), n);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          uint32_t v[2], p[2];
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            v[h] = slot < G ? n[2 * i + h] : (slot == G ? N2i : 0u);
-            p[h] = slot < G ? N2i - n[2 * i + h] : 0u;
-          }
-          if constexpr (NB == 1) {
-            bv[0][i] = pack_bf16x2((float)v[0], (float)v[1]);
-            bp[0][i] = pack_bf16x2((float)p[0], (float)p[1]);
-          } else {
-            bv[0][i] = pack_bf16x2((float)(v[0] & 0xFF00u), (float)(v[1] & 0xFF00u));
-            bp[0][i] = pack_bf16x2((float)(p[0] & 0xFF00u), (float)(p[1] & 0xFF00u));
-            bv[NB - 1][i] = pack_bf16x2((float)(v[0] & 0xFFu), (float)(v[1] & 0xFFu));
-            bp[NB - 1][i] = pack_bf16x2((float)(p[0] & 0xFFu), (float)(p[1] & 0xFFu));
-          }
-        }
-      }
-#pragma unroll
-      for (int h = 0; h < NB; ++h) {
-        const bf16x8_t Bp = __builtin_bit_cast(bf16x8_t, bp[h]);
-        const bf16x8_t Bv = __builtin_bit_cast(bf16x8_t, bv[h]);
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-          for (int sp = 0; sp < NS; ++sp) {
-            acc[0][rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0][rt][sp], Bp, acc[0][rt][nt], 0, 0, 0);
-            acc[0][rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1][rt][sp], Bv, acc[0][rt][nt], 0, 0, 0);
-            acc[1][rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[2][rt][sp], Bv, acc[1][rt][nt], 0, 0, 0);
-            acc[2][rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[3][rt][sp], Bv, acc[2][rt][nt], 0, 0, 0);
-          }
-        }
+      for (int nt = 0; nt < NT; ++nt) {
+        if (nt >= nt_used) continue;
+        if constexpr (CNT == 1) *(uint2*)x.w[nt] = *(const uint2*)(p + crow[nt]);
+        else *(uint4*)x.w[nt] = *(const uint4*)(p + crow[nt]);
       }
     }
   };
-
-  // slot-sum form: keys of the lane's 8 cells as u16 pairs, and the column
-  // tiles any of the K-step's 32 cells falls in (the four lane groups hold
-  // different cells; every lane ends with the same mask)
+  // slots of the lane's 8 cells as u16 pairs (like label codes), and the column tiles any of the
+  // K-step's 32 cells falls in (the four lane groups hold different cells;
+  // every lane ends with the same mask)
   auto keys_of = [&](const uint4& lv, uint32_t (&kp)[4]) -> uint32_t {
     const uint32_t L2[4] = {lv.x, lv.y, lv.z, lv.w};
     uint32_t e[8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      e[2 * i] = klut[min(L2[i] & 0xFFFFu, 256u)];
-      e[2 * i + 1] = klut[min(L2[i] >> 16, 256u)];
+      e[2 * i] = klut[(L2[i] >> 8) & 0xFFu];
+      e[2 * i + 1] = klut[L2[i] >> 24];
     }
     uint32_t t = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      kp[i] = __builtin_amdgcn_perm(e[2 * i + 1], e[2 * i], 0x0C040C00u);
+      kp[i] = __builtin_amdgcn_perm(e[2 * i + 1], e[2 * i], 0x040C000Cu);  // slots in the high bytes
       t |= e[2 * i] | e[2 * i + 1];
     }
     t >>= 16;
     return __builtin_amdgcn_readlane(t, 0) | __builtin_amdgcn_readlane(t, 16) |
            __builtin_amdgcn_readlane(t, 32) | __builtin_amdgcn_readlane(t, 48);
   };
-  auto mma_step_sp = [&](bf16x8_t (&A)[4][RT][NS], const uint32_t (&kp)[4], uint32_t tmask) {
+  // f(nt, raw 16-bit integers of tile nt: compare results or counts) for the
+  // tiles the K-step touches; u8 counts stay packed in the first two words
+  auto for_tiles = [&](const BRaw& x, const uint32_t (&kp)[4], uint32_t tmask, auto&& f) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      if (nt >= nt_used || !((tmask >> nt) & 1u)) continue;
-      const uint32_t s2 = (uint32_t)(nt * 16 + r) * 0x10001u;
-      u32x4_t bv;
+      if (nt >= nt_used) continue;
+      if constexpr (KEYS) {
+        if (!((tmask >> nt) & 1u)) continue;
+        f(nt, hot8(kp, (uint32_t)(nt * 16 + r) * 0x01000100u));
+      } else if constexpr (CNT == 0) {
+        const uint32_t L2[4] = {x.lab.x, x.lab.y, x.lab.z, x.lab.w};
+        f(nt, hot8(L2, colL[nt], colM[nt]));
+      } else {
+        uint32_t any = 0u;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t m = pk_min_u16(kp[i] ^ s2, 0x00010001u);
-        bv[i] = pk_sub_u16(0x3F803F80u, pk_mul_lo_u16(m, 0x3F803F80u));
-      }
-      const bf16x8_t Bv = __builtin_bit_cast(bf16x8_t, bv);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-        for (int sp = 0; sp < NS; ++sp) {
-#pragma unroll
-          for (int pl = 0; pl < 4; ++pl)
-            acc[pl][rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[pl][rt][sp], Bv, acc[pl][rt][nt], 0, 0, 0);
-        }
+        for (int i = 0; i < 2 * CNT; ++i) any |= x.w[nt][i];
+        if (SUMS && __ballot(any != 0u) == 0ull) continue;
+        if constexpr (CNT == 1) f(nt, u32x4_t{x.w[nt][0], x.w[nt][1], 0u, 0u});
+        else f(nt, u32x4_t{x.w[nt][0], x.w[nt][1], x.w[nt][2], x.w[nt][3]});
       }
     }
   };
-  // one K-step of either form
-  auto mma_any = [&](bf16x8_t (&A)[4][RT][NS], const uint4& lv, int64_t cell0) {
-    if constexpr (SP) {
-      uint32_t kp[4];
-      const uint32_t tm = keys_of(lv, kp);
-      mma_step_sp(A, kp, tm);
-    } else {
-      mma_step(A, lv, cell0);
-    }
+  const uint32_t n2pair = (uint32_t)a.N2 * 0x10001u;
+  auto mma_step = [&](f16x8_t (&A)[4][NS], const BRaw& x, const uint32_t (&kp)[4], uint32_t tmask) {
+    for_tiles(x, kp, tmask, [&](int nt, const u32x4_t& raw) {
+      auto mul = [&](int i, int pl, const f16x8_t& v) {
+#pragma unroll
+        for (int sp = 0; sp < NS; ++sp)
+          acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[pl][sp], v, acc[i][nt], 0, 0, 0);
+      };
+      auto mul_all = [&](const Opnd& o) {
+        if constexpr (SUMS) {
+#pragma unroll
+          for (int pl = 0; pl < 4; ++pl) mul(pl, pl, o.n);
+        } else {
+          mul(0, 0, o.rest);
+          mul(1, 2, o.n);
+          mul(2, 3, o.n);
+          mul(0, 1, o.n);
+        }
+      };
+      if constexpr (CNT == 0) {
+        mul_all(opnd_hot<kOne, !SUMS>(raw));
+      } else if constexpr (CNT == 1) {
+        mul_all(opnd_u8<!SUMS>(raw[0], raw[1], opnd_top(a.N2)));
+      } else {  // integers up to 65025 as two exact float16 parts
+        const u32x4_t rest = isub8(n2pair, raw);
+        mul_all(Opnd{part8<false>(raw), part8<false>(rest)});
+        mul_all(Opnd{part8<true>(raw), part8<true>(rest)});
+      }
+    });
   };
 
-  // Software pipeline over this wave's nst steps: D steps of logits and
-  // labels in flight.  Slot j holds step k + j; it is turned into A operands
-  // first and then refilled with step k + j + D (clamped to the last step, so
-  // the loads are unconditional and the wait counts stay exact).  Every
-  // branch here is wave-uniform.
+  // Software pipeline over this wave's nst steps: D steps of logits (and
+  // labels) in flight, the count operands one step ahead.  Slot j holds step
+  // k + j; it is turned into A operands first and then refilled with step
+  // k + j + D (clamped to the last step, so the loads are unconditional).
+  // Every branch here is wave-uniform.
   // step counters in 32 bits: their compares stay scalar (a wave has at most
   // HW / 32 < 2^31 steps)
   const int nst = (int)(s1 - s0);
-  auto planes = [&](const Raw8<DT> (&raw)[RT], bf16x8_t (&A)[4][RT][NS]) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      bf16x8_t T[4][NS];
-      if constexpr (TAB) {
-        bf16x8_t T1[4];
-        planes8_lut(raw[rt].w[0], lut, T1);
-#pragma unroll
-        for (int pl = 0; pl < 4; ++pl) T[pl][0] = T1[pl];
-      } else {
-        planes8_formula<DT, NS, false>(raw[rt], ep, 8, unw, T, ub[rt], up[rt]);
-      }
-#pragma unroll
-      for (int pl = 0; pl < 4; ++pl)
-#pragma unroll
-        for (int sp = 0; sp < NS; ++sp) A[pl][rt][sp] = T[pl][sp];
-    }
-  };
   if (nst > 0) {
-    Raw8<DT> buf[D][RT];
-    uint4 lbuf[D];
-    // slot j <- step s0 + min(k, nst - 1): logits, labels
-    auto fetch_z = [&](int j, int k) {
-      const int64_t st = s0 + (k < nst ? k : nst - 1);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) load_raw8<DT>(a.logits, rowoff[rt] + st * kStep, buf[j][rt], vec);
-    };
-    auto fetch_l = [&](int j, int k) {
-      const int64_t st = s0 + (k < nst ? k : nst - 1);
-      lbuf[j] = *(const uint4*)(labp + st * kStep);
-    };
+    constexpr int DB = CNT ? 2 : D;  // right operands in flight
+    Raw8<DT> buf[D];
+    BRaw bb[DB];
+    auto at = [&](int k) { return s0 + (k < nst ? k : nst - 1); };
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-      fetch_z(j, j);
-      fetch_l(j, j);
+      load_raw8<DT>(a.logits, rowoff + at(j) * kStep, buf[j]);
+      if (CNT == 0) fetch_b(bb[j % DB], at(j));
     }
+    if constexpr (CNT != 0) fetch_b(bb[0], at(0));
     setup();
     int k = 0;
     if constexpr (TAB) {
-      // table path, software-pipelined one step deep: the LDS reads of step
-      // k + 1 are issued before the one-hot operands and MFMAs of step k, so
-      // their latency hides behind that work
-      uint2 E[RT][8];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) lut_lookup8(buf[0][rt].w[0], lut, E[rt]);
+      // software-pipelined one step deep: the table reads of step k + 1 are
+      // issued before the right operands and MFMAs of step k, so their
+      // latency hides behind that work
+      uint2 E[8];
+      lut_lookup8(buf[0].w[0], lut, E);
       auto step = [&](int j, int kj, bool refill) {
-        bf16x8_t A[4][RT][NS];
+        f16x8_t A[4][1];
+        {
+          f16x8_t T[4];
+          lut_planes(E, T);
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          bf16x8_t T1[4];
-          lut_planes(E[rt], T1);
-#pragma unroll
-          for (int pl = 0; pl < 4; ++pl) A[pl][rt][0] = T1[pl];
+          for (int pl = 0; pl < 4; ++pl) A[pl][0] = T[pl];
         }
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) lut_lookup8(buf[(j + 1) % D][rt].w[0], lut, E[rt]);
+        uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
+        if constexpr (KEYS) tm = keys_of(bb[j % DB].lab, kp);
+        lut_lookup8(buf[(j + 1) % D].w[0], lut, E);
         __builtin_amdgcn_sched_barrier(0);
-        if (refill) fetch_z(j, kj + D);
-        mma_step(A, lbuf[j], (s0 + kj) * kStep + g4 * 8);
+        if (refill) load_raw8<DT>(a.logits, rowoff + at(kj + D) * kStep, buf[j]);
+        if constexpr (CNT != 0) fetch_b(bb[(j + 1) % DB], at(kj + 1));
+        mma_step(A, bb[j % DB], kp, tm);
         __builtin_amdgcn_sched_barrier(0);
-        if (refill) fetch_l(j, kj + D);
+        if (CNT == 0 && refill) fetch_b(bb[j % DB], at(kj + D));
       };
       for (; k + D <= nst; k += D) {
         if (prog && (k & (2 * D - 1)) == 0) pace(prog, k);
@@ -598,178 +756,157 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
       for (int j = 0; j < D - 1; ++j)  // the last nst % D steps
         if (k + j < nst) step(j, k + j, false);
     } else {
+      auto step = [&](int j, int kj, bool refill) {
+        // the key table reads go out before the plane work
+        uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
+        if constexpr (KEYS) tm = keys_of(bb[j % DB].lab, kp);
+        if constexpr (CNT != 0) fetch_b(bb[(j + 1) % DB], at(kj + 1));
+        f16x8_t A[4][NS];
+        planes8_formula<DT, NS, false>(buf[j], ep, 8, unw, A, ub, up);
+        // keep each refill below the last read of its slot, so that it reuses
+        // the slot's registers instead of rotating the whole pipeline
+        __builtin_amdgcn_sched_barrier(0);
+        if (refill) load_raw8<DT>(a.logits, rowoff + at(kj + D) * kStep, buf[j]);
+        mma_step(A, bb[j % DB], kp, tm);
+        __builtin_amdgcn_sched_barrier(0);
+        if (CNT == 0 && refill) fetch_b(bb[j % DB], at(kj + D));
+      };
       for (; k + D <= nst; k += D) {
         if (prog && (k & (2 * D - 1)) == 0) pace(prog, k);
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-          // slot-sum form: the key table reads go out before the plane work
-          uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
-          if constexpr (SP) tm = keys_of(lbuf[j], kp);
-          bf16x8_t A[4][RT][NS];
-          planes(buf[j], A);
-          // keep each refill below the last read of its slot, so that it reuses
-          // the slot's registers instead of rotating the whole pipeline
-          __builtin_amdgcn_sched_barrier(0);
-          fetch_z(j, k + j + D);
-          if constexpr (SP) mma_step_sp(A, kp, tm);
-          else mma_step(A, lbuf[j], (s0 + k + j) * kStep + g4 * 8);
-          __builtin_amdgcn_sched_barrier(0);
-          fetch_l(j, k + j + D);
-        }
+        for (int j = 0; j < D; ++j) step(j, k + j, true);
       }
 #pragma unroll
-      for (int j = 0; j < D - 1; ++j) {  // the last nst % D steps
-        if (k + j < nst) {
-          bf16x8_t A[4][RT][NS];
-          planes(buf[j], A);
-          mma_any(A, lbuf[j], (s0 + k + j) * kStep + g4 * 8);
-        }
-      }
+      for (int j = 0; j < D - 1; ++j)  // the last nst % D steps
+        if (k + j < nst) step(j, k + j, false);
     }
   } else {
     setup();
   }
 
-  bool bad = false;
-  if constexpr (TAB) {
-    // the ones column sees every cell of the row through the w plane, so a
-    // NaN marker anywhere in the K-range shows up in acc[2]
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bad |= __builtin_isnan(acc[2][rt][nt][e]);
-    bad = __ballot(bad) != 0;
-    if (bad) {  // |z| >= 64, inf or nan somewhere in the range: formulas, one step at a time
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) acc[i][rt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      for (int64_t st = s0; st < s1; ++st) {
-        bf16x8_t A[4][RT][NS];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          Raw8<DT> raw;
-          load_raw8<DT>(a.logits, rowoff[rt] + st * kStep, raw, vec);
-          bf16x8_t T[4][NS];
-          planes8_formula<DT, NS, false>(raw, ep, 8, false, T, ub[rt], up[rt]);
-#pragma unroll
-          for (int pl = 0; pl < 4; ++pl)
-#pragma unroll
-            for (int sp = 0; sp < NS; ++sp) A[pl][rt][sp] = T[pl][sp];
-        }
-        mma_step(A, *(const uint4*)(labp + st * kStep), st * kStep + g4 * 8);
-      }
-    }
-  }
-
+  const int64_t tail0 = full * kStep + g4 * 8;  // the tail step's first cell of this lane
   if (has_tail) {  // last partial step: guarded loads, masked planes
-    const int64_t st = full;
-    const int64_t cell0 = st * kStep + g4 * 8;
-    const int64_t nvalid = a.HW - cell0;
-    bf16x8_t A[4][RT][NS];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      Raw8<DT> raw;
-      uint32_t u[DT == ML_F32 ? 8 : 4];
-      const int64_t i0 = rowoff[rt] + st * kStep;
-#pragma unroll
-      for (int k = 0; k < (DT == ML_F32 ? 8 : 4); ++k) u[k] = 0;
-      if constexpr (DT == ML_F32) {
-        for (int k = 0; k < 8; ++k)
-          if (k < nvalid) u[k] = __float_as_uint(((const float*)a.logits)[i0 + k]);
-        raw.w[0] = make_uint4(u[0], u[1], u[2], u[3]);
-        raw.w[1] = make_uint4(u[4], u[5], u[6], u[7]);
-      } else {
-        for (int k = 0; k < 8; ++k)
-          if (k < nvalid)
-            u[k >> 1] |= (uint32_t)((const uint16_t*)a.logits)[i0 + k] << ((k & 1) * 16);
-        raw.w[0] = make_uint4(u[0], u[1], u[2], u[3]);
-      }
-      bf16x8_t T[4][NS];
-      planes8_formula<DT, NS, true>(raw, ep, nvalid, unw, T, ub[rt], up[rt]);
-#pragma unroll
-      for (int pl = 0; pl < 4; ++pl)
-#pragma unroll
-        for (int sp = 0; sp < NS; ++sp) A[pl][rt][sp] = T[pl][sp];
-    }
-    const uint4 lv = *(const uint4*)(labp + st * kStep);
-    mma_any(A, lv, cell0);
+    Raw8<DT> raw;
+    load_raw8_part<DT>(a.logits, rowoff + full * kStep, a.HW - tail0, raw);
+    f16x8_t A[4][NS];
+    planes8_formula<DT, NS, true>(raw, ep, a.HW - tail0, unw, A, ub, up);
+    BRaw x;
+    fetch_b(x, full);
+    uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
+    if constexpr (KEYS) tm = keys_of(x.lab, kp);
+    mma_step(A, x, kp, tm);
   }
 
-  if (red.buf) {
-    constexpr int TW = NP * RT * NT;  // float4 per lane per writer
+  // every non-finite or oversized plane shows in the sums of A_neg and A_pos
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < (SUMS ? 2 : 1); ++i)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad |= !(fabsf(acc[i][nt][e]) < INFINITY);
+  bad = __ballot(bad) != 0;
+  if (bad) {  // bf16 operands, one step at a time
+    constexpr int NR = InTraits<DT>::kRedo;
+    clear();
+    const int64_t last = has_tail ? full + 1 : s1;
+    for (int64_t st = s0; st < last; ++st) {
+      if (st >= s1 && st < full) continue;
+      Raw8<DT> raw;
+      const int64_t nv = a.HW - (st * kStep + g4 * 8);
+      load_raw8_part<DT>(a.logits, rowoff + st * kStep, nv, raw);
+      bf16x8_t A[4][NR];
+      planes8_redo<DT>(raw, ep, nv, A);
+      BRaw x;
+      fetch_b(x, st);
+      uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
+      if constexpr (KEYS) tm = keys_of(x.lab, kp);
+      for_tiles(x, kp, tm, [&](int nt, const u32x4_t& raw) {
+        const u32x4_t n = CNT == 1 ? widen8<0>(raw[0], raw[1]) : raw;
+        auto mul = [&](int i, int pl, const u32x4_t& v) {
+          // counts up to 255 are exact in bf16; larger ones as high and low byte
+          const bf16x8_t lo = CNT == 0 ? redo8(v, 0xFFFFu, 8) : redo8(v, 0xFFu), hi = redo8(v, 0xFF00u);
+#pragma unroll
+          for (int sp = 0; sp < NR; ++sp) {
+            acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[pl][sp], lo, acc[i][nt], 0, 0, 0);
+            if constexpr (CNT == 2)
+              acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[pl][sp], hi, acc[i][nt], 0, 0, 0);
+          }
+        };
+        const uint32_t all = CNT == 0 ? kHot * 0x10001u : n2pair;
+        if constexpr (SUMS) {
+  #pragma unroll
+        for (int pl = 0; pl < 4; ++pl) mul(pl, pl, n);
+        } else {
+          mul(0, 0, isub8(all, n));
+          mul(0, 1, n);
+          mul(1, 2, n);
+          mul(2, 3, n);
+        }
+      });
+    }
+  }
+  {
+    const float sc = bad ? 1.f : (CNT == 0 && TAB ? 65536.f : 1.f) / kPlaneScale;
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[i][nt] *= sc;
+  }
+
+  if constexpr (SUMS) if (red.buf) {
+    constexpr int TW = 2 * NT;  // float4 per lane per writer
     for (int h = red.R >> 1; h >= 1; h >>= 1) {
       const int64_t slot = red.grp * (red.R >> 1) + (red.r & (h - 1));
-      if (red.r >= h && red.r < 2 * h) {
-        f32x4_t* d = red.buf + slot * TW * 64 + lane;
+      f32x4_t* d = red.buf + slot * TW * 64 + lane;
 #pragma unroll
-        for (int i = 0; i < NP; ++i)
+      for (int ph = 0; ph < 2; ++ph) {
+        if (red.r >= h && red.r < 2 * h) {
 #pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-              if (nt < nt_used) d[((i * RT + rt) * NT + nt) * 64] = acc[i][rt][nt];
-        if (unw) {
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt) red.rsbuf[(slot * RT + rt) * 64 + lane] = make_float2(ub[rt], up[rt]);
+              if (nt < nt_used) d[(i * NT + nt) * 64] = acc[2 * ph + i][nt];
+          if (unw && ph == 0) red.rsbuf[slot * 64 + lane] = make_float2(ub, up);
         }
-      }
-      __syncthreads();
-      if (red.r < h) {
-        const f32x4_t* d = red.buf + slot * TW * 64 + lane;
+        __syncthreads();
+        if (red.r < h) {
 #pragma unroll
-        for (int i = 0; i < NP; ++i)
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-              if (nt < nt_used) acc[i][rt][nt] += d[((i * RT + rt) * NT + nt) * 64];
-        if (unw) {
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt) {
-            const float2 v = red.rsbuf[(slot * RT + rt) * 64 + lane];
-            ub[rt] += v.x;
-            up[rt] += v.y;
+              if (nt < nt_used) acc[2 * ph + i][nt] += d[(i * NT + nt) * 64];
+          if (unw && ph == 0) {
+            const float2 v = red.rsbuf[slot * 64 + lane];
+            ub += v.x;
+            up += v.y;
           }
         }
+        __syncthreads();
       }
-      __syncthreads();
     }
     if (red.r != 0) return;
   }
 
   // ---- write this wave's partial sums (only the tiles in use)
-  constexpr int rows = 16 * RT, nslot = 16 * NT;
+  constexpr int nslot = 16 * NT;
 #pragma unroll
   for (int i = 0; i < NP; ++i)
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
+    for (int nt = 0; nt < NT; ++nt) {
+      if (nt >= nt_used) continue;
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        if (nt >= nt_used) continue;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = rt * 16 + g4 * 4 + e;
-          out[(i * rows + row) * nslot + nt * 16 + r] = acc[i][rt][nt][e];
-        }
-      }
+      for (int e = 0; e < 4; ++e) out[(i * 16 + g4 * 4 + e) * nslot + nt * 16 + r] = acc[i][nt][e];
+    }
   if (unw) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      float vb = ub[rt], vp = up[rt];
-      // lanes r, r+16, r+32, r+48 hold the same row: fixed-order pair sums
-      vb += __shfl_xor(vb, 16, 64);
-      vp += __shfl_xor(vp, 16, 64);
-      vb += __shfl_xor(vb, 32, 64);
-      vp += __shfl_xor(vp, 32, 64);
-      if (g4 == 0) {
-        rs_out[(rt * 16 + r) * 2] = vb;
-        rs_out[(rt * 16 + r) * 2 + 1] = vp;
-      }
+    // lanes r, r+16, r+32, r+48 hold the same row: fixed-order pair sums
+    ub += __shfl_xor(ub, 16, 64);
+    up += __shfl_xor(up, 16, 64);
+    ub += __shfl_xor(ub, 32, 64);
+    up += __shfl_xor(up, 32, 64);
+    if (g4 == 0) {
+      rs_out[r * 2] = ub;
+      rs_out[r * 2 + 1] = up;
     }
   }
 }
@@ -785,18 +922,17 @@ constexpr int kClassOf = NT == 2 ? 0 : NT == 7 ? 1 : 2;
 // grid's groups is task u % n at partial u / n, its R waves take R
 // consecutive splits of the R * KS-way split and add their sums in LDS
 // (n * KS * R <= slots, so the groups fit the grid).
-template <int DT, int RT, int NT, int CNT, bool TAB>
+template <int DT, int NT, int CNT, bool TAB>
 __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs a) {
   constexpr int CI = kClassOf<NT>;
   constexpr int WV = cost_waves(NT, TAB);
   constexpr bool kRed = CI > 0;  // classes whose splits the schedule may group
-  constexpr bool SP = CNT == 0 && !TAB && NT >= 7;  // slot-sum form (see cost_wave)
-  constexpr int NP = SP ? 4 : 3;                    // planes per partial tile
+  constexpr bool KEYS = CNT == 0 && NT >= 7;
   __shared__ __align__(16) unsigned char lut_s[TAB ? kLutBytes : 16];
   __shared__ int prog_s[WV];
-  __shared__ f32x4_t red_s[kRed ? (WV / 2) * NP * RT * NT * 64 : 1];
-  __shared__ uint32_t klut_s[SP ? WV : 1][SP ? 260 : 1];
-  __shared__ float2 red_rs[kRed ? (WV / 2) * RT * 64 : 1];
+  __shared__ f32x4_t red_s[kRed ? (WV / 2) * 2 * NT * 64 : 1];
+  __shared__ uint32_t klut_s[KEYS ? WV : 1][KEYS ? 260 : 1];
+  __shared__ float2 red_rs[kRed ? (WV / 2) * 64 : 1];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t n = __builtin_amdgcn_readfirstlane(a.sched[CI]);
   const int64_t KS = __builtin_amdgcn_readfirstlane(a.sched[kClasses + CI]);
@@ -807,8 +943,8 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
     if constexpr (TAB) build_lut(lut_s, a.ep);
     __syncthreads();
   };
-  constexpr int64_t tile = NP * 16 * RT * 16 * NT;
-  uint32_t* klut = SP ? &klut_s[SP ? wave : 0][0] : nullptr;
+  constexpr int64_t tile = class_planes(CI) * 16 * 16 * NT;
+  uint32_t* klut = KEYS ? &klut_s[KEYS ? wave : 0][0] : nullptr;
   if (kRed && R > 1) {
     const int gpw = WV / R;  // groups per workgroup
     const int grp = wave / R, r = wave - grp * R;
@@ -817,25 +953,22 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
     const int64_t u = u0 + grp;
     if (u >= total) {  // an idle group still meets every barrier of the others
       setup();
-      for (int h = R >> 1; h >= 1; h >>= 1) {
-        __syncthreads();
-        __syncthreads();
-      }
+      for (int h = R >> 1; h >= 1; h >>= 1)
+        for (int k = 0; k < kRedBarriers; ++k) __syncthreads();
       return;
     }
     const int64_t i = u % n, kp = u / n;
     const int64_t task = __builtin_amdgcn_readfirstlane(a.sched[kSchedList + CI * a.plan.ntasks + i]);
     const int64_t lb = task / a.rtiles, rtile = task % a.rtiles;
     float* out = a.partials + a.plan.float_base[CI] + u * tile;
-    float* rs = a.rowsum ? a.rowsum + (a.plan.slot_base[CI] + u) * (16 * RT) * 2 : nullptr;
+    float* rs = a.rowsum ? a.rowsum + (a.plan.slot_base[CI] + u) * 16 * 2 : nullptr;
     SplitRed red;
     red.buf = red_s;
     red.rsbuf = red_rs;
     red.R = R;
     red.r = r;
     red.grp = grp;
-    cost_wave<DT, RT, NT, CNT, TAB>(a, lb, rtile, kp * R + r, KS * R, lut_s, out, rs, nullptr, setup, red,
-                                    klut);
+    cost_wave<DT, NT, CNT, TAB>(a, lb, rtile, kp * R + r, KS * R, lut_s, out, rs, nullptr, setup, red, klut);
     return;
   }
   const int64_t w0 = (int64_t)blockIdx.x * WV;
@@ -850,33 +983,53 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
   const int64_t task = __builtin_amdgcn_readfirstlane(a.sched[kSchedList + CI * a.plan.ntasks + i]);
   const int64_t lb = task / a.rtiles, rtile = task % a.rtiles;
   float* out = a.partials + a.plan.float_base[CI] + w * tile;
-  float* rs = a.rowsum ? a.rowsum + (a.plan.slot_base[CI] + w) * (16 * RT) * 2 : nullptr;
+  float* rs = a.rowsum ? a.rowsum + (a.plan.slot_base[CI] + w) * 16 * 2 : nullptr;
   // pace the waves only where many share the workgroup's CU
-  cost_wave<DT, RT, NT, CNT, TAB>(a, lb, rtile, ks, KS, lut_s, out, rs, WV >= 16 ? prog_s : nullptr,
-                                  setup, SplitRed(), klut);
+  cost_wave<DT, NT, CNT, TAB>(a, lb, rtile, ks, KS, lut_s, out, rs, WV >= 16 ? prog_s : nullptr, setup,
+                              SplitRed(), klut);
 }
 
-// ---- bf16 table path with LDS-staged logits (16-row tiles, <= 32 columns) ------
-// HBM streams a row best in long runs, while a 16x16x32 MFMA operand spreads
-// one K-step over 16 rows (64 bytes each).  So the logits go through LDS: a
-// group of 4 K-steps (16 rows x 128 cells, 4 KB) is fetched by four
-// global_load_lds_dwordx4, each moving 1 KB as 4 rows x 256 contiguous bytes
-// straight into the wave's LDS ring, and read back in the operand layout with
-// one ds_read_b128 per K-step.  Instruction i, lane l fetches the 16-byte
-// chunk c = (l & 15) ^ R of row R = 4 i + (l >> 4); the hardware stores lane
-// l at ring slot 64 i + l = 16 R + (c ^ R), so the reader of K-step s (lane
-// (r, g4) wants chunk 4 s + g4 of row r) finds it at slot
-// 16 r + ((4 s + g4) ^ r), and the 16 lanes of each read phase touch 16
-// different bank groups.  The ring holds kRingGroups groups, so a group's
-// fetch is in flight while the previous one is computed, without costing
-// registers.  Work items are ordered task-fastest (see row_partials_at), so
-// a workgroup's 16 waves stream 16 adjacent row tiles at the same offset.
+// ---- class 0 of bf16 table calls: row-tile pairs, 32x32x16 products ------------
+// One wave takes 32 query rows (row tiles 2k and 2k + 1 of one image) and the
+// 32 column slots of class 0 over its K-range, in K-steps of 16 cells: lane
+// (r = lane & 31, h = lane >> 5) holds 8 cells of the step for query row r (A
+// operand) and for column slot r (B operand), and its accumulators hold
+// column r at rows 8 (v / 4) + 4 h + v % 4 of register v.
 //
-// LDS map of a 16-wave workgroup: positive table block [0, 8 kLutBlock), the
+// HBM streams a row best in long runs, so the logits go through LDS: a group
+// of 4 K-steps (32 rows x 64 cells, 4 KB) is fetched by four
+// global_load_lds_dwordx4, each moving 1 KB as 8 rows x 128 contiguous bytes
+// straight into the wave's LDS ring, and read back in the operand layout with
+// one ds_read_b128 per K-step.  Instruction i has lane l load row R = 8 i +
+// (l >> 3) at 16-byte chunk c = (l & 7) ^ (R & 7); the hardware stores lane l
+// at ring slot 64 i + l = 8 R + (c ^ (R & 7)), so the 8 lanes of each read phase
+// (8 consecutive rows, one chunk) touch 8 different bank groups.  The ring
+// holds kRingGroups groups, so a group's fetch is in flight while the previous
+// one is computed, without costing registers.
+//
+// Label maps: K-step s of a group holds cells 16 s + 8 h + (0 .. 7), and the
+// labels are loaded a group ahead.  u8 counts: the K-steps of a group may hold its
+// 64 cells in any order that both operands share, so K-step s holds cells 32 h +
+// 8 s + (0 .. 7) and a lane's counts of the whole group are 32 consecutive bytes
+// (two 16-byte loads, the wave's a run of 2 KB).
+//
+// A workgroup is 4 pairs x 4 adjacent K-splits (wave = 4 pair + split): the
+// four splits of a pair are summed in LDS at the end, in the fixed order
+// (s0 + s2) + (s1 + s3), and only that sum is written, so the partial sums
+// that reach memory (and the finalize's reads of them) are a quarter of one
+// tile per wave.  The schedule's class-0 split count is the number of such
+// quads, KSq; the kernel runs 4 KSq K-ranges.
+//
+// Bound by vector-ALU issue (59 ops per K-step of 512 logits), LDS table reads and
+// load latency at 4 waves per SIMD: 210 M logits against label maps 102 -> 97 us
+// (bf16 operands took 65 ops per K-step), 671 M against u8 counts of 4x targets 314 us
+// (with the 7-tile class's 94 us; 886 + 208 us on the formula path).
+//
+// LDS map of the 16-wave workgroup: positive table block [0, 8 kLutBlock), the
 // rings of waves 0 and 1 in the gap before the negative block at kLutNegOff,
 // the negative block, then the rings of waves 2..15 (163,072 bytes).
 constexpr int kGroupSteps = 4;            // K-steps per group
-constexpr uint32_t kGroupBytes = 4096;    // 16 rows x 128 cells x 2 bytes
+constexpr uint32_t kGroupBytes = 4096;    // 32 rows x 64 cells x 2 bytes
 constexpr int kRingGroups = 2;
 constexpr uint32_t kRingBytes = kRingGroups * kGroupBytes;
 constexpr uint32_t kDmaWaves = 16;
@@ -889,7 +1042,7 @@ constexpr uint32_t kDmaLds =
 static_assert(kDmaLds <= 160 * 1024, "table and rings fit the LDS of one CU");
 
 // Ring bases are 256-byte aligned, so a reader's address of K-step s is its
-// step-0 address with bits 6-7 flipped: (4 s + g4) ^ r = (g4 ^ r) ^ 4 s.
+// step-0 address with bits of s flipped (see cost_wave_pair).
 constexpr uint32_t kRingLo = (kLutBlockBytes + 255) & ~255u;
 constexpr uint32_t kRingHi = (kLutNegOff + kLutBlockBytes + 255) & ~255u;
 __device__ __forceinline__ uint32_t ring_base(int wave) {
@@ -902,35 +1055,16 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // assembly: the compiler would otherwise wait for every outstanding fetch
 // before any LDS read, since it cannot tell which ring slot a
 // global_load_lds writes.
-__device__ __forceinline__ uint4 ring_read(uint32_t addr) {
-  uint4 v;
+__device__ __forceinline__ u32x4_t ring_read(uint32_t addr) {
+  u32x4_t v;
   asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(addr) : "memory");
   return v;
 }
 
-typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ u16x2_t as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2_t, v); }
-__device__ __forceinline__ uint32_t as_u32(u16x2_t v) { return __builtin_bit_cast(uint32_t, v); }
-
-// Table byte offsets (sign block included) of the two bf16 logits packed in
-// u, as lut_lookup8 computes them, in compiler-visible packed 16-bit ops (no
-// inline assembly, so no hazard padding after each one): the clamped index
-// times 8 stays below 2^15, so the sign bit ORs in without carry.
-__device__ __forceinline__ uint32_t lut_addr_pair(uint32_t u) {
-  const u16x2_t m = as_u16x2(u & 0x7FFF7FFFu);
-  const u16x2_t idx = __builtin_elementwise_min(
-      __builtin_elementwise_sub_sat(m, (u16x2_t){(unsigned short)kLutSub, (unsigned short)kLutSub}),
-      (u16x2_t){(unsigned short)(kLutN + 1), (unsigned short)(kLutN + 1)});
-  uint32_t addr = (u & 0x80008000u) | as_u32(idx << (u16x2_t){3, 3});
-  // kept whole, so its two halves are one mask and one shift of it
-  asm("" : "+v"(addr));
-  return addr;
-}
-
 // Table entries of 8 bf16 cells (as lut_lookup8) read with assembly, and the
 // wait for them tied to their registers.  lut_base: the table's LDS address.
-__device__ __forceinline__ void lut_lookup8_asm(const uint4& x, uint32_t lut_base, uint64_t E[8]) {
-  const uint32_t u[4] = {x.x, x.y, x.z, x.w};
+__device__ __forceinline__ void lut_lookup8_asm(const u32x4_t& x, uint32_t lut_base, uint64_t E[8]) {
+  const uint32_t u[4] = {x[0], x[1], x[2], x[3]};
   uint32_t ad[4];  // the four words' chains side by side, then the reads
 #pragma unroll
   for (int i = 0; i < 4; ++i) ad[i] = lut_addr_pair(u[i]);
@@ -942,299 +1076,75 @@ __device__ __forceinline__ void lut_lookup8_asm(const uint4& x, uint32_t lut_bas
   }
 }
 // Wait for every outstanding LDS read; E (table entries) and x (ring words
-// read earlier) are tied to it, so nothing that uses them moves above it.
-__device__ __forceinline__ void lds_wait(uint64_t E[8], uint4& x) {
+// read earlier) are tied to it, so nothing that uses them moves above it.  Each
+// is tied as the whole register group that its read writes: split into words, the
+// compiler may copy them while the read is in flight.
+__device__ __forceinline__ void lds_wait(uint64_t E[8], u32x4_t& x) {
   asm volatile("s_waitcnt lgkmcnt(0)"
                : "+v"(E[0]), "+v"(E[1]), "+v"(E[2]), "+v"(E[3]), "+v"(E[4]), "+v"(E[5]), "+v"(E[6]),
-                 "+v"(E[7]), "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
+                 "+v"(E[7]), "+v"(x));
 }
 // Wait for every outstanding LDS read at the end of a pipeline; the
 // registers of reads nothing consumes are tied to it, so they stay reserved
 // until the data has landed.
-__device__ __forceinline__ void lds_drain(uint64_t E[8], uint4 (&x)[2]) {
+__device__ __forceinline__ void lds_drain(uint64_t E[8], u32x4_t (&x)[2]) {
   asm volatile("s_waitcnt lgkmcnt(0)"
                : "+v"(E[0]), "+v"(E[1]), "+v"(E[2]), "+v"(E[3]), "+v"(E[4]), "+v"(E[5]), "+v"(E[6]),
-                 "+v"(E[7]), "+v"(x[0].x), "+v"(x[0].y), "+v"(x[0].z), "+v"(x[0].w), "+v"(x[1].x),
-                 "+v"(x[1].y), "+v"(x[1].z), "+v"(x[1].w)
+                 "+v"(E[7]), "+v"(x[0]), "+v"(x[1])
                :
                : "memory");
 }
 // One ds_read_b128 of the ring, not waited for (see lds_wait).
-__device__ __forceinline__ uint4 ring_read_async(uint32_t addr) {
-  uint4 v;
+__device__ __forceinline__ u32x4_t ring_read_async(uint32_t addr) {
+  u32x4_t v;
   asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
   return v;
 }
-__device__ __forceinline__ void lut_planes64(const uint64_t E64[8], bf16x8_t A[4]) {
+__device__ __forceinline__ void lut_planes64(const uint64_t E64[8], f16x8_t A[4]) {
   uint2 E[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) E[i] = make_uint2((uint32_t)E64[i], (uint32_t)(E64[i] >> 32));
   lut_planes(E, A);
 }
-// 16 bytes of labels, loaded with assembly; label_wait<N> waits until at most
-// N vector-memory operations issued after it are outstanding.
-__device__ __forceinline__ u32x4_t label_load(const void* p) {
+// 16 bytes of labels or counts from base + off + OFF, loaded with assembly (a
+// wave-uniform base and a 32-bit lane offset: one address register);
+// label_wait<N> waits until at most N vector-memory operations issued after it
+// are outstanding.
+template <int OFF>
+__device__ __forceinline__ u32x4_t label_load(const void* base, uint32_t off) {
+  // (a uniform value that the compiler keeps in vector registers would not fit
+  // the scalar operand)
+  const uint64_t u = (uint64_t)(uintptr_t)base;
+  const uint64_t sb = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u) |
+                      ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32)) << 32);
   u32x4_t v;
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(v) : "v"(p) : "memory");
+  asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(v) : "v"(off), "s"(sb), "n"(OFF) : "memory");
   return v;
 }
 template <int N>
 __device__ __forceinline__ void label_wait(u32x4_t& v) {
   asm volatile("s_waitcnt vmcnt(%1)" : "+v"(v) : "n"(N));
 }
-// Drain every vector-memory operation; the label registers are tied to it,
+// Drain every vector-memory operation; the operand registers are tied to it,
 // so loads issued but never used (the pipeline's last ones) keep their
 // registers until they have landed (an assembly load's destination would
 // otherwise count as free at once and could be reused while it is in flight).
-__device__ __forceinline__ void drain_loads(u32x4_t (&l)[4]) {
-  asm volatile("s_waitcnt vmcnt(0)" : "+v"(l[0]), "+v"(l[1]), "+v"(l[2]), "+v"(l[3]) : : "memory");
+template <int N>
+__device__ __forceinline__ void drain_loads(u32x4_t (&l)[N]) {
+  if constexpr (N == 4)
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(l[0]), "+v"(l[1]), "+v"(l[2]), "+v"(l[3]) : : "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(l[0]), "+v"(l[1]) : : "memory");
 }
 
-template <int NT, class Setup>
-__device__ __forceinline__ void cost_wave_dma(const CostArgs& a, int64_t lb, int64_t rtile,
-                                              int64_t ks, int64_t KS, const unsigned char* lut,
-                                              uint32_t ring, float* out, Setup&& setup) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15, g4 = lane >> 4;
-  const int64_t b = lb % a.B;
-  const int G = __builtin_amdgcn_readfirstlane(a.ncols[b]);
-  const int nt_used = (G + 1 + 15) >> 4;
-  const int64_t q0 = rtile * 16;
-
-  uint32_t colL[NT], coefB[NT], baseB[NT];
-  const uint32_t n2pair = pack_bf16x2(a.N2, a.N2);
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int slot = nt * 16 + r;
-    colL[nt] = 0;
-    coefB[nt] = slot < G ? 0x3F803F80u : 0u;
-    baseB[nt] = slot < G ? 0x3F803F80u : (slot == G ? n2pair : 0u);
-    if (slot < G) {
-      const int c = a.colmap[b * a.nslot + slot];
-      const int act = c + (c >= a.bg ? 1 : 0);
-      colL[nt] = (uint32_t)act * 0x10001u;
-    }
-  }
-  f32x4_t acc[3][NT];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[i][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // this wave's K-steps: whole groups [g0, g1) of the row's full K-steps
-  const int64_t full = a.HW / kStep;
-  const int64_t ngr = ceil_div(full, kGroupSteps);
-  const int64_t gper = ceil_div(ngr, KS);
-  const int64_t g0 = min(ngr, ks * gper), g1 = min(ngr, g0 + gper);
-  const int64_t s0 = g0 * kGroupSteps;
-  const int nst = (int)(min(full, g1 * kGroupSteps) - s0);
-  const bool has_tail = (a.HW % kStep) != 0 && ks == KS - 1;
-
-  // fetch sources: instruction i of a group reads row R = 4 i + (lane >> 4)
-  // (clamped to the last query) at chunk (lane & 15) ^ R; element offsets
-  // from zrow0 stay below 2^31 (host check)
-  const uint16_t* zrow0 = (const uint16_t*)a.logits + (lb * a.Q + q0) * a.HW;
-  const uint32_t HW32 = (uint32_t)a.HW, qlast = (uint32_t)(a.Q - 1 - q0);
-  auto fetch_group = [&](int slot, int64_t g) {  // g in [g0, g1)
-    const uint32_t cell0 = (uint32_t)(g * (kGroupSteps * kStep));
-    const bool edge = cell0 + kGroupSteps * kStep > HW32;  // wave-uniform
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t R = 4u * i + g4;
-      uint32_t cell = cell0 + 8u * (((uint32_t)lane & 15u) ^ R);
-      if (edge) cell = min(cell, HW32 - 8u);  // past the row end: its last chunk (never used)
-      const uint32_t off = min(R, qlast) * HW32 + cell;
-      __builtin_amdgcn_global_load_lds((const void*)(zrow0 + off),
-                                       (lds_void_t*)(size_t)(ring + slot * kGroupBytes + i * 1024), 16, 0, 0);
-    }
-  };
-  // reader of K-step s: ring + slot * kGroupBytes + 16 (16 r + ((4 s + g4) ^ r))
-  const uint32_t rd = ring + 16u * (16u * r + ((uint32_t)g4 ^ (uint32_t)r));
-  auto step_addr = [&](int t) {
-    const int s = t & (kGroupSteps - 1), slot = (t / kGroupSteps) & (kRingGroups - 1);
-    return (rd ^ (64u * s)) + slot * kGroupBytes;
-  };
-  const uint16_t* labp = a.lab16 + b * a.HWp + g4 * 8;
-  u32x4_t lbuf[kGroupSteps];
-  auto fetch_l = [&](int j, int t) {
-    const int64_t st = s0 + (t < nst ? t : nst - 1);
-    lbuf[j] = label_load(labp + st * kStep);
-  };
-
-  auto mma = [&](const bf16x8_t (&A)[4], const uint4& lv) {
-    const uint32_t L2[4] = {lv.x, lv.y, lv.z, lv.w};
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      if (nt >= nt_used) continue;
-      u32x4_t bp, bv;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t m = pk_min_u16(L2[i] ^ colL[nt], 0x00010001u);
-        bp[i] = pk_mul_lo_u16(m, coefB[nt]);
-        bv[i] = pk_sub_u16(baseB[nt], bp[i]);
-      }
-      const bf16x8_t Bp = __builtin_bit_cast(bf16x8_t, bp);
-      const bf16x8_t Bv = __builtin_bit_cast(bf16x8_t, bv);
-      acc[0][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0], Bp, acc[0][nt], 0, 0, 0);
-      acc[0][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1], Bv, acc[0][nt], 0, 0, 0);
-      acc[1][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[2], Bv, acc[1][nt], 0, 0, 0);
-      acc[2][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[3], Bv, acc[2][nt], 0, 0, 0);
-    }
-  };
-
-  // Every load of the pipeline is issued in this order, so the vmcnt waits
-  // below are exact: labels of steps 0..3, groups 0 and 1; then per step t:
-  // [refill of this group's slot (s = 3)] [label of step t + 4].  The label
-  // of step t is then followed by exactly (near the start: at least) 7 later
-  // loads when it is used, and a group's fetch by at least 2 when its first
-  // step is read from the ring (two steps before that step).  LDS reads run
-  // two steps ahead for the ring and one for the table: step t waits for
-  // both (lds_wait), then issues the ring read of step t + 2 and the table
-  // reads of step t + 1.
-  if (nst > 0) {
-    const int ngl = (int)(g1 - g0);
-    const uint32_t lut_base = (uint32_t)(size_t)(lds_void_t*)lut;
-#pragma unroll
-    for (int j = 0; j < kGroupSteps; ++j) fetch_l(j, j);
-    fetch_group(0, g0);
-    fetch_group(1, g0 + (ngl > 1 ? 1 : 0));
-    setup();
-    __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): group 0 landed (group 1 may be in flight)
-    uint64_t E[8];
-    uint4 xr[2];  // ring words of steps t + 1 (xr[(t + 1) & 1]) and t + 2
-    lut_lookup8_asm(ring_read(step_addr(0)), lut_base, E);
-    xr[1] = nst > 1 ? ring_read_async(step_addr(1)) : make_uint4(0u, 0u, 0u, 0u);
-    for (int t0 = 0; t0 < nst; t0 += kGroupSteps) {
-#pragma unroll
-      for (int s = 0; s < kGroupSteps; ++s) {  // s compile-time: lbuf and xr stay in registers
-        const int t = t0 + s;
-        if (t < nst) {
-          uint4& xn = xr[(s + 1) & 1];  // step t + 1
-          uint4& xnn = xr[s & 1];       // step t + 2
-          lds_wait(E, xn);
-          bf16x8_t A[4];
-          lut_planes64(E, A);
-          if (t + 1 < nst) lut_lookup8_asm(xn, lut_base, E);
-          if (t + 2 < nst) {
-            if (s == kGroupSteps - 2)  // step t + 2 opens the next group: its fetch has landed
-              __builtin_amdgcn_s_waitcnt(0x0F72);  // when at most 2 later loads are pending
-            xnn = ring_read_async(step_addr(t + 2));
-          }
-          if (s == kGroupSteps - 1) {  // every step of this slot is read: refill it two groups on
-            const int k = t0 / kGroupSteps;
-            fetch_group(k & (kRingGroups - 1), g0 + min(k + kRingGroups, ngl - 1));
-          }
-          label_wait<7>(lbuf[s]);
-          __builtin_amdgcn_sched_barrier(0);
-          mma(A, __builtin_bit_cast(uint4, lbuf[s]));
-          __builtin_amdgcn_sched_barrier(0);
-          fetch_l(s, t + kGroupSteps);
-        }
-      }
-    }
-    drain_loads(lbuf);  // also: no fetch may land in LDS after the wave ends
-  } else {
-    setup();
-  }
-
-  // |z| >= 64, inf or nan somewhere in the range (the ones column's w plane
-  // sees every cell): formulas, one step at a time
-  bool bad = false;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bad |= __builtin_isnan(acc[2][nt][e]);
-  bad = __ballot(bad) != 0;
-  const ElemParams ep = a.ep;
-  const int64_t rowoff = (lb * a.Q + min(q0 + r, a.Q - 1)) * a.HW + g4 * 8;
-  auto formula_step = [&](int64_t st, int64_t nvalid) {
-    Raw8<ML_BF16> raw;
-    const uint16_t* zp = (const uint16_t*)a.logits + rowoff + st * kStep;
-    uint32_t u[4] = {0u, 0u, 0u, 0u};
-    for (int k = 0; k < 8; ++k)
-      if (k < nvalid) u[k >> 1] |= (uint32_t)zp[k] << ((k & 1) * 16);
-    raw.w[0] = make_uint4(u[0], u[1], u[2], u[3]);
-    bf16x8_t T[4][1];
-    float ub = 0.f, up = 0.f;
-    if (nvalid >= 8) planes8_formula<ML_BF16, 1, false>(raw, ep, 8, false, T, ub, up);
-    else planes8_formula<ML_BF16, 1, true>(raw, ep, nvalid, false, T, ub, up);
-    const bf16x8_t A[4] = {T[0][0], T[1][0], T[2][0], T[3][0]};
-    mma(A, *(const uint4*)(labp + st * kStep));
-  };
-  if (bad) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[i][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int64_t st = s0; st < s0 + nst; ++st) formula_step(st, 8);
-  }
-  if (has_tail) formula_step(full, a.HW - (full * kStep + g4 * 8));
-
-  constexpr int nslot = 16 * NT;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      if (nt >= nt_used) continue;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) out[(i * 16 + g4 * 4 + e) * nslot + nt * 16 + r] = acc[i][nt][e];
-    }
-}
-
-template <int NT>
-__global__ __launch_bounds__(64 * kDmaWaves) void cost_dma_kernel(CostArgs a) {
-  constexpr int CI = kClassOf<NT>;
-  __shared__ __align__(16) unsigned char lds[kDmaLds];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t n = __builtin_amdgcn_readfirstlane(a.sched[CI]);
-  const int64_t KS = __builtin_amdgcn_readfirstlane(a.sched[kClasses + CI]);
-  const int64_t total = n * KS;
-  const int64_t w0 = (int64_t)blockIdx.x * kDmaWaves;
-  if (w0 >= total) return;  // the whole workgroup is idle
-  auto setup = [&]() {
-    build_lut(lds, a.ep);
-    __syncthreads();
-  };
-  const int64_t w = w0 + wave;
-  if (w >= total) {
-    setup();
-    return;
-  }
-  const int64_t i = w % n, ks = w / n;
-  const int64_t task = __builtin_amdgcn_readfirstlane(a.sched[kSchedList + CI * a.plan.ntasks + i]);
-  const int64_t lb = task / a.rtiles, rtile = task % a.rtiles;
-  constexpr int64_t tile = 3 * 16 * 16 * NT;
-  float* out = a.partials + a.plan.float_base[CI] + w * tile;
-  const uint32_t ring = (uint32_t)(size_t)(lds_void_t*)lds + ring_base(wave);
-  cost_wave_dma<NT>(a, lb, rtile, ks, KS, lds, ring, out, setup);
-}
-
-// ---- class 0 as row-tile pairs: 32x32x16 products ------------------------------
-// One wave takes 32 query rows (row tiles 2k and 2k + 1 of one image) and the
-// 32 column slots of class 0 over its K-range, in K-steps of 16 cells:
-// lane (r = lane & 31, h = lane >> 5) holds cells 8 h .. 8 h + 7 of the step
-// for query row r (A operand) and for column slot r (B operand), and its
-// accumulators hold column r at rows 8 (v / 4) + 4 h + v % 4 of register v.
-// Against the 16-row kernel, one B operand (the label compare) now serves 32
-// query rows, which halves the vector-ALU work of the column side per logit.
-// Logits go through the same LDS ring: a group is 4 K-steps (64 cells) of the
-// 32 rows, 128 bytes per row; instruction i of a group fetch has lane l load
-// row R = 8 i + (l >> 3) at chunk c = (l & 7) ^ (R & 7) into slot
-// 8 R + (c ^ (R & 7)), so the 8 lanes of each ds_read_b128 phase (8
-// consecutive rows, one chunk) touch 8 different bank groups.
-//
-// A workgroup is 4 pairs x 4 adjacent K-splits (wave = 4 pair + split): the
-// four splits of a pair are summed in LDS at the end, in the fixed order
-// (s0 + s2) + (s1 + s3), and only that sum is written, so the partial sums
-// that reach memory (and the finalize's reads of them) are a quarter of one
-// tile per wave.  The schedule's class-0 split count is the number of such
-// quads, KSq; the kernel runs 4 KSq K-ranges.
 constexpr int kPairStep = 16;                               // cells per K-step
 constexpr int kPairGroupCells = kGroupSteps * kPairStep;    // 64 cells x 32 rows = 4 KB
-constexpr int64_t kPairTile = 3 * 32 * 32;                  // partial tile (floats)
+constexpr int64_t kPairTile = 3 * 32 * 32;            // partial tile (floats)
 static_assert(kPairGroupCells * 32 * 2 == (int)kGroupBytes, "a pair group fills one ring slot");
+static_assert(kPairGroupCells == kCountCells, "a group's counts are one block");
 
-template <class Setup>
+// CNT: 0 label map, 1 u8 counts
+template <int CNT, class Setup>
 __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, int64_t q0, int64_t ks,
                                                int64_t KS, const unsigned char* lut, uint32_t ring,
                                                f32x16_t (&acc)[3], Setup&& setup) {
@@ -1243,27 +1153,35 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
   const int64_t b = lb % a.B;
   const int G = __builtin_amdgcn_readfirstlane(a.ncols[b]);
 
-  // column operand of slot r (see cost_wave): real columns compare labels,
-  // slot G is the ones column, the rest is padding
-  uint32_t colL = 0;
-  const uint32_t coefB = r < G ? 0x3F803F80u : 0u;
-  const uint32_t baseB = r < G ? 0x3F803F80u : (r == G ? pack_bf16x2(a.N2, a.N2) : 0u);
+  // the lane's column: its label pair and mask, or its row of the count tiles (see cost_wave)
+  int act = -1;
   if (r < G) {
     const int c = a.colmap[b * a.nslot + r];
-    colL = (uint32_t)(c + (c >= a.bg ? 1 : 0)) * 0x10001u;
+    act = c + (c >= a.bg ? 1 : 0);
   }
+  const uint32_t colL = act >= 0 ? label_code(act) * 0x10001u : 0u;
+  uint32_t colM = r == G ? 0u : 0xFFFFFFFFu;
+  asm("" : "+v"(colM));  // a register, not a select at every use
+  const int64_t cstep = (int64_t)a.counts.rows * kCountCells;  // bytes per block of counts
+  const uint8_t* cimg = CNT ? a.counts.p + b * a.counts.nb * cstep : nullptr;
+  const uint32_t crow = (uint32_t)(act >= 0 ? act : (int)a.GT_total + 1) * kCountCells;
+  auto clear = [&]() {
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+      for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+  };
+  clear();
 
-  const int64_t full = a.HW / kPairStep;
+  const uint32_t top = (uint32_t)__builtin_amdgcn_readfirstlane((int)opnd_top(a.N2));
+  // full K-steps of this split (whole groups with counts), then the tail
+  const int64_t full = CNT ? a.HW / kPairGroupCells * kGroupSteps : a.HW / kPairStep;
   const int64_t ngr = ceil_div(full, kGroupSteps);
   const int64_t gper = ceil_div(ngr, KS);
   const int64_t g0 = min(ngr, ks * gper), g1 = min(ngr, g0 + gper);
   const int64_t s0 = g0 * kGroupSteps;
   const int nst = (int)(min(full, g1 * kGroupSteps) - s0);
-  const bool has_tail = (a.HW % kPairStep) != 0 && ks == KS - 1;
+  const int64_t steps = ks == KS - 1 ? ceil_div(a.HW, kPairStep) : full;  // past `full`: this split's tail
 
   // fetch sources: rows past the last query read the last query's row
   // (never used); element offsets from zrow0 stay below 2^31 (host check)
@@ -1277,67 +1195,84 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
       const uint32_t R = 8u * i + ((uint32_t)lane >> 3);
       uint32_t cell = cell0 + 8u * (((uint32_t)lane & 7u) ^ (R & 7u));
       if (edge) cell = min(cell, HW32 - 8u);  // past the row end: its last chunk (never used)
-      const uint32_t off = min(R, qlast) * HW32 + cell;
-      __builtin_amdgcn_global_load_lds((const void*)(zrow0 + off),
+      // bytes below 2^32: a scalar base and a 32-bit lane offset
+      const uint32_t off = (min(R, qlast) * HW32 + cell) * 2u;
+      __builtin_amdgcn_global_load_lds((const void*)((const char*)zrow0 + off),
                                        (lds_void_t*)(size_t)(ring + slot * kGroupBytes + i * 1024), 16, 0, 0);
     }
   };
-  // reader of K-step s: ring + slot * kGroupBytes + 128 r + 16 ((2 s + h) ^ (r & 7));
-  // the ring is 256-byte aligned, so that is the step-0 address with bits 5-6
-  // flipped by 2 s
-  const uint32_t rd = ring + 128u * r + 16u * ((uint32_t)h ^ ((uint32_t)r & 7u));
+  // reader of K-step s of a group: ring + slot * kGroupBytes + 128 r + 16 (c ^ (r & 7))
+  // for chunk c = 2 s + h (labels) or 4 h + s (counts); the ring is 256-byte
+  // aligned, so that is the step-0 address with bits 5-6 or 4-5 flipped by s
+  const uint32_t rd = ring + 128u * r + 16u * ((uint32_t)(CNT ? 4 * h : h) ^ ((uint32_t)r & 7u));
   auto step_addr = [&](int t) {
     const int s = t & (kGroupSteps - 1), slot = (t / kGroupSteps) & (kRingGroups - 1);
-    return (rd ^ (32u * s)) + slot * kGroupBytes;
+    return (rd ^ ((CNT ? 16u : 32u) * s)) + slot * kGroupBytes;
   };
-  const uint16_t* labp = a.lab16 + b * a.HWp + h * 8;
-  u32x4_t lbuf[kGroupSteps];
+  const uint16_t* labp = a.lab16 + (CNT ? 0 : b * a.HWp);
+  u32x4_t lbuf[CNT ? 2 : kGroupSteps];  // labels of 4 K-steps, or counts of K-steps 0, 1 and 2, 3
   auto fetch_l = [&](int j, int t) {
-    const int64_t st = s0 + (t < nst ? t : nst - 1);
-    lbuf[j] = label_load(labp + st * kPairStep);
+    // t opaque: min(1, nst - 1) would become a vector select, and its readfirstlane
+    // sit right before the load that uses it (a hazard inside assembly)
+    asm("" : "+s"(t));
+    const int64_t st = s0 + min(t, nst - 1);
+    lbuf[j] = label_load<0>(labp + st * kPairStep, 16u * h);
+  };
+  auto fetch_c = [&](int j, int64_t g) {
+    const uint8_t* p = cimg + min(g, g1 - 1) * cstep;
+    lbuf[j] = j ? label_load<16>(p, crow + 32u * h) : label_load<0>(p, crow + 32u * h);
   };
 
-  auto mma = [&](const bf16x8_t (&A)[4], const uint4& lv) {
-    const uint32_t L2[4] = {lv.x, lv.y, lv.z, lv.w};
-    u32x4_t bp, bv;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t m = pk_min_u16(L2[i] ^ colL, 0x00010001u);
-      bp[i] = pk_mul_lo_u16(m, coefB);
-      bv[i] = pk_sub_u16(baseB, bp[i]);
-    }
-    const bf16x8_t Bp = __builtin_bit_cast(bf16x8_t, bp);
-    const bf16x8_t Bv = __builtin_bit_cast(bf16x8_t, bv);
-    acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0], Bp, acc[0], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[2], Bv, acc[1], 0, 0, 0);
-    acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[3], Bv, acc[2], 0, 0, 0);
-    acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[1], Bv, acc[0], 0, 0, 0);
+  auto mma = [&](const f16x8_t (&A)[4], const Opnd& o) {
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], o.rest, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[2], o.n, acc[1], 0, 0, 0);
+    acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[3], o.n, acc[2], 0, 0, 0);
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], o.n, acc[0], 0, 0, 0);
   };
 
-  // The pipeline and its wait counts are those of cost_wave_dma: per K-step
-  // one label load, per group one 4-instruction fetch, in the same order.
+  // Every load of the pipeline is issued in a fixed order, so the vmcnt waits
+  // below are exact.
+  //   Labels: labels of steps 0..3, groups 0 and 1; then per step t:
+  //   [refill of this group's slot (s = 3)] [label of step t + 4].  The label
+  //   of step t is then followed by exactly (near the start: at least) 7 later
+  //   loads when it is used, and a group's fetch by at least 2 when its first
+  //   step is read from the ring (two steps before that step).
+  //   Counts: half 0 of group 0, groups 0 and 1, half 1 of group 0; then in group
+  //   k: [half 0 of k + 1, after step 1 used it] [refill (s = 3)] [half 1 of
+  //   k + 1, after step 3].  Half 0 is followed by 5 later loads when step 0
+  //   uses it; half 1 by 1 when step 2 does, and group k + 1's fetch is older.
+  // LDS reads run two steps ahead for the ring and one for the table: step t waits
+  // for both (lds_wait), then issues the table reads of step t + 1 and the ring
+  // read of step t + 2.
   if (nst > 0) {
     const int ngl = (int)(g1 - g0);
     const uint32_t lut_base = (uint32_t)(size_t)(lds_void_t*)lut;
+    if constexpr (CNT) {
+      fetch_c(0, g0);
+    } else {
 #pragma unroll
-    for (int j = 0; j < kGroupSteps; ++j) fetch_l(j, j);
+      for (int j = 0; j < kGroupSteps; ++j) fetch_l(j, j);
+    }
     fetch_group(0, g0);
     fetch_group(1, g0 + (ngl > 1 ? 1 : 0));
+    if constexpr (CNT) fetch_c(1, g0);
     setup();
-    __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): group 0 landed (group 1 may be in flight)
+    // group 0 landed (group 1, and the counts' second half, may be in flight)
+    if constexpr (CNT) __builtin_amdgcn_s_waitcnt(0x0F75);  // vmcnt(5)
+    else __builtin_amdgcn_s_waitcnt(0x0F74);                // vmcnt(4)
     uint64_t E[8];
-    uint4 xr[2];  // ring words of steps t + 1 (xr[(t + 1) & 1]) and t + 2
+    u32x4_t xr[2];  // ring words of steps t + 1 (xr[(t + 1) & 1]) and t + 2
     lut_lookup8_asm(ring_read(step_addr(0)), lut_base, E);
-    xr[1] = nst > 1 ? ring_read_async(step_addr(1)) : make_uint4(0u, 0u, 0u, 0u);
+    xr[1] = nst > 1 ? ring_read_async(step_addr(1)) : u32x4_t{0u, 0u, 0u, 0u};
     for (int t0 = 0; t0 < nst; t0 += kGroupSteps) {
 #pragma unroll
       for (int s = 0; s < kGroupSteps; ++s) {  // s compile-time: lbuf and xr stay in registers
         const int t = t0 + s;
-        if (t < nst) {
-          uint4& xn = xr[(s + 1) & 1];  // step t + 1
-          uint4& xnn = xr[s & 1];       // step t + 2
+        if (CNT || t < nst) {  // with counts every group is whole
+          u32x4_t& xn = xr[(s + 1) & 1];  // step t + 1
+          u32x4_t& xnn = xr[s & 1];       // step t + 2
           lds_wait(E, xn);
-          bf16x8_t A[4];
+          f16x8_t A[4];
           lut_planes64(E, A);
           // E is consumed above the next lookups, which then reuse its
           // registers.  Past the last step the lookups and ring reads still
@@ -1346,18 +1281,32 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
           // lds_drain below waits for them.
           __builtin_amdgcn_sched_barrier(0);
           lut_lookup8_asm(xn, lut_base, E);
-          if (s == kGroupSteps - 2)  // step t + 2 opens the next group: its fetch has landed
-            __builtin_amdgcn_s_waitcnt(0x0F72);  // when at most 2 later loads are pending
+          if (s == kGroupSteps - 2) {  // step t + 2 opens the next group: its fetch has landed
+            if constexpr (CNT) label_wait<1>(lbuf[1]);
+            else __builtin_amdgcn_s_waitcnt(0x0F72);  // when at most 2 later loads are pending
+          }
           xnn = ring_read_async(step_addr(t + 2));
           if (s == kGroupSteps - 1) {  // every step of this slot is read: refill it two groups on
             const int k = t0 / kGroupSteps;
             fetch_group(k & (kRingGroups - 1), g0 + min(k + kRingGroups, ngl - 1));
           }
-          label_wait<7>(lbuf[s]);
+          Opnd o;
+          if constexpr (CNT) {
+            if (s == 0) label_wait<5>(lbuf[0]);
+            o = opnd_u8<true>(lbuf[s >> 1][2 * (s & 1)], lbuf[s >> 1][2 * (s & 1) + 1], top);
+          } else {
+            label_wait<7>(lbuf[s]);
+            const uint32_t L2[4] = {lbuf[s][0], lbuf[s][1], lbuf[s][2], lbuf[s][3]};
+            o = opnd_hot<kHot, true>(hot8(L2, colL, colM));
+          }
           __builtin_amdgcn_sched_barrier(0);
-          mma(A, __builtin_bit_cast(uint4, lbuf[s]));
+          mma(A, o);
           __builtin_amdgcn_sched_barrier(0);
-          fetch_l(s, t + kGroupSteps);
+          if constexpr (CNT) {
+            if (s & 1) fetch_c(s >> 1, g0 + t0 / kGroupSteps + 1);
+          } else {
+            fetch_l(s, t + kGroupSteps);
+          }
         }
       }
     }
@@ -1367,35 +1316,62 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
     setup();
   }
 
-  // |z| >= 64, inf or nan somewhere in the range: formulas, one step at a time
-  bool bad = false;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) bad |= __builtin_isnan(acc[2][e]);
-  bad = __ballot(bad) != 0;
+  // steps at natural cell order (16 st + 8 h + (0 .. 7)), guarded: the tail, and a redone range
   const ElemParams ep = a.ep;
   const int64_t rowoff = (lb * a.Q + min(q0 + r, a.Q - 1)) * a.HW + h * 8;
-  auto formula_step = [&](int64_t st, int64_t nvalid) {
-    Raw8<ML_BF16> raw;
-    const uint16_t* zp = (const uint16_t*)a.logits + rowoff + st * kPairStep;
-    uint32_t u[4] = {0u, 0u, 0u, 0u};
-    for (int k = 0; k < 8; ++k)
-      if (k < nvalid) u[k >> 1] |= (uint32_t)zp[k] << ((k & 1) * 16);
-    raw.w[0] = make_uint4(u[0], u[1], u[2], u[3]);
-    bf16x8_t T[4][1];
-    float ub = 0.f, up = 0.f;
-    if (nvalid >= 8) planes8_formula<ML_BF16, 1, false>(raw, ep, 8, false, T, ub, up);
-    else planes8_formula<ML_BF16, 1, true>(raw, ep, nvalid, false, T, ub, up);
-    const bf16x8_t A[4] = {T[0][0], T[1][0], T[2][0], T[3][0]};
-    mma(A, *(const uint4*)(labp + st * kPairStep));
+  // the 16-bit integers of step st (compare results or counts)
+  auto counts_of = [&](int64_t st) -> u32x4_t {
+    if constexpr (CNT) {
+      const int64_t cell = st * kPairStep + h * 8;
+      const uint2 c = *(const uint2*)(cimg + (cell >> 6) * cstep + crow + (cell & 63));
+      return widen8<0>(c.x, c.y);
+    } else {
+      const uint4 lv = *(const uint4*)(labp + st * kPairStep + h * 8);
+      const uint32_t L2[4] = {lv.x, lv.y, lv.z, lv.w};
+      return hot8(L2, colL, colM);
+    }
   };
-  if (bad) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
-    for (int64_t st = s0; st < s0 + nst; ++st) formula_step(st, 8);
+  const uint32_t all = CNT ? (uint32_t)a.N2 * 0x10001u : kHot * 0x10001u;
+  for (int64_t st = full; st < steps; ++st) {
+    const int64_t nv = a.HW - (st * kPairStep + h * 8);
+    Raw8<ML_BF16> raw;
+    load_raw8_part<ML_BF16>(a.logits, rowoff + st * kPairStep, nv, raw);
+    f16x8_t T[4][1];
+    float ub = 0.f, up = 0.f;
+    planes8_formula<ML_BF16, 1, true>(raw, ep, nv, false, T, ub, up);
+    const f16x8_t A[4] = {T[0][0], T[1][0], T[2][0], T[3][0]};
+    const u32x4_t n = counts_of(st);
+    if constexpr (CNT) mma(A, Opnd{part8<false>(n), part8<false>(isub8(all, n))});
+    else mma(A, opnd_hot<kHot, true>(n));
   }
-  if (has_tail) formula_step(full, a.HW - (full * kPairStep + h * 8));
+  // |z| >= 64, inf or nan somewhere in the range: bf16 operands, one step at a time
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) bad |= !(fabsf(acc[0][e]) < INFINITY);
+  bad = __ballot(bad) != 0;
+  if (bad) {
+    clear();
+    for (int64_t st = s0; st < steps; ++st) {
+      if (st >= s0 + nst && st < full) st = full;
+      if (st >= steps) break;
+      const int64_t nv = a.HW - (st * kPairStep + h * 8);
+      Raw8<ML_BF16> raw;
+      load_raw8_part<ML_BF16>(a.logits, rowoff + st * kPairStep, nv, raw);
+      bf16x8_t A[4][1];
+      planes8_redo<ML_BF16>(raw, ep, nv, A);
+      const u32x4_t n = counts_of(st);
+      const bf16x8_t Bp = redo8(isub8(all, n), 0xFFFFu, CNT ? 0 : 8), Bv = redo8(n, 0xFFFFu, CNT ? 0 : 8);
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0][0], Bp, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[2][0], Bv, acc[1], 0, 0, 0);
+      acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[3][0], Bv, acc[2], 0, 0, 0);
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[1][0], Bv, acc[0], 0, 0, 0);
+    }
+  }
+  const float sc = bad ? 1.f : (CNT ? 1.f : 65536.f) / kPlaneScale;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] *= sc;
 }
 
 // One wave's accumulators in LDS (12 KB): 4 consecutive registers per lane
@@ -1419,6 +1395,7 @@ __device__ __forceinline__ void acc_add_lds(f32x16_t (&acc)[3], const float* buf
     }
 }
 
+template <int CNT>
 __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
   __shared__ __align__(16) unsigned char lds[kDmaLds];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1447,7 +1424,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
     const int64_t task = __builtin_amdgcn_readfirstlane(a.sched[kSchedList + j * rt + 2 * rp]);
     lb = task / rt;
     const uint32_t ring = (uint32_t)(size_t)(lds_void_t*)lds + ring_base(wave);
-    cost_wave_pair(a, lb, 32 * rp, 4 * ksq + kq, 4 * KSq, lds, ring, acc, setup);
+    cost_wave_pair<CNT>(a, lb, 32 * rp, 4 * ksq + kq, 4 * KSq, lds, ring, acc, setup);
   } else {
     setup();
   }
@@ -1456,6 +1433,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
   float* red = (float*)lds;
   constexpr int kAccFloats = 3 * 16 * 64;
   const int pp = wave >> 2;
+  static_assert(8 * kAccFloats * 4 <= (int)kDmaLds, "eight waves' sums fit the LDS");
   __syncthreads();
   if (p < np && kq >= 2) acc_to_lds(red + (2 * pp + kq - 2) * kAccFloats, acc, lane);
   __syncthreads();
@@ -1467,7 +1445,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
   acc_add_lds(acc, red + pp * kAccFloats, lane);
 
   // item ksq * np + p: [3][32 rows][32 slots]; rows of the second tile only
-  // for a real pair, slots up to the ones column only (what the finalize reads)
+  // for a real pair, slots up to G only (what the finalize reads)
   const int r = lane & 31, h = lane >> 5;
   const int G = __builtin_amdgcn_readfirstlane(a.ncols[lb % a.B]);
   const bool two = 2 * rp + 1 < rt;
@@ -1484,75 +1462,44 @@ __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
 }
 
 // ---- launch plan ---------------------------------------------------------------
-// Resident waves of one cost kernel instance on the current device (cached).
-template <int DT, int RT, int NT, int CNT, bool TAB>
-static int occ_slots() {
-  static std::atomic<int> cache[64];
+// Resident waves of a kernel of `waves` waves per workgroup on the current
+// device, cached per device in `cache`.
+static int occ_slots(std::atomic<int> (&cache)[64], const void* kernel, int waves) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   int v = cache[dev].load(std::memory_order_relaxed);
   if (v == 0) {
     int nb = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, cost_kernel<DT, RT, NT, CNT, TAB>, 64 * cost_waves(NT, TAB), 0) !=
-            hipSuccess || nb < 1)
-      nb = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, 64 * waves, 0) != hipSuccess || nb < 1) nb = 1;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
       cus = 256;
-    v = nb * cus * cost_waves(NT, TAB);
+    v = nb * cus * waves;
     cache[dev].store(v, std::memory_order_relaxed);
   }
   return v;
 }
-
-// The LDS-staged table kernel needs 16-byte aligned rows (HW % 8 == 0) whose
-// per-tile element offsets fit 32 bits.
-static bool dma_ok(const Dims& d) { return d.HW % 8 == 0 && d.HW >= 8 && d.HW * 16 < ((int64_t)1 << 31); }
-
-// Resident waves of the LDS-staged table kernel on the current device (cached).
-static int occ_slots_dma() {
+template <int DT, int NT, int CNT, bool TAB>
+static int occ_slots_of() {
   static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  int v = cache[dev].load(std::memory_order_relaxed);
-  if (v == 0) {
-    int nb = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, cost_dma_kernel<2>, 64 * kDmaWaves, 0) !=
-            hipSuccess || nb < 1)
-      nb = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-      cus = 256;
-    v = nb * cus * (int)kDmaWaves;
-    cache[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
+  return occ_slots(cache, (const void*)cost_kernel<DT, NT, CNT, TAB>, cost_waves(NT, TAB));
 }
-
-// Resident waves of the row-tile pair kernel on the current device (cached).
+template <int CNT>
 static int occ_slots_pair() {
   static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  int v = cache[dev].load(std::memory_order_relaxed);
-  if (v == 0) {
-    int nb = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, cost_pair_kernel, 64 * kDmaWaves, 0) !=
-            hipSuccess || nb < 1)
-      nb = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-      cus = 256;
-    v = nb * cus * (int)kDmaWaves;
-    cache[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
+  return occ_slots(cache, (const void*)cost_pair_kernel<CNT>, (int)kDmaWaves);
 }
 
 // cnt: 0 label map, 1 u8 counts, 2 u16 counts
-template <int DT, int RT, int NT>
+template <int DT, int NT>
 static int occ_slots_for(int cnt, bool tab) {
-  if (cnt == 1) return occ_slots<DT, RT, NT, 1, false>();
-  if (cnt == 2) return occ_slots<DT, RT, NT, 2, false>();
-  if (DT == ML_BF16 && tab) return occ_slots<DT, RT, NT, 0, DT == ML_BF16>();
-  return occ_slots<DT, RT, NT, 0, false>();
+  constexpr bool kTab = DT == ML_BF16;
+  if (kTab && tab)
+    return cnt == 1   ? occ_slots_of<DT, NT, 1, kTab>()
+           : cnt == 2 ? occ_slots_of<DT, NT, 2, kTab>()
+                      : occ_slots_of<DT, NT, 0, kTab>();
+  return cnt == 1   ? occ_slots_of<DT, NT, 1, false>()
+         : cnt == 2 ? occ_slots_of<DT, NT, 2, false>()
+                    : occ_slots_of<DT, NT, 0, false>();
 }
 
 static int cu_count() {
@@ -1570,20 +1517,18 @@ static int cu_count() {
 // With three classes the narrower ones leave `side` CUs' worth of waves free:
 // their launches may run beside the widest class's assignment (one
 // workgroup per image on the forward's side stream).
-template <int DT, int RT>
-static void plan_slots(CostPlan& p, int cnt, bool tab, bool dma, int64_t side) {
+template <int DT>
+static void plan_slots(CostPlan& p, int cnt, bool tab, int64_t side) {
   const int cus = cu_count();
   side = std::min<int64_t>(side, cus / 8);
   for (int ci = 0; ci < p.nclass; ++ci) {
     int v = 0;
     switch (ci) {
       case 0:
-        v = p.pair0 ? occ_slots_pair()
-            : DT == ML_BF16 && tab && cnt == 0 && dma ? occ_slots_dma()
-                                                      : occ_slots_for<DT, RT, 2>(cnt, tab);
+        v = !p.pair0 ? occ_slots_for<DT, 2>(cnt, tab) : cnt ? occ_slots_pair<1>() : occ_slots_pair<0>();
         break;
-      case 1: v = occ_slots_for<DT, RT, 7>(cnt, tab); break;
-      default: v = occ_slots_for<DT, RT, 16>(cnt, tab); break;
+      case 1: v = occ_slots_for<DT, 7>(cnt, tab); break;
+      default: v = occ_slots_for<DT, 16>(cnt, tab); break;
     }
     if (p.nclass == kClasses && ci < kClasses - 1) v -= (int)((int64_t)v * side / cus);
     p.slots[ci] = (int)std::min<int64_t>(std::max(v, 8), kCostSlots);
@@ -1594,18 +1539,25 @@ CostPlan make_cost_plan(const Dims& d, int dtype, bool tab) {
   CostPlan p = bound_cost_plan(d);
   const int cnt = d.counts_mode ? d.cw : 0;
   p.pair0 = dtype == ML_BF16 && tab && d.pair_ok ? 1 : 0;
-  // the wide classes' slot-sum form runs on label maps without the table
-  for (int c = 0; c < kClasses; ++c) p.planes[c] = c > 0 && !d.counts_mode && !(dtype == ML_BF16 && tab) ? 4 : 3;
   const int64_t side = std::min<int64_t>(d.LB, kSideCUs);
   switch (dtype) {
-    case ML_F32: plan_slots<ML_F32, 1>(p, cnt, false, false, side); break;
-    case ML_BF16: plan_slots<ML_BF16, 1>(p, cnt, tab, dma_ok(d), side); break;
-    case ML_F16: plan_slots<ML_F16, 1>(p, cnt, false, false, side); break;
+    case ML_F32: plan_slots<ML_F32>(p, cnt, false, side); break;
+    case ML_BF16: plan_slots<ML_BF16>(p, cnt, tab, side); break;
+    case ML_F16: plan_slots<ML_F16>(p, cnt, false, side); break;
   }
   return p;
 }
 
-template <int DT, int RT, int NT>
+template <int DT, int NT, bool TAB>
+static void launch_cnt(const CostArgs& a, const Dims& d, hipStream_t st) {
+  const int WV = cost_waves(NT, TAB);
+  const dim3 grid((unsigned)ceil_div(std::max<int64_t>(a.plan.slots[kClassOf<NT>], a.plan.ntasks), WV)), blk(64 * WV);
+  if (!d.counts_mode) hipLaunchKernelGGL((cost_kernel<DT, NT, 0, TAB>), grid, blk, 0, st, a);
+  else if (d.cw == 1) hipLaunchKernelGGL((cost_kernel<DT, NT, 1, TAB>), grid, blk, 0, st, a);
+  else hipLaunchKernelGGL((cost_kernel<DT, NT, 2, TAB>), grid, blk, 0, st, a);
+}
+
+template <int DT, int NT>
 static int launch_one(const CostArgs& a, const Dims& d, bool tab, hipStream_t st) {
   constexpr int CI = kClassOf<NT>;
   if (NT == 2 && a.plan.pair0) {
@@ -1617,51 +1569,36 @@ static int launch_one(const CostArgs& a, const Dims& d, bool tab, hipStream_t st
     // KSq <= ks_max / 4; surplus workgroups exit at once
     const int64_t np_max = d.LB * ((d.rtiles + 1) / 2);
     const int64_t wgs = ceil_div(a.plan.slots[CI], 16) + ceil_div(np_max, 4) + d.ks_max / 4 + 1;
-    hipLaunchKernelGGL(cost_pair_kernel, dim3((unsigned)wgs), dim3(64 * kDmaWaves), 0, st, a);
+    const dim3 grid((unsigned)wgs), blk(64 * kDmaWaves);
+    if (d.counts_mode) hipLaunchKernelGGL(cost_pair_kernel<1>, grid, blk, 0, st, a);
+    else hipLaunchKernelGGL(cost_pair_kernel<0>, grid, blk, 0, st, a);
     return check_launch("pair_cost");
   }
-  if constexpr (DT == ML_BF16 && NT == 2) {
-    if (tab && !d.counts_mode && dma_ok(d)) {
-      const dim3 grid((unsigned)ceil_div(std::max<int64_t>(a.plan.slots[CI], a.plan.ntasks), kDmaWaves));
-      hipLaunchKernelGGL((cost_dma_kernel<NT>), grid, dim3(64 * kDmaWaves), 0, st, a);
-      return check_launch("pair_cost");
-    }
-  }
-  const int WV = cost_waves(NT, DT == ML_BF16 && tab && !d.counts_mode);
-  const dim3 grid((unsigned)ceil_div(std::max<int64_t>(a.plan.slots[CI], a.plan.ntasks), WV));
-  if (d.counts_mode && d.cw == 2)
-    hipLaunchKernelGGL((cost_kernel<DT, RT, NT, 2, false>), grid, dim3(64 * WV), 0, st, a);
-  else if (d.counts_mode)
-    hipLaunchKernelGGL((cost_kernel<DT, RT, NT, 1, false>), grid, dim3(64 * WV), 0, st, a);
-  else if (DT == ML_BF16 && tab)
-    hipLaunchKernelGGL((cost_kernel<DT, RT, NT, 0, DT == ML_BF16>), grid, dim3(64 * WV), 0, st, a);
-  else
-    hipLaunchKernelGGL((cost_kernel<DT, RT, NT, 0, false>), grid, dim3(64 * WV), 0, st, a);
+  if (DT == ML_BF16 && tab) launch_cnt<DT, NT, DT == ML_BF16>(a, d, st);
+  else launch_cnt<DT, NT, false>(a, d, st);
   return check_launch("pair_cost");
 }
 
 // One launch per column-tile class up to the padded width; each image is
 // processed by exactly one of them.
-template <int DT, int RT>
+template <int DT>
 static int launch_classes(const CostArgs& a, const Dims& d, bool tab, unsigned classes, hipStream_t st) {
   int rc = 0;
-  if (classes & 1u) rc = launch_one<DT, RT, 2>(a, d, tab, st);
-  if (!rc && a.plan.nclass > 1 && (classes & 2u)) rc = launch_one<DT, RT, 7>(a, d, tab, st);
-  if (!rc && a.plan.nclass > 2 && (classes & 4u)) rc = launch_one<DT, RT, 16>(a, d, tab, st);
+  if (classes & 1u) rc = launch_one<DT, 2>(a, d, tab, st);
+  if (!rc && a.plan.nclass > 1 && (classes & 2u)) rc = launch_one<DT, 7>(a, d, tab, st);
+  if (!rc && a.plan.nclass > 2 && (classes & 4u)) rc = launch_one<DT, 16>(a, d, tab, st);
   return rc;
 }
-
-int cost_rt_for(int, int) { return 1; }
 
 int launch_cost(const CostArgs& a, const Dims& d, int dtype, bool, hipStream_t st, unsigned classes,
                 bool prof) {
   ProfScope ps_(prof ? "pair_cost" : nullptr, st);
-  // bf16 with label maps and no unweighted row sums: table path
-  const bool tab = dtype == ML_BF16 && !d.counts_mode && a.use_lut && a.rowsum == nullptr;
+  // bf16 without unweighted row sums: table path
+  const bool tab = dtype == ML_BF16 && a.use_lut && a.rowsum == nullptr;
   switch (dtype) {
-    case ML_F32: return launch_classes<ML_F32, 1>(a, d, false, classes, st);
-    case ML_BF16: return launch_classes<ML_BF16, 1>(a, d, tab, classes, st);
-    case ML_F16: return launch_classes<ML_F16, 1>(a, d, false, classes, st);
+    case ML_F32: return launch_classes<ML_F32>(a, d, false, classes, st);
+    case ML_BF16: return launch_classes<ML_BF16>(a, d, tab, classes, st);
+    case ML_F16: return launch_classes<ML_F16>(a, d, false, classes, st);
   }
   return fail(ML_EINVAL, "unsupported mask logits dtype");
 }

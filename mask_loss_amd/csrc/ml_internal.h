@@ -43,7 +43,7 @@ constexpr int64_t kPrepFillBytes = (int64_t)56 << 20;
 constexpr int64_t kFinFillBytes = (int64_t)16 << 20;
 
 // Column-tile classes of the cost contraction: an image with G non-empty GT
-// columns (+ the ones column) is handled by the kernel instance whose tile
+// columns (+ slot G) is handled by the kernel instance whose tile
 // count NT is the smallest of {2, 7, 16} that holds G + 1 columns.  Which
 // classes have images is known on the device only, and every class launch
 // costs its dispatch latency even when empty, so the classes are few.
@@ -71,6 +71,12 @@ constexpr int64_t kCostSlots = 4096;
 // the widest class's assignment (at most one per image, at most 1/8 of them)
 constexpr int kSideCUs = 16;
 
+// Planes of class ci's partial tile (see ml_cost.hip): bce numerator, I, T of
+// every column slot, slot G of an image with G non-empty columns being the ones
+// column (class 0); or the slot sums N, Pos, I, T, slot G holding the pixels of
+// no column.
+__host__ __device__ constexpr int class_planes(int ci) { return ci == 0 ? 3 : 4; }
+
 // Host-side plan of the cost launches.  Each class launch has `slots[c]`
 // waves (what the GPU holds resident at that kernel's occupancy, at most
 // kCostSlots); on the device the schedule picks the class's K-split KS_c =
@@ -96,13 +102,6 @@ struct CostPlan {
   // the class's images at one K-split, and its partial tile holds both row
   // tiles ([3][2 rows][nslot]).  No row-sum records on this path.
   int pair0;
-  // Planes per partial tile of each class: 3 (bce numerator, I, T) or 4 for
-  // classes 1 and 2 on label maps without the bf16 table (per-slot sums of
-  // A_neg, A_pos, A_p, A_w over the cells whose label is that slot's column;
-  // slot G holds the cells of no column).  Finalize rebuilds the bce
-  // numerator of slot g as the sum of the other slots' A_neg sums plus g's
-  // A_pos sum, and P, S as the sums over all slots.
-  int planes[kClasses];
 };
 // Device schedule (ints in the workspace): n[kClasses], ks[kClasses] (the
 // K-split partials of each task that reach the partial sums), red[kClasses]
@@ -134,7 +133,7 @@ struct RowPartials {
 __device__ inline RowPartials row_partials_at(const float* partials, const CostPlan& plan, int ci,
                                               int64_t i, int KS, int64_t n, int qin, int64_t rows) {
   const int64_t nslot_c = 16 * class_nt(ci);
-  const int64_t tile = plan.planes[ci] * rows * nslot_c;
+  const int64_t tile = class_planes(ci) * rows * nslot_c;
   RowPartials r;
   r.KS = KS;
   if (ci == 0 && plan.pair0) {
@@ -165,22 +164,32 @@ struct Dims {
   int64_t GT_out, bg;        // compacted column count, normalised background slot
   int64_t HWp;               // HW padded to a multiple of kStep
   int NT;                    // 16-wide column tiles (valid GT columns + ones column)
-  int RT;                    // 16-row tiles per wave
-  int rows;                  // rows per cost workgroup (16 * RT)
+  int rows;                  // query rows per task (one 16-row tile)
   int64_t rtiles;            // row tiles per image
   int64_t ks_max;            // most K-splits per task (>= 8 K-steps per wave)
   int nslot;                 // 16 * NT
   bool counts_mode;          // s > 1: per-cell count operands
   int cw;                    // bytes per count: 1 (u8, s <= 15) or 2 (u16, s >= 16)
   int64_t crows;             // count rows per 64-cell block (see CountTiles)
-  bool pair_ok;              // bf16 label maps whose rows suit the row-tile pair kernel
+  bool pair_ok;              // bf16 logits and targets that suit the row-tile pair kernel
 };
+
+// Label maps of s == 1 targets on the matching path: one u16 code per cell, the
+// label in the high byte (make_dims admits labels below 256), so that codes of
+// two labels differ by at least kHot as unsigned numbers under xor.  Cells of no
+// column carry a code that no column has: the background slot's, or 255's.
+constexpr uint32_t kHot = 0x0100u;
+__host__ __device__ inline uint32_t label_code(int64_t lab) { return (uint32_t)lab << 8; }
+__host__ __device__ inline uint32_t no_column_code(int64_t bg, int64_t GT_total) {
+  return label_code(bg < GT_total ? bg : 255);
+}
 
 // Per-cell label counts of s > 1 targets (the reference's count tensor,
 // src/cuda/utils.cuh:6-36) in blocks of 64 cells: [B][ceil(HW / 64)][rows][64]
 // of cw bytes, row r < GT_total holding label r and, on the matching path, row
 // GT_total the pixels of no output column (labels outside [0, GT_total) and
-// the background slot; that slot's own row then stays zero).  A block holds
+// the background slot; that slot's own row then stays zero) and row GT_total + 1
+// the ones column, s^2 everywhere.  A block holds
 // every label of 64 cells side by side, so the contraction reads its operand
 // tile (many labels, the same cells) as one run, and one label's counts along
 // the cells (the backward) come in runs of 64.
@@ -200,7 +209,6 @@ inline size_t count_bytes(int64_t B, int64_t HW, int64_t rows, int cw) {
 }
 
 bool make_dims(const ml_shape* s, int64_t background_index, int dtype, Dims& d, std::string& err);
-int cost_rt_for(int dtype, int NT);
 
 // Byte offsets inside the forward's saved state (see ml_saved_bytes): the
 // float head (per-query stats, then the per-layer block), the matched-row list
@@ -254,7 +262,8 @@ struct FillSlice {
 
 struct PrepArgs {
   const int64_t* targets;
-  uint16_t* lab16;       // s == 1
+  uint16_t* lab16;       // s == 1: codes (label_code), or labels where `codes` is 0
+  int codes = 1;
   CountTiles counts{};   // s > 1 (its p is written)
   int64_t rest = -1;     // count row of the pixels of no column, or -1: none kept
   FillSlice fill;        // done by extra workgroups of the column pass
@@ -293,7 +302,7 @@ struct CostArgs {
   const int* ncols;
   const int* colmap;
   const int* sched;  // device schedule (see CostPlan)
-  float* partials;   // per work item: [planes][rows][16 * NT_class] (CostPlan::planes)
+  float* partials;   // per work item: [class_planes][rows][16 * NT_class]
   float* rowsum;     // per work item: [rows][2] unweighted (force_masks) or null
   CostPlan plan;
   int64_t L, B, Q, HW, HWp, rtiles, GT_total, bg, rows;
@@ -503,8 +512,8 @@ int launch_point_sample_backward(int dtype, const void* gout, const float* coord
                                  int64_t C, int64_t H, int64_t W, int64_t P, int64_t cb, int align,
                                  void* gin, float* acc, hipStream_t st);
 int launch_point_labels(const int64_t* targets, const float* coords, int64_t B, int64_t Ht,
-                        int64_t Wt, int64_t P, int64_t GT_total, int64_t* out64, uint16_t* out16,
-                        int64_t HWp, hipStream_t st);
+                        int64_t Wt, int64_t P, int64_t GT_total, int64_t bg, int64_t* out64,
+                        uint16_t* codes, int64_t HWp, hipStream_t st);
 int launch_dense(const DenseArgs& a, bool dice, bool backward, hipStream_t st);
 size_t dense_partials_bytes(int64_t L, int64_t B, int64_t C, int64_t HW, bool dice);
 int launch_zero_fill(void* p, size_t bytes, hipStream_t st);

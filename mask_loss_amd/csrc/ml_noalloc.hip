@@ -20,6 +20,8 @@
 
 namespace ml {
 
+// Cost plans are fitted to half of it (fit_cost_plan); the other half takes the
+// shapes whose smallest plan is larger.
 constexpr size_t kScratchBytes = ML_NOALLOC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 

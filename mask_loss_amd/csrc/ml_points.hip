@@ -11,8 +11,7 @@
 // * point_labels_kernel: the label under each point with the reference's
 //   floor mapping ix = clamp(long(x * (W_t - 1)), 0, W_t - 1)
 //   (pw_sigmoid_ce.py:497-502, pw_dice_loss.py:242-245), as int64 and/or as
-//   the u16 compact label row the cost contraction reads (labels outside
-//   [0, GT_total) -> no label).
+//   the u16 label codes the cost contraction reads (label_code).
 //
 // Planes of up to 64 KB are staged in LDS (point_sample_lds_kernel: each
 // plane read from HBM once with coalesced loads, the corners gathered from
@@ -736,8 +735,8 @@ __device__ __forceinline__ int64_t point_cell(float x, int64_t size) {
 // [P, HWp) of the u16 row get no label.
 __global__ __launch_bounds__(256) void point_labels_kernel(const int64_t* targets, const float* coords,
                                                            int64_t Ht, int64_t Wt, int64_t P,
-                                                           int64_t GT_total, int64_t* out64,
-                                                           uint16_t* out16, int64_t HWp) {
+                                                           int64_t GT_total, int64_t bg, int64_t* out64,
+                                                           uint16_t* codes, int64_t HWp) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t b = blockIdx.y;
   if (p < P) {
@@ -745,21 +744,21 @@ __global__ __launch_bounds__(256) void point_labels_kernel(const int64_t* target
     const int64_t ix = point_cell(cp[0], Wt), iy = point_cell(cp[1], Ht);
     const int64_t lab = targets[(b * Ht + iy) * Wt + ix];
     if (out64) out64[b * P + p] = lab;
-    if (out16)
-      out16[b * HWp + p] = (uint64_t)lab < (uint64_t)GT_total ? (uint16_t)lab : (uint16_t)kNoLabel;
-  } else if (out16 && p < HWp) {
-    out16[b * HWp + p] = (uint16_t)kNoLabel;
+    if (codes)
+      codes[b * HWp + p] = (uint16_t)((uint64_t)lab < (uint64_t)GT_total ? label_code(lab) : no_column_code(bg, GT_total));
+  } else if (codes && p < HWp) {
+    codes[b * HWp + p] = (uint16_t)no_column_code(bg, GT_total);
   }
 }
 
 int launch_point_labels(const int64_t* targets, const float* coords, int64_t B, int64_t Ht,
-                        int64_t Wt, int64_t P, int64_t GT_total, int64_t* out64, uint16_t* out16,
-                        int64_t HWp, hipStream_t st) {
-  const int64_t n = out16 ? HWp : P;
+                        int64_t Wt, int64_t P, int64_t GT_total, int64_t bg, int64_t* out64,
+                        uint16_t* codes, int64_t HWp, hipStream_t st) {
+  const int64_t n = codes ? HWp : P;
   if (B == 0 || n == 0) return ML_OK;
   if (B > 65535) return fail(ML_EINVAL, "point labels: too many images");
   hipLaunchKernelGGL(point_labels_kernel, dim3((unsigned)ceil_div(n, 256), (unsigned)B), dim3(256), 0,
-                     st, targets, coords, Ht, Wt, P, GT_total, out64, out16, HWp);
+                     st, targets, coords, Ht, Wt, P, GT_total, bg, out64, codes, HWp);
   return check_launch("point_labels");
 }
 

@@ -1,6 +1,8 @@
 // Target preparation: int64 label map -> compact per-image target operands.
 //
-//   s == 1 : u16 label per cell (labels outside [0, GT_total) -> 0xFFFF)
+//   s == 1 : u16 label code per cell (label_code; cells of no output column
+//            share one code), or the u16 label itself for the dense losses
+//            (labels outside [0, GT_total) -> 0xFFFF)
 //   s  > 1 : count of each label inside the s x s block of every cell
 //            (CountTiles), the reference's count tensor
 //            (src/cuda/utils.cuh:6-36); u8 for s <= 15, u16 for s >= 16
@@ -285,11 +287,12 @@ __global__ __launch_bounds__(256) void prep_labels_kernel(PrepArgs a) {
   if (cell0 < a.HWp) {
     uint32_t wv[4];
     int64_t prev = -1;
+    const uint32_t none = no_column_code(a.bg, a.GT_total);  // the background's own code is this one
     const int64_t lane0 = __shfl(lab[0], 0, 64);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const bool valid = (uint64_t)lab[k] < (uint64_t)a.GT_total;
-      const uint32_t v = valid ? (uint32_t)lab[k] : (uint32_t)kNoLabel;
+      const uint32_t v = a.codes ? (valid ? label_code(lab[k]) : none) : valid ? (uint32_t)lab[k] : (uint32_t)kNoLabel;
       if (k & 1) wv[k >> 1] |= v << 16;
       else wv[k >> 1] = v;
       if (mark && valid && lab[k] != prev && !(k == 0 && lab[0] == lane0 && (threadIdx.x & 63) != 0))
@@ -344,6 +347,9 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
   auto row_of = [&](int64_t lab) -> int {
     return (uint64_t)lab < (uint64_t)a.GT_total && (a.rest < 0 || lab != a.bg) ? (int)lab : (int)a.rest;
   };
+  auto clear = [&]() {
+    for (int i = tid; i < rc * (kCntCells * CW / 16); i += kCntThreads) ((uint4*)tile)[i] = make_uint4(0u, 0u, 0u, 0u);
+  };
   int64_t lab[S ? S : 1];
   bool whole = false;  // every pixel of the cell carries lab[0]
   bool first = true;   // ... and the wave's first cell does not already mark that label
@@ -363,6 +369,7 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
         for (int k = 0; k < S; ++k) lab[k] = p[k];
       }
     }
+    clear();  // while the labels are on their way
     const int64_t l0 = __shfl(act ? lab[0] : 0, (tid & 63) & ~3, 64);
     bool same = !act || lab[0] == l0;
 #pragma unroll
@@ -371,13 +378,19 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
     whole = in && ((m >> ((tid & 63) & ~3)) & 0xFull) == 0xFull;
     const int64_t lw = __shfl(lab[0], 0, 64);
     first = (tid & 63) == 0 || (m & 0xFull) != 0xFull || lab[0] != lw;
+  } else {
+    clear();
   }
   uint8_t* const out0 = (uint8_t*)a.counts.p;
   for (int64_t r0 = 0; r0 < a.counts.rows; r0 += rc) {  // one round unless there are many rows
     const int64_t nr = min((int64_t)rc, a.counts.rows - r0);
-    for (int i = tid; i < (int)(nr * kCntCells * CW / 16); i += kCntThreads)
-      ((uint4*)tile)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (r0 > 0) clear();
     __syncthreads();
+    const int64_t ones = a.rest + 1 - r0;  // the ones column's row: 4 CW words in each of the four blocks
+    if (a.rest >= 0 && ones >= 0 && ones < nr && tid < 16 * CW) {
+      const uint32_t v = (uint32_t)(s * s) * (CW == 1 ? 0x01010101u : 0x00010001u);
+      ((uint4*)tile)[(int)((tid / (4 * CW)) * nr + ones) * 4 * CW + tid % (4 * CW)] = make_uint4(v, v, v, v);
+    }
     // n pixels of one label in this thread's cell
     auto add = [&](int64_t lb, uint32_t n, bool single) {
       const bool valid = (uint64_t)lb < (uint64_t)a.GT_total;
@@ -427,14 +440,13 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
       }
     }
     __syncthreads();
-    // block k of this workgroup: rows [r0, r0 + nr) are one run of the tiles
-    const int per = (int)(nr * kCountCells * CW / 16);  // 16-byte words
+    // rows [r0, r0 + nr) of each of this workgroup's blocks (all rows: one run)
+    const uint32_t per = (uint32_t)(nr * kCountCells * CW / 16);  // 16-byte words
     const int64_t blk0 = (int64_t)blockIdx.x * (kCntCells / kCountCells);
-    for (int k = 0; k < kCntCells / kCountCells; ++k) {
-      if (blk0 + k >= a.counts.nb) break;
-      uint4* dst = (uint4*)(out0 + ((b * a.counts.nb + blk0 + k) * a.counts.rows + r0) * kCountCells * CW);
-      for (int i = tid; i < per; i += kCntThreads) dst[i] = ((const uint4*)tile)[k * per + i];
-    }
+    const uint32_t words = per * (uint32_t)min((int64_t)(kCntCells / kCountCells), a.counts.nb - blk0);
+    uint4* dst = (uint4*)(out0 + ((b * a.counts.nb + blk0) * a.counts.rows + r0) * kCountCells * CW);
+    const uint32_t skip = (uint32_t)(a.counts.rows - nr) * (kCountCells * CW / 16);  // the other rows of a block
+    for (uint32_t i = tid; i < words; i += kCntThreads) dst[i + (skip ? i / per * skip : 0u)] = ((const uint4*)tile)[i];
     __syncthreads();
   }
   if (mark) pres_store(a, pres, b);
@@ -515,7 +527,7 @@ int launch_prep_points(const PrepArgs& a, const Dims& d, int64_t Hs, int64_t Ws,
                      dim3(256), 0, st, m);
   int rc = check_launch("prep");
   if (rc) return rc;
-  rc = launch_point_labels(a.targets, coords, d.B, Hs, Ws, d.HW, a.GT_total, nullptr, a.lab16, d.HWp, st);
+  rc = launch_point_labels(a.targets, coords, d.B, Hs, Ws, d.HW, a.GT_total, a.bg, nullptr, a.lab16, d.HWp, st);
   if (rc) return rc;
   hipLaunchKernelGGL(prep_columns_kernel, dim3(1u + (unsigned)a.fill.blocks), dim3(1024), 0, st, a);
   return check_launch("prep_columns");
