@@ -1040,9 +1040,9 @@ __global__ __launch_bounds__(256) void assign_kernel(AssignArgs a) {
           }
           wave_sync();
           if (a.strategy == ML_PSEUDO_GREEDY) {
-            if (lane == 0)
-              for (int64_t q = 0; q < Q; ++q)
-                if (p2g[q] >= 0 && cap[p2g[q]] > 0) cap[p2g[q]] -= 1;
+            // (each column was matched at most once)
+            for (int64_t q = lane; q < Q; q += 64)
+              if (p2g[q] >= 0 && cap[p2g[q]] > 0) cap[p2g[q]] -= 1;
             wave_sync();
             int nr = 0;
             for (int64_t q0 = 0; q0 < Q; q0 += 64) {
@@ -1060,11 +1060,14 @@ __global__ __launch_bounds__(256) void assign_kernel(AssignArgs a) {
         int nrem = (int)Q;
         for (int64_t rd = 0; rd < K && okh; ++rd) {
           int M = 0;
-          for (int t = 0; t < nv; ++t)
-            if (cap[vcols[t]] > 0) {
-              if (lane == 0) hrows[M] = vcols[t];
-              ++M;
-            }
+          for (int t0 = 0; t0 < nv; t0 += 64) {
+            const int t = t0 + lane;
+            const int c = t < nv ? vcols[t] : 0;
+            const bool open = t < nv && cap[c] > 0;
+            const uint64_t m = __ballot(open);
+            if (open) hrows[M + __popcll(m & ((1ull << lane) - 1ull))] = c;
+            M += __popcll(m);
+          }
           if (M == 0 || nrem == 0) break;
           if (M > nrem) M = nrem;
           wave_sync();
@@ -1092,12 +1095,11 @@ __global__ __launch_bounds__(256) void assign_kernel(AssignArgs a) {
             nn += __popcll(m);
           }
           wave_sync();
-          if (lane == 0)
-            for (int k = 0; k < nrem; ++k) {
-              const int q = preds[k];
-              const int c = p2g[q];
-              if (c >= 0 && hout[k] >= 0 && hrows[hout[k]] == c && cap[c] > 0) cap[c] -= 1;
-            }
+          // this round's matches, at most one per column
+          for (int k = lane; k < nrem; k += 64) {
+            const int c = p2g[preds[k]];
+            if (c >= 0 && hout[k] >= 0 && hrows[hout[k]] == c && cap[c] > 0) cap[c] -= 1;
+          }
           wave_sync();
           for (int k = lane; k < nn; k += 64) preds[k] = way[k];
           nrem = nn;
