@@ -227,6 +227,17 @@ int ml_mask_matching_backward(const ml_shape* s, const ml_params* p,
                               const void* saved, int grad_prefilled, void* grad_mask_logits,
                               void* grad_cls_logits, void* workspace,
                               size_t workspace_bytes, ml_stream_t stream);
+/* The same with the upstream gradients of layer l at grad_*[l * stride]
+ * (elements): a gradient broadcast over the layers (stride 0) needs no copy. */
+int ml_mask_matching_backward_strided(const ml_shape* s, const ml_params* p, const float* grad_mask,
+                                      int64_t grad_mask_stride, const float* grad_dice,
+                                      int64_t grad_dice_stride, const float* grad_cls,
+                                      int64_t grad_cls_stride, int mask_dtype, const void* mask_logits,
+                                      const int64_t* mask_targets, int cls_dtype,
+                                      const void* cls_logits, const int64_t* cls_targets,
+                                      const int64_t* pred_to_gt, const void* saved, int grad_prefilled,
+                                      void* grad_mask_logits, void* grad_cls_logits, void* workspace,
+                                      size_t workspace_bytes, ml_stream_t stream);
 
 /* ---- pairwise label cost (L,B,Q,GT_out) float; use_softmax selects the
  * softmax-CE form, otherwise sigmoid-BCE with (gamma, alpha). -------------- */

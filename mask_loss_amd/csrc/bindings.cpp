@@ -332,9 +332,16 @@ std::vector<torch::Tensor> backward_impl(
                   pred_to_gt.size(2) == s.Q,
               "pred_to_gt must have shape (L,B,Q)");
   auto f32 = mask_logits.options().dtype(torch::kFloat32);
-  auto gm = g_mask.to(f32).contiguous();
-  auto gd = g_dice.to(f32).contiguous();
-  auto gc = g_cls.to(f32).contiguous();
+  // (L,) gradients are read at their own stride: one broadcast from a sum over
+  // the layers is not copied out first
+  auto levels = [&](const torch::Tensor& g) {
+    auto x = g.to(f32);
+    return x.dim() == 1 ? x : x.contiguous();
+  };
+  auto stride = [&](const torch::Tensor& g) { return g.dim() == 1 ? g.stride(0) : (int64_t)1; };
+  auto gm = levels(g_mask);
+  auto gd = levels(g_dice);
+  auto gc = levels(g_cls);
   TORCH_CHECK(gm.numel() == s.L && gd.numel() == s.L && gc.numel() == s.L,
               "upstream gradients must have shape (L,)");
   const int mdt = dtype_code(mask_logits, "mask_logits");
@@ -357,8 +364,8 @@ std::vector<torch::Tensor> backward_impl(
   }
   const size_t wsb = ml_mask_matching_backward_workspace_size(&s, &p, mdt);
   auto ws = workspace(wsb, mask_logits);
-  ml_ok(ml_mask_matching_backward(
-      &s, &p, gm.data_ptr<float>(), gd.data_ptr<float>(), gc.data_ptr<float>(), mdt,
+  ml_ok(ml_mask_matching_backward_strided(
+      &s, &p, gm.data_ptr<float>(), stride(gm), gd.data_ptr<float>(), stride(gd), gc.data_ptr<float>(), stride(gc), mdt,
       mask_logits.data_ptr(), mask_targets.data_ptr<int64_t>(), cdt, cls_logits.data_ptr(),
       cls_targets.data_ptr<int64_t>(), pred_to_gt.data_ptr<int64_t>(),
       saved ? saved->data_ptr() : nullptr, grad_prefill.has_value() ? 1 : 0, grad_mask.data_ptr(),

@@ -169,8 +169,8 @@ __global__ __launch_bounds__(256) void bwd_mask_kernel(BwdArgs a) {
   const bool vec = a.dtype == ML_F32 ? (a.HW % 4 == 0) : (a.HW % 8 == 0);
   const int64_t rbase = row * a.HW;
   const float inv_md = a.layer[l * ML_LAYERS + ML_LAYER_INV_MASK_DEN];
-  const float mc = a.g_mask[l] * inv_md;
-  const float dc = a.g_dice[l] * inv_md;
+  const float mc = a.g_mask[l * a.gs_mask] * inv_md;
+  const float dc = a.g_dice[l * a.gs_dice] * inv_md;
   const int64_t nch = ceil_div(a.HW, 8);
 
   if ((!matched && !a.force_masks) || (mc == 0.f && dc == 0.f)) {
@@ -239,8 +239,8 @@ __device__ __forceinline__ void bwd_chunk(const BwdArgs& a, int64_t row, int64_t
   const bool vec = a.dtype == ML_F32 ? (a.HW % 4 == 0) : (a.HW % 8 == 0);
   const int64_t rbase = row * a.HW;
   const float inv_md = a.layer[l * ML_LAYERS + ML_LAYER_INV_MASK_DEN];
-  const float mc = a.g_mask[l] * inv_md;
-  const float dc = a.g_dice[l] * inv_md;
+  const float mc = a.g_mask[l * a.gs_mask] * inv_md;
+  const float dc = a.g_dice[l * a.gs_dice] * inv_md;
   const int64_t c0 = chunk * kBwdChunk + (int64_t)tid * 8;
 
   if ((!matched && !a.force_masks) || (mc == 0.f && dc == 0.f)) {
@@ -408,7 +408,7 @@ __device__ __forceinline__ void cls_row(const BwdArgs& a, int64_t row) {
   const bool matched = out >= 0 && act < a.GT_total;
   const bool has_void = a.void_idx >= 0;
   const bool need_cls = a.force_cls || has_void;
-  const float coeff = a.g_cls[l] * (a.cls_scale * a.layer[l * ML_LAYERS + ML_LAYER_INV_CLS_DEN]);
+  const float coeff = a.g_cls[l * a.gs_cls] * (a.cls_scale * a.layer[l * ML_LAYERS + ML_LAYER_INV_CLS_DEN]);
   int64_t y = -1;
   bool zero = (!matched && !need_cls) || coeff == 0.f;
   if (!zero && matched) {
@@ -588,8 +588,8 @@ __device__ __forceinline__ void lut_load(const BwdArgs& a, int64_t it, int64_t n
   m.I = st[ML_STAT_I];
   m.T = st[ML_STAT_T];
   const float inv_md = a.layer[l * ML_LAYERS + ML_LAYER_INV_MASK_DEN];
-  m.mc = a.g_mask[l] * inv_md;
-  m.dc = a.g_dice[l] * inv_md;
+  m.mc = a.g_mask[l * a.gs_mask] * inv_md;
+  m.dc = a.g_dice[l * a.gs_dice] * inv_md;
   const int64_t act = m.out + (m.out >= a.bg ? 1 : 0);
   const int64_t actc = m.out >= 0 && act < a.GT_total ? act : 0;  // a valid slot to read
   const int64_t rbase = m.row * a.HW;

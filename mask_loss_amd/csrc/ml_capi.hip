@@ -935,6 +935,20 @@ int ml_mask_matching_backward(const ml_shape* s, const ml_params* p, const float
                               const int64_t* pred_to_gt, const void* saved,
                               int grad_prefilled, void* grad_mask_logits, void* grad_cls_logits,
                               void* workspace, size_t workspace_bytes, ml_stream_t stream) {
+  return ml_mask_matching_backward_strided(s, p, grad_mask, 1, grad_dice, 1, grad_cls, 1, mask_dtype, mask_logits,
+                                           mask_targets, cls_dtype, cls_logits, cls_targets, pred_to_gt, saved,
+                                           grad_prefilled, grad_mask_logits, grad_cls_logits, workspace,
+                                           workspace_bytes, stream);
+}
+
+int ml_mask_matching_backward_strided(const ml_shape* s, const ml_params* p, const float* grad_mask,
+                                      int64_t grad_mask_stride, const float* grad_dice, int64_t grad_dice_stride,
+                                      const float* grad_cls, int64_t grad_cls_stride, int mask_dtype,
+                                      const void* mask_logits, const int64_t* mask_targets, int cls_dtype,
+                                      const void* cls_logits, const int64_t* cls_targets,
+                                      const int64_t* pred_to_gt, const void* saved, int grad_prefilled,
+                                      void* grad_mask_logits, void* grad_cls_logits, void* workspace,
+                                      size_t workspace_bytes, ml_stream_t stream) {
   int rc = check_params(p, s->C, true);
   if (rc) return rc;
   if (!dtype_ok(mask_dtype) || !dtype_ok(cls_dtype)) return fail(ML_EINVAL, "unsupported dtype");
@@ -997,6 +1011,9 @@ int ml_mask_matching_backward(const ml_shape* s, const ml_params* p, const float
   ba.g_mask = grad_mask;
   ba.g_dice = grad_dice;
   ba.g_cls = grad_cls;
+  ba.gs_mask = grad_mask_stride;
+  ba.gs_dice = grad_dice_stride;
+  ba.gs_cls = grad_cls_stride;
   ba.grad = grad_mask_logits;
   ba.cls_logits = cls_logits;
   ba.cls_dtype = cls_dtype;

@@ -405,6 +405,7 @@ struct BwdArgs {
   const float* g_mask;
   const float* g_dice;
   const float* g_cls;
+  int64_t gs_mask, gs_dice, gs_cls;  // their strides over the layers
   void* grad;             // (L,B,Q,HW) in dtype
   const void* cls_logits;
   int cls_dtype;

@@ -1,0 +1,61 @@
+"""Forms of the matching step beside those of test_gpu_parity.py: upstream
+gradients at other strides, and the strategies with more columns than lanes."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import assign as OA  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ml():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import mask_loss_amd
+    return mask_loss_amd.mask_loss
+
+
+def inputs(seed, L, B, Q, H, W, G, C, dtype=torch.float32):
+    rng = np.random.default_rng(seed)
+    z = torch.from_numpy(rng.normal(0, 2, size=(L, B, Q, H, W)).astype(np.float32)).to(dtype).cuda()
+    t = torch.from_numpy(rng.integers(0, G + 1, size=(B, H, W))).cuda()
+    zc = torch.from_numpy(rng.normal(size=(L, B, Q, C)).astype(np.float32)).cuda()
+    ct = torch.from_numpy(rng.integers(0, C - 1, size=(B, G + 1))).cuda()
+    return z, t, zc, ct
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", ["broadcast", "every_other", "column"])
+def test_upstream_gradient_strides(ml, dtype, form):
+    L = 3
+    z, t, zc, ct = inputs(1, L, 2, 12, 9, 16, 5, 4, dtype)
+    head, tail = (1.0, 1.0, 1.0, 1.0, 0, 1.0, 0.05), (0.0, -1.0, 0.0, -1.0, 3, True, True)
+    out = ml.mask_matching_fused(z, t, zc, ct, *head, 1e30, -1.0, True, False, 1, 0, *tail)
+    if form == "broadcast":
+        g = [torch.tensor(v, device="cuda").expand(L) for v in (1.0, 0.5, -2.0)]
+    elif form == "every_other":
+        g = [torch.arange(2 * L, device="cuda", dtype=torch.float32).add_(k)[::2] for k in range(3)]
+    else:
+        g = list(torch.randn(L, 3, device="cuda").unbind(1))
+    args = (z, t, zc, ct, out[0], *head, -1.0, True, False, *tail, out[5])
+    got = ml.mask_matching_backward_fused(*g, *args)
+    ref = ml.mask_matching_backward_fused(*[x.contiguous() for x in g], *args)
+    assert all(x.stride(0) != 1 for x in g)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+    assert got[0].abs().sum() > 0
+
+
+@pytest.mark.parametrize("strategy", [0, 1, 2, 3])
+@pytest.mark.parametrize("K,G,Q", [(1, 70, 200), (2, 70, 100), (3, 130, 150), (2, 3, 40)])
+def test_strategies_with_many_columns(ml, strategy, K, G, Q):
+    z, t, zc, ct = inputs(2, 1, 2, Q, 24, 24, G, 6)
+    head, tail = (1.0, 1.0, 1.0, 1.0, 0, 1.0, 0.05), (0.0, -1.0, 0.0, -1.0, 5, True, True)
+    out = ml.mask_matching(z, t, zc, ct, *head, 1e30, -1.0, True, False, K, strategy, *tail)
+    sep = ml.pairwise_mask_loss_forward(z, t, zc, ct, *head, 0.0, -1.0, 0.0, -1.0, True, True)
+    total = ((sep[0] + sep[1]) + sep[2]).double().cpu().numpy().reshape(2, Q, G)
+    p2g, rounds = OA.assign_batch(total, 1e30, K, strategy)
+    assert np.array_equal(out[0].cpu().numpy().reshape(2, Q), p2g)
+    assert np.array_equal(out[1].cpu().numpy().reshape(2, Q), rounds)
