@@ -139,13 +139,12 @@ __device__ __forceinline__ RowCoef row_coef(const BwdArgs& a, float S, float P, 
 }
 
 // d(loss)/dz of one cell with target count tk
-template <int EM = 0>
 __device__ __forceinline__ float grad_elem(float z, float tk, const ElemParams& ep, float N2,
                                            const RowCoef& r) {
   const Sig s = sig_terms(z);
-  const float w = unc_weight_m<EM>(s, ep);
+  const float w = unc_weight(s, ep);
   float mn, mp;
-  focal_mods_m<EM>(s, ep, mn, mp);
+  focal_mods(s, ep, mn, mp);
   const float g = ep.gamma;
   const float negc = fmaxf(N2 - tk, 0.f);
   const float gpos = -w * ep.ap * tk * mp * (g * s.p * s.cp + s.q1);
@@ -221,6 +220,32 @@ __global__ __launch_bounds__(256) void bwd_mask_kernel(BwdArgs a) {
   }
 }
 
+// The same for the operator's default modes (no focal terms, weight H^1, no
+// alphas), with the row's factors multiplied out:
+//   w (k1 ((N2 - t) p - t (1-p)) + p (1-p) (k2 - k3 t)).
+// With e = exp(-|z|), d = 1 + e: p (1-p) = (e / d) (1 / d), and the entropy is
+// log2 d + (e / d) |z| log2 e.
+struct RowMul {
+  float k1, k2, k3;
+};
+__device__ __forceinline__ RowMul row_mul(const RowCoef& r, float N2) {
+  const float d = r.dc * r.kd;
+  return RowMul{r.mc * r.sf, d * r.num * N2, d * 2.f * r.D};
+}
+__device__ __forceinline__ float grad_elem_default(float z, float tk, float ug_min, float N2, const RowMul& k) {
+  const float t = -fabsf(z) * kLog2e;
+  const float e = __builtin_amdgcn_exp2f(t);
+  const float d = 1.f + e;
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float er = e * r;
+  const float h = __builtin_fmaf(-er, t, __builtin_amdgcn_logf(d));
+  const float w = __builtin_amdgcn_fmed3f(h, ug_min, 1.f);
+  const bool up = z >= 0.f;
+  const float p = up ? r : er, q = up ? er : r;
+  const float a = __builtin_fmaf(N2 - tk, p, -(tk * q));
+  return w * __builtin_fmaf(k.k1, a, er * r * __builtin_fmaf(-k.k3, tk, k.k2));
+}
+
 // Statistics-driven path: one workgroup per (row, chunk of kBwdChunk cells);
 // each thread issues all kBwdU of its logit / label loads before computing,
 // so a matched row is spread over many workgroups and its loads overlap.
@@ -258,6 +283,8 @@ __device__ __forceinline__ void bwd_chunk(const BwdArgs& a, int64_t row, int64_t
   const float T = matched ? st[ML_STAT_T] : 0.f;
   const RowCoef rc = row_coef(a, S, P, I, T, mc, dc);
   const ElemParams ep = a.mask_ep;
+  const bool plain = default_modes(ep) && ep.an == 1.f && ep.ap == 1.f;
+  const RowMul rm = row_mul(rc, a.N2);
   float z[kBwdU][8], t[kBwdU][8];
 #pragma unroll
   for (int u = 0; u < kBwdU; ++u) {
@@ -273,9 +300,9 @@ __device__ __forceinline__ void bwd_chunk(const BwdArgs& a, int64_t row, int64_t
     if (cell0 < a.HW) {
       float gr[8];
       // one branch on the modes per 8 cells (wave-uniform), not per cell
-      if (default_modes(ep)) {
+      if (plain) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) gr[k] = grad_elem<1>(z[u][k], matched ? t[u][k] : 0.f, ep, a.N2, rc);
+        for (int k = 0; k < 8; ++k) gr[k] = grad_elem_default(z[u][k], matched ? t[u][k] : 0.f, ep.ug_min, a.N2, rm);
       } else {
 #pragma unroll
         for (int k = 0; k < 8; ++k) gr[k] = grad_elem(z[u][k], matched ? t[u][k] : 0.f, ep, a.N2, rc);
