@@ -1040,6 +1040,7 @@ int ml_mask_matching_backward_strided(const ml_shape* s, const ml_params* p, con
 namespace {
 struct DensePlan {
   Dims d;             // B, H, W, Ht, Wt, s, HW, HWp, counts_mode; GT_total := C
+  int64_t groups;     // dense_groups: > 0: no targets in the workspace
   size_t tgt_bytes, partial_off, total;
 };
 
@@ -1073,15 +1074,26 @@ bool dense_plan(const ml_dense_shape* s, bool dice, bool backward, DensePlan& P,
   d.counts_mode = d.s > 1;
   d.cw = d.s >= 16 ? 2 : 1;
   d.crows = d.C;
-  P.tgt_bytes = align256(target_bytes(d));
+  P.groups = dense_groups(d.B, d.C, d.HW, d.s, dice, backward);
+  P.tgt_bytes = P.groups ? 0 : align256(target_bytes(d));
   P.partial_off = P.tgt_bytes;
-  P.total = P.tgt_bytes + (backward ? 0 : align256(dense_partials_bytes(d.L, d.B, d.C, d.HW, dice)));
+  P.total = P.tgt_bytes + (backward ? 0 : align256(dense_partials_bytes(d.L, d.B, d.C, d.HW, P.groups, dice)));
+  if (P.groups) P.total = std::max<size_t>(P.total, 256);  // a size of 0 stands for an unsupported shape
   return true;
 }
 
 int dense_prep(const DensePlan& P, const int64_t* targets, unsigned char* w, DenseArgs& a,
                hipStream_t st) {
   const Dims& d = P.d;
+  a.L = d.L; a.B = d.B; a.C = d.C; a.HW = d.HW; a.HWp = d.HWp; a.HtWt = d.Ht * d.Wt;
+  a.N2 = (float)d.N2;
+  a.groups = P.groups;
+  if (P.groups) {
+    a.targets = targets;
+    a.W = d.W; a.Ht = d.Ht; a.Wt = d.Wt; a.s = d.s;
+    a.tvec = (uintptr_t)targets % 16 == 0;
+    return ML_OK;
+  }
   PrepArgs pa{};
   pa.targets = targets;
   set_targets(pa, d, w);
@@ -1092,8 +1104,6 @@ int dense_prep(const DensePlan& P, const int64_t* targets, unsigned char* w, Den
   pa.GT_total = d.C; pa.GT_out = d.C; pa.bg = d.C;
   a.lab16 = pa.lab16;
   a.counts = pa.counts;
-  a.L = d.L; a.B = d.B; a.C = d.C; a.HW = d.HW; a.HWp = d.HWp; a.HtWt = d.Ht * d.Wt;
-  a.N2 = (float)d.N2;
   if (d.B == 0) return ML_OK;
   return launch_prep(pa, d, st);
 }

@@ -427,7 +427,11 @@ struct DenseArgs {
   const void* logits;
   int dtype;
   const uint16_t* lab16;   // s == 1: label per cell (0xFFFF outside [0, C))
-  CountTiles counts;       // s > 1, one row per class
+  CountTiles counts;       // s > 1, one row per class; unset where groups > 0
+  int64_t groups;          // > 0: class groups of the kernels that count for themselves (dense_groups)
+  const int64_t* targets;  // ... from the label maps (B, Ht, Wt)
+  int64_t W, Ht, Wt, s;
+  int tvec;                // ... which start on a 16-byte boundary, as each row's pixel pairs do
   int64_t L, B, C, HW, HWp, HtWt;
   float N2;
   ElemParams ep;           // focal terms (sigmoid CE)
@@ -516,7 +520,8 @@ int launch_point_labels(const int64_t* targets, const float* coords, int64_t B, 
                         int64_t Wt, int64_t P, int64_t GT_total, int64_t bg, int64_t* out64,
                         uint16_t* codes, int64_t HWp, hipStream_t st);
 int launch_dense(const DenseArgs& a, bool dice, bool backward, hipStream_t st);
-size_t dense_partials_bytes(int64_t L, int64_t B, int64_t C, int64_t HW, bool dice);
+int64_t dense_groups(int64_t B, int64_t C, int64_t HW, int64_t s, bool dice, bool backward);
+size_t dense_partials_bytes(int64_t L, int64_t B, int64_t C, int64_t HW, int64_t groups, bool dice);
 int launch_zero_fill(void* p, size_t bytes, hipStream_t st);
 
 // Zero `n16` 16-byte words, then `ntail` trailing bytes, as workgroup `blk`

@@ -13,6 +13,7 @@
 // cost schedule.
 #include <algorithm>
 
+#include "ml_counts.h"
 #include "ml_internal.h"
 
 namespace ml {
@@ -322,8 +323,6 @@ __global__ __launch_bounds__(256) void prep_labels_kernel(PrepArgs a) {
 // at s = 4 with 61 rows: 22.6 us (67 MB read, 32 MB written, 4.4 TB/s; a copy
 // runs at 5.15), against 6.7 + 24.5 us for clearing the counts and adding to
 // them in memory pixel by pixel.
-constexpr int kCntCells = 256;
-constexpr int kCntThreads = 4 * kCntCells;
 constexpr size_t kCntLds = 40 * 1024;  // of the rows in LDS: three workgroups per CU
 template <int CW, int S>
 __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, int rc, int vec) {
@@ -337,50 +336,14 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
   const int64_t HW = a.H * a.W;
   const bool mark = a.pbits != nullptr;
   if (mark) pres_clear(pres);
-  const int tid = threadIdx.x, cl = tid >> 2, sub = tid & 3;
-  const int64_t cell = (int64_t)blockIdx.x * kCntCells + cl;
-  const bool in = cell < HW;
-  const int64_t s = S ? S : a.s;
-  const int64_t ci = in ? cell / a.W : 0, cj = in ? cell - ci * a.W : 0;
-  const int64_t* src = a.targets + (b * a.Ht + ci * s) * a.Wt + cj * s;
-  // row of a label in the tiles, -1 for none
-  auto row_of = [&](int64_t lab) -> int {
-    return (uint64_t)lab < (uint64_t)a.GT_total && (a.rest < 0 || lab != a.bg) ? (int)lab : (int)a.rest;
-  };
+  const int tid = threadIdx.x, cl = tid >> 2;
   auto clear = [&]() {
     for (int i = tid; i < rc * (kCntCells * CW / 16); i += kCntThreads) ((uint4*)tile)[i] = make_uint4(0u, 0u, 0u, 0u);
   };
-  int64_t lab[S ? S : 1];
-  bool whole = false;  // every pixel of the cell carries lab[0]
-  bool first = true;   // ... and the wave's first cell does not already mark that label
-  if constexpr (S != 0) {
-    const bool act = in && sub < S;
-    if (act) {
-      const int64_t* p = src + sub * a.Wt;
-      if (vec) {
-#pragma unroll
-        for (int k = 0; k < S; k += 2) {
-          const longlong2 v = *(const longlong2*)(p + k);
-          lab[k] = v.x;
-          lab[k + 1] = v.y;
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < S; ++k) lab[k] = p[k];
-      }
-    }
-    clear();  // while the labels are on their way
-    const int64_t l0 = __shfl(act ? lab[0] : 0, (tid & 63) & ~3, 64);
-    bool same = !act || lab[0] == l0;
-#pragma unroll
-    for (int k = 1; k < S; ++k) same = same && (!act || lab[k] == l0);
-    const uint64_t m = __ballot(same);
-    whole = in && ((m >> ((tid & 63) & ~3)) & 0xFull) == 0xFull;
-    const int64_t lw = __shfl(lab[0], 0, 64);
-    first = (tid & 63) == 0 || (m & 0xFull) != 0xFull || lab[0] != lw;
-  } else {
-    clear();
-  }
+  CellLabels<S> px;
+  px.load(a.targets, b, a.Ht, a.Wt, a.W, HW, a.s, (int64_t)blockIdx.x * kCntCells + cl, vec != 0);
+  clear();  // while the labels are on their way
+  px.settle();
   uint8_t* const out0 = (uint8_t*)a.counts.p;
   for (int64_t r0 = 0; r0 < a.counts.rows; r0 += rc) {  // one round unless there are many rows
     const int64_t nr = min((int64_t)rc, a.counts.rows - r0);
@@ -388,57 +351,16 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
     __syncthreads();
     const int64_t ones = a.rest + 1 - r0;  // the ones column's row: 4 CW words in each of the four blocks
     if (a.rest >= 0 && ones >= 0 && ones < nr && tid < 16 * CW) {
-      const uint32_t v = (uint32_t)(s * s) * (CW == 1 ? 0x01010101u : 0x00010001u);
+      const uint32_t v = (uint32_t)(px.s * px.s) * (CW == 1 ? 0x01010101u : 0x00010001u);
       ((uint4*)tile)[(int)((tid / (4 * CW)) * nr + ones) * 4 * CW + tid % (4 * CW)] = make_uint4(v, v, v, v);
     }
-    // n pixels of one label in this thread's cell
-    auto add = [&](int64_t lb, uint32_t n, bool single) {
-      const bool valid = (uint64_t)lb < (uint64_t)a.GT_total;
-      if (mark && valid && r0 == 0 && !(single && !first)) pres_mark(pres, lb);
-      const int64_t r = (int64_t)row_of(lb) - r0;
-      if (r < 0 || r >= nr) return;
-      const uint32_t e = (uint32_t)(((cl >> 6) * nr + r) * kCountCells + (cl & (kCountCells - 1)));
-      if (single) {
-        if constexpr (CW == 1) tile[e] = (unsigned char)n;
-        else ((uint16_t*)tile)[e] = (uint16_t)n;
-      } else if constexpr (CW == 1) {
-        atomicAdd((uint32_t*)tile + (e >> 2), n << ((e & 3u) * 8u));
-      } else {
-        atomicAdd((uint32_t*)tile + (e >> 1), n << ((e & 1u) * 16u));
-      }
-    };
-    if constexpr (S != 0) {
-      if (whole) {
-        if (sub == 0) add(lab[0], S * S, true);
-      } else if (in && sub < S) {
-        uint32_t n = 1;
-#pragma unroll
-        for (int k = 1; k < S; ++k) {
-          if (lab[k] != lab[k - 1]) {
-            add(lab[k - 1], n, false);
-            n = 0;
-          }
-          ++n;
-        }
-        add(lab[S - 1], n, false);
-      }
-    } else if (in) {
-      for (int64_t dy = sub; dy < s; dy += 4) {
-        const int64_t* p = src + dy * a.Wt;
-        int64_t run = p[0];
-        uint32_t n = 1;
-        for (int64_t dx = 1; dx < s; ++dx) {
-          const int64_t v = p[dx];
-          if (v != run) {
-            add(run, n, false);
-            run = v;
-            n = 0;
-          }
-          ++n;
-        }
-        add(run, n, false);
-      }
-    }
+    px.runs([&](int64_t lab, uint32_t n, bool single) {
+      const bool valid = (uint64_t)lab < (uint64_t)a.GT_total;
+      if (mark && valid && r0 == 0 && !(single && !px.first)) pres_mark(pres, lab);
+      // a label of no column counts in the row kept for those (or nowhere)
+      const int64_t r = (valid && (a.rest < 0 || lab != a.bg) ? lab : a.rest) - r0;
+      if (r >= 0 && r < nr) tile_add<CW>(tile, (int)nr, (int)r, cl, n, single);
+    });
     __syncthreads();
     // rows [r0, r0 + nr) of each of this workgroup's blocks (all rows: one run)
     const uint32_t per = (uint32_t)(nr * kCountCells * CW / 16);  // 16-byte words

@@ -123,3 +123,31 @@ def test_dense(ml, shape):
     ref = O.dice_loss_backward(go.cpu().numpy(), z64, t, *sums, 1.0, nm, 1.5)
     close_extra(ml.backward_dice_loss(go, zt, tt, I, P, T, 1.0, nm, 1.5).cpu().numpy(), ref, 1e-5,
                 1e-2 * np.abs(ref).max(), dice_grad_cancellation(go.cpu().numpy(), z64, t, *sums, 1.0, nm, 1.5))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("shape", [(2, 8, 8, 1, True), (3, 15, 17, 16, False), (4, 16, 20, 17, True),
+                                   (4, 16, 16, 161, False), (15, 5, 13, 330, False), (15, 4, 4, 3, True)],
+                         ids=lambda v: "s%d_%dx%d_C%d_%d" % v)
+def test_dense_groups(ml, shape, dtype):
+    """The kernels that count for themselves: class groups of 1, 16 and 17
+    rows, two groups by LDS (161), the counts in memory (330 classes at s = 15)."""
+    s, H, W, C, shifted = shape
+    rng = np.random.default_rng(s * H + C)
+    L, B = 2, 2
+    t = label_map(rng, B, H, W, s, C - 1, 0.3)
+    zt, z64 = rounded(rng.normal(0, 2.0, size=(L, B, C, H, W)), dtype)
+    zt, tt = zt.cuda(), on_gpu(t, shifted)
+    nm, go = float(L * B * C), torch.tensor([1.0, -0.5], device="cuda")
+    close(ml.forward_sigmoid_ce_loss(zt, tt, nm, 1.5, 2.0, 0.25).cpu().numpy(),
+          O.sigmoid_ce_loss(z64, t, nm, 1.5, 2.0, 0.25), 1e-5, 1e-2)
+    # half the spacing of float16 below 2^-14, where these gradients lie
+    sub = 2.0 ** -25 if dtype == "float16" else 0.0
+    ref = O.sigmoid_ce_backward(go.cpu().numpy(), z64, t, nm, 1.5, 2.0, 0.25)
+    close_extra(ml.backward_sigmoid_ce_loss(go, zt, tt, nm, 1.5, 2.0, 0.25).float().cpu().numpy(), ref, RTOL[dtype],
+                1e-2 * np.abs(ref).max(), sub)
+    loss, I, P, T = ml.forward_dice_loss(zt, tt, 1.0, nm, 1.5)
+    sums = [v.cpu().numpy() for v in (I, P, T)]
+    ref = O.dice_loss_backward(go.cpu().numpy(), z64, t, *sums, 1.0, nm, 1.5)
+    close_extra(ml.backward_dice_loss(go, zt, tt, I, P, T, 1.0, nm, 1.5).float().cpu().numpy(), ref, RTOL[dtype],
+                1e-2 * np.abs(ref).max(), sub + dice_grad_cancellation(go.cpu().numpy(), z64, t, *sums, 1.0, nm, 1.5))
