@@ -258,7 +258,7 @@ int launch_point_sample(int dtype, const void* in, const float* coords, int64_t 
 // * global float atomics into a float workspace and a conversion pass for
 //   larger planes.
 // On 800 planes of 128 x 128 with 12,544 points and 20% of the rows nonzero
-// (configuration 2), the grouped form takes 102 us (bucket sort 34 us, gather
+// (configuration 2), the grouped form takes 84 us (bucket sort 16 us, gather
 // 68 us) against 146 us for the LDS atomics (38 us with plain, racy adds:
 // the atomics bind it); global float atomics take 1.9 ms, and a radix sort
 // of the corner entries (18 launches) took 110 us alone.  Samples with a
@@ -385,49 +385,79 @@ static CsrLayout csr_layout(int64_t H, int64_t W, int64_t P, int64_t cb) {
   return l;
 }
 
-// One workgroup per coordinate set.
+// kCsrParts workgroups per coordinate set, each sorting the points of its own
+// run of buckets.  grid (sets, kCsrParts)
+//
+// One workgroup per set is bound by its CU: 12,544 points leave as 25,000
+// scattered stores and 66 KB of offsets (33.5 us on 8 sets, 8 CUs at work).
+// Here every part reads all points (100 KB, from L2), keeps those of its
+// buckets in an LDS list, counts the ones before its first bucket, and writes
+// its own eighth: 15.5 us, half of it the points' arithmetic, which all parts do.
+constexpr int kCsrParts = 8;
+constexpr int kCsrPartBuckets = (int)((kCsrMaxBuckets + kCsrParts - 1) / kCsrParts);
+constexpr int kCsrPointBits = 14;
+static_assert(kCsrMaxPoints <= (1 << kCsrPointBits), "a list entry is a point and a local bucket");
 __global__ __launch_bounds__(kCsrThreads) void corner_csr_kernel(const float* coords, int H, int W, int P,
                                                                  int align, uint32_t* off_all,
                                                                  uint32_t* pt_all, float4* wt_all) {
-  __shared__ uint32_t cnt[kCsrMaxBuckets];
-  __shared__ uint32_t wsum[kCsrThreads / 64];
+  __shared__ uint32_t cnt[kCsrPartBuckets];
+  __shared__ uint32_t list[kCsrMaxPoints];  // this part's points: point | local bucket << kCsrPointBits
+  __shared__ uint32_t wsum[kCsrThreads / 64], wseen[kCsrThreads / 64];
+  __shared__ uint32_t nlist;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t set = blockIdx.x;
   const int NB = (H + 1) * (W + 1);
+  const int per = (NB + kCsrParts - 1) / kCsrParts, first = min((int)blockIdx.y * per, NB);
+  const int nb = min(per, NB - first);  // 0 in the last parts of a tiny plane
   const float* cs = coords + set * P * 2;
   uint32_t* off = off_all + set * (NB + 1);
   uint32_t* pt = pt_all + set * P;
   float4* wt = wt_all + set * P;
   const bool al = align != 0;
-  // the set's points, kCsrPointsPerThread per thread, all loads issued at once
-  // (and again for the scatter, from the cache, rather than held across the scan)
-  float2 xy[kCsrPointsPerThread];
-  auto load_points = [&]() {
+  float2 xy[kCsrPointsPerThread];  // all loads issued at once
 #pragma unroll
-    for (int u = 0; u < kCsrPointsPerThread; ++u) {
-      const int p = u * kCsrThreads + tid;
-      xy[u] = p < P ? *(const float2*)(cs + 2 * p) : make_float2(0.f, 0.f);
-    }
-  };
-  load_points();
-  for (int i = tid; i < NB; i += kCsrThreads) cnt[i] = 0u;
+  for (int u = 0; u < kCsrPointsPerThread; ++u) {
+    const int p = u * kCsrThreads + tid;
+    xy[u] = p < P ? *(const float2*)(cs + 2 * p) : make_float2(0.f, 0.f);
+  }
+  for (int i = tid; i < nb; i += kCsrThreads) cnt[i] = 0u;
+  if (tid == 0) nlist = 0u;
   __syncthreads();
-  int bk[kCsrPointsPerThread];  // the point's bucket, -1 when no corner is in the plane
+  int bk[kCsrPointsPerThread];  // the point's local bucket, -1 outside this part's
+  uint32_t mine = 0, seen = 0;  // seen: points of earlier buckets, points of all buckets << 16
 #pragma unroll
   for (int u = 0; u < kCsrPointsPerThread; ++u) {
     const int p = u * kCsrThreads + tid;
     const float c2[2] = {xy[u].x, xy[u].y};
     const Corners<int> c = corners_of<int>(c2, H, W, al);
-    const bool any = c.k[0] | c.k[1] | c.k[2] | c.k[3];
-    bk[u] = p < P && any ? (c.y0 + 1) * (W + 1) + (c.x0 + 1) : -1;
-    if (bk[u] >= 0) atomicAdd(&cnt[bk[u]], 1u);
+    const bool any = p < P && (c.k[0] | c.k[1] | c.k[2] | c.k[3]);
+    const int lb = (c.y0 + 1) * (W + 1) + (c.x0 + 1) - first;
+    const bool own = any && lb >= 0 && lb < nb;
+    seen += any ? (lb < 0 ? 0x10001u : 0x10000u) : 0u;
+    bk[u] = own ? lb : -1;
+    mine += own;
+    if (own) atomicAdd(&cnt[lb], 1u);
   }
+  uint32_t at = mine;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t t = __shfl_up(at, d, 64);
+    if (lane >= d) at += t;
+    seen += __shfl_xor(seen, d, 64);
+  }
+  uint32_t base = 0;
+  if (lane == 63) base = atomicAdd(&nlist, at);
+  at += __shfl(base, 63, 64) - mine;
+  if (lane == 0) wseen[wave] = seen;
+#pragma unroll
+  for (int u = 0; u < kCsrPointsPerThread; ++u)
+    if (bk[u] >= 0) list[at++] = (uint32_t)(u * kCsrThreads + tid) | (uint32_t)bk[u] << kCsrPointBits;
   __syncthreads();
   // thread t scans the run of R consecutive buckets starting at t R
-  const int R = (NB + kCsrThreads - 1) / kCsrThreads, b0 = tid * R;
+  const int R = (nb + kCsrThreads - 1) / kCsrThreads, b0 = tid * R;
   uint32_t run = 0;
   for (int k = 0; k < R; ++k)
-    if (b0 + k < NB) run += cnt[b0 + k];
+    if (b0 + k < nb) run += cnt[b0 + k];
   uint32_t incl = run;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -436,30 +466,29 @@ __global__ __launch_bounds__(kCsrThreads) void corner_csr_kernel(const float* co
   }
   if (lane == 63) wsum[wave] = incl;
   __syncthreads();
-  uint32_t pos = incl - run, total = 0;
+  uint32_t pos = incl - run, all = 0;
   for (int w = 0; w < kCsrThreads / 64; ++w) {
-    pos += w < wave ? wsum[w] : 0u;
-    total += wsum[w];
+    pos += (w < wave ? wsum[w] : 0u) + (wseen[w] & 0xFFFFu);
+    all += wseen[w] >> 16;
   }
   for (int k = 0; k < R; ++k)
-    if (b0 + k < NB) {
+    if (b0 + k < nb) {
       const uint32_t n = cnt[b0 + k];
-      off[b0 + k] = pos;
+      off[first + b0 + k] = pos;
       cnt[b0 + k] = pos;  // the bucket's next free record
       pos += n;
     }
-  if (tid == 0) off[NB] = total;
-  load_points();
+  if (blockIdx.y == 0 && tid == 0) off[NB] = all;
   __syncthreads();
-#pragma unroll
-  for (int u = 0; u < kCsrPointsPerThread; ++u) {
-    if (bk[u] < 0) continue;
-    const int p = u * kCsrThreads + tid;
-    const float c2[2] = {xy[u].x, xy[u].y};
+  const uint32_t n = nlist;
+  for (uint32_t i = tid; i < n; i += kCsrThreads) {
+    const uint32_t e = list[i], p = e & ((1u << kCsrPointBits) - 1u);
+    const float2 v = *(const float2*)(cs + 2 * p);
+    const float c2[2] = {v.x, v.y};
     const Corners<int> c = corners_of<int>(c2, H, W, al);
-    const uint32_t at = atomicAdd(&cnt[bk[u]], 1u);
-    pt[at] = (uint32_t)p;
-    wt[at] = make_float4(c.w[0], c.w[1], c.w[2], c.w[3]);
+    const uint32_t r = atomicAdd(&cnt[e >> kCsrPointBits], 1u);
+    pt[r] = p;
+    wt[r] = make_float4(c.w[0], c.w[1], c.w[2], c.w[3]);
   }
 }
 
@@ -673,7 +702,7 @@ static int launch_bwd_dt(const void* gout, const float* coords, int64_t N, int64
     uint32_t* pt = (uint32_t*)(w + l.pt);
     float4* wt = (float4*)(w + l.wt);
     const int64_t sets = std::min(cb, N);  // coordinate sets that some plane reads
-    hipLaunchKernelGGL(corner_csr_kernel, dim3((unsigned)sets), dim3(kCsrThreads), 0, st, coords, (int)H,
+    hipLaunchKernelGGL(corner_csr_kernel, dim3((unsigned)sets, kCsrParts), dim3(kCsrThreads), 0, st, coords, (int)H,
                        (int)W, (int)P, align, off, pt, wt);
     int rc = check_launch("point_sample_backward");
     if (rc) return rc;

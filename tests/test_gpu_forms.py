@@ -6,6 +6,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from oracle import assign as OA  # noqa: E402
+from oracle import points_oracle as PO  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +60,24 @@ def test_strategies_with_many_columns(ml, strategy, K, G, Q):
     p2g, rounds = OA.assign_batch(total, 1e30, K, strategy)
     assert np.array_equal(out[0].cpu().numpy().reshape(2, Q), p2g)
     assert np.array_equal(out[1].cpu().numpy().reshape(2, Q), rounds)
+
+
+@pytest.mark.parametrize("one_cell", [False, True])
+@pytest.mark.parametrize("H,W,P", [(1, 1, 50), (2, 1, 1025), (4, 8, 16384), (64, 128, 16384), (128, 128, 12544)])
+def test_point_gradient_buckets(ml, H, W, P, one_cell):
+    """The points' buckets split over workgroups: planes of fewer buckets than
+    workgroups, every point in one bucket, points outside the plane and
+    non-finite ones.  Quarter-cell positions and whole gradients make every
+    product and sum exact in float32, so the results are the oracle's."""
+    rng = np.random.default_rng(H + W + P)
+    B, C = 3, 8
+    size = np.array([W, H])
+    pos = rng.integers(-8, 4 * size + 8, size=(B, P, 2))
+    if one_cell:
+        pos = 4 * (size // 2) + rng.integers(0, 4, size=(B, P, 2)) - 4
+    c = ((pos / 4 + 0.5) / size).astype(np.float32)
+    g = rng.integers(-3, 4, size=(B, C, P)).astype(np.float64)
+    ref = PO.point_sample_backward(g[..., : P - 7], c[:, : P - 7], H, W, False)
+    c[:, P - 7:] = np.array([np.nan, np.inf, -np.inf, 1e30, -1e30, np.nan, 7.0])[:, None]
+    got = ml.point_sample_backward(torch.from_numpy(g).float().cuda(), torch.from_numpy(c).cuda(), H, W, False)
+    np.testing.assert_array_equal(got.cpu().numpy(), ref)
