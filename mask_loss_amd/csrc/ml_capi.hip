@@ -1040,7 +1040,7 @@ int ml_mask_matching_backward_strided(const ml_shape* s, const ml_params* p, con
 namespace {
 struct DensePlan {
   Dims d;             // B, H, W, Ht, Wt, s, HW, HWp, counts_mode; GT_total := C
-  int64_t groups;     // dense_groups: > 0: no targets in the workspace
+  int64_t groups;     // dense_groups
   size_t tgt_bytes, partial_off, total;
 };
 
@@ -1075,10 +1075,9 @@ bool dense_plan(const ml_dense_shape* s, bool dice, bool backward, DensePlan& P,
   d.cw = d.s >= 16 ? 2 : 1;
   d.crows = d.C;
   P.groups = dense_groups(d.B, d.C, d.HW, d.s, dice, backward);
-  P.tgt_bytes = P.groups ? 0 : align256(target_bytes(d));
+  P.tgt_bytes = align256(target_bytes(d));  // kept in the size where no counts are stored: one rule for callers
   P.partial_off = P.tgt_bytes;
   P.total = P.tgt_bytes + (backward ? 0 : align256(dense_partials_bytes(d.L, d.B, d.C, d.HW, P.groups, dice)));
-  if (P.groups) P.total = std::max<size_t>(P.total, 256);  // a size of 0 stands for an unsupported shape
   return true;
 }
 
