@@ -1044,7 +1044,7 @@ struct DensePlan {
   size_t tgt_bytes, partial_off, total;
 };
 
-bool dense_plan(const ml_dense_shape* s, bool dice, bool backward, DensePlan& P,
+bool dense_plan(const ml_dense_shape* s, int dtype, bool dice, bool backward, DensePlan& P,
                 std::string& err) {
   if (!s || s->L < 0 || s->B < 0 || s->C < 0 || s->H <= 0 || s->W <= 0) {
     err = "dense loss: invalid shape";
@@ -1074,7 +1074,7 @@ bool dense_plan(const ml_dense_shape* s, bool dice, bool backward, DensePlan& P,
   d.counts_mode = d.s > 1;
   d.cw = d.s >= 16 ? 2 : 1;
   d.crows = d.C;
-  P.groups = dense_groups(d.B, d.C, d.HW, d.s, dice, backward);
+  P.groups = dense_groups(d.L, d.B, d.C, d.HW, d.s, dtype == ML_F32, dice, backward);
   P.tgt_bytes = align256(target_bytes(d));  // kept in the size where no counts are stored: one rule for callers
   P.partial_off = P.tgt_bytes;
   P.total = P.tgt_bytes + (backward ? 0 : align256(dense_partials_bytes(d.L, d.B, d.C, d.HW, P.groups, dice)));
@@ -1111,7 +1111,7 @@ int dense_prep(const DensePlan& P, const int64_t* targets, unsigned char* w, Den
 size_t ml_dense_loss_workspace_size(const ml_dense_shape* s, int dtype, int dice, int backward) {
   DensePlan P;
   std::string err;
-  if (!dtype_ok(dtype) || !dense_plan(s, dice != 0, backward != 0, P, err)) return 0;
+  if (!dtype_ok(dtype) || !dense_plan(s, dtype, dice != 0, backward != 0, P, err)) return 0;
   return P.total;
 }
 
@@ -1121,7 +1121,7 @@ static int dense_call(const ml_dense_shape* s, int dtype, bool dice, bool backwa
   if (!dtype_ok(dtype)) return fail(ML_EINVAL, "unsupported dtype");
   DensePlan P;
   std::string err;
-  if (!dense_plan(s, dice, backward, P, err)) return fail(ML_EINVAL, err);
+  if (!dense_plan(s, dtype, dice, backward, P, err)) return fail(ML_EINVAL, err);
   if (ws_bytes < P.total) return fail(ML_EWORKSPACE, "workspace too small");
   unsigned char* w = (unsigned char*)ws;
   a.dtype = dtype;

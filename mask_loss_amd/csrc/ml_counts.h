@@ -1,4 +1,4 @@
-// The target pixels of one low-resolution cell, taken by four threads: the
+// The target pixels of one low-resolution cell, taken by T threads: the
 // building block of the label-count kernels (s > 1).
 #pragma once
 
@@ -7,10 +7,11 @@
 namespace ml {
 
 constexpr int kCntCells = 256;              // cells per workgroup: four 64-cell blocks
-constexpr int kCntThreads = 4 * kCntCells;  // thread 4 c + k: every fourth target row of cell c, from row k
+constexpr int kCntThreads = 4 * kCntCells;
 
-// S = s for the unrolled forms 2 and 4, else 0.
-template <int S>
+// S = s for the unrolled forms 2 and 4, else 0.  Thread T c + k takes every
+// T-th target row of cell c, from row k (T = 2 only for S = 2).
+template <int S, int T = 4>
 struct CellLabels {
   int64_t lab[S ? S : 1];
   const int64_t* src;  // the cell's first pixel
@@ -25,7 +26,7 @@ struct CellLabels {
                                        int64_t HW, int64_t s_, int64_t cell, bool vec) {
     in = cell < HW;
     s = S ? S : (int)s_;
-    sub = threadIdx.x & 3;
+    sub = threadIdx.x & (T - 1);
     Wt = Wt_;
     const int64_t ci = in ? cell / W : 0, cj = in ? cell - ci * W : 0;
     src = targets + (b * Ht + ci * s) * Wt + cj * s;
@@ -51,14 +52,15 @@ struct CellLabels {
     if constexpr (S != 0) {
       const int lane = threadIdx.x & 63;
       const bool act = in && sub < S;
-      const int64_t l0 = __shfl(act ? lab[0] : 0, lane & ~3, 64);
+      const int64_t l0 = __shfl(act ? lab[0] : 0, lane & ~(T - 1), 64);
       bool same = !act || lab[0] == l0;
 #pragma unroll
       for (int k = 1; k < S; ++k) same = same && (!act || lab[k] == l0);
       const uint64_t m = __ballot(same);
-      whole = in && ((m >> (lane & ~3)) & 0xFull) == 0xFull;
+      constexpr uint64_t all = (1u << T) - 1u;
+      whole = in && ((m >> (lane & ~(T - 1))) & all) == all;
       const int64_t lw = __shfl(lab[0], 0, 64);
-      first = lane == 0 || (m & 0xFull) != 0xFull || lab[0] != lw;
+      first = lane == 0 || (m & all) != all || lab[0] != lw;
     }
   }
   // f(label, n, single): this thread's pixels as runs of one label; single:
@@ -81,7 +83,7 @@ struct CellLabels {
         f(lab[S - 1], n, false);
       }
     } else if (in) {
-      for (int dy = sub; dy < s; dy += 4) {
+      for (int dy = sub; dy < s; dy += T) {
         const int64_t* p = src + dy * Wt;
         int64_t run = p[0];
         uint32_t n = 1;

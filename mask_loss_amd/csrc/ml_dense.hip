@@ -448,13 +448,26 @@ __global__ __launch_bounds__(kCntThreads) void dense_fused_kernel(DenseArgs a, i
 // (kFuseRows) make more groups, each reads the labels (8 s^2 bytes a cell)
 // again, against the 2 bytes per cell and class of storing and reading a count.
 constexpr int64_t kFuseRows = 160;
+// A wave takes a class row, so below 16 classes waves are idle while the labels
+// of 256 cells wait: 2 classes of 8 maps of 512 x 512, s = 2: CE forward 71 us
+// against 34 with the counts in memory, gradients 81 and 74 against 33 and 30;
+// 19 classes of 6 x 2 maps of 256 x 256, s = 2: 28, 31 and 27 against 34, 38 and 31.
+constexpr int64_t kFuseLeast = 16;
+// The counts' launch saves a fixed time, and streaming 4 cells per lane under
+// the labels' wait is slower per logit than the plane kernels (8 cells per
+// lane), more so for 16-bit logits.  float32: 17 M logits 39, 48 and 43 us
+// against 65, 71 and 63; 34 M 96, 127 and 123 against 67, 93 and 88.  bf16 /
+// float16: 12.5 M 29, 26 and 22 against 31, 34 and 26; 16 M 40, 49 and 40
+// against 29, 33 and 23; 84 M 126, 163 and 170 against 90, 133 and 91.
+constexpr int64_t kFuseElems = 3 << 22;
 // More groups than that only where the cells alone would leave CUs without a
 // workgroup: with 256 workgroups of 150 classes the three kernels below take
 // 16.0, 20.6 and 18.8 us, with 512 of 75 classes 16.6, 24.9 and 23.3, with
 // 1024 of 38 classes 21.6, 30.8 and 28.2.
 constexpr int64_t kFuseBlocks = 256;
-int64_t dense_groups(int64_t B, int64_t C, int64_t HW, int64_t s, bool dice, bool backward) {
-  if (s < 2 || s > 15 || (dice && !backward) || B < 1 || C < 1 || B > 65535) return 0;
+int64_t dense_groups(int64_t L, int64_t B, int64_t C, int64_t HW, int64_t s, bool f32, bool dice, bool backward) {
+  if (s < 2 || s > 15 || (dice && !backward) || B < 1 || C < kFuseLeast || B > 65535) return 0;
+  if (L * B * C * HW > kFuseElems * (f32 ? 2 : 1)) return 0;
   const int64_t least = ceil_div(C, kFuseRows);
   if ((least - 1) * 8 * s * s > 2 * C) return 0;
   const int64_t fill = std::min(ceil_div(kFuseBlocks, ceil_div(HW, kCntCells) * B), ceil_div(C, 16));

@@ -520,7 +520,7 @@ int launch_point_labels(const int64_t* targets, const float* coords, int64_t B, 
                         int64_t Wt, int64_t P, int64_t GT_total, int64_t bg, int64_t* out64,
                         uint16_t* codes, int64_t HWp, hipStream_t st);
 int launch_dense(const DenseArgs& a, bool dice, bool backward, hipStream_t st);
-int64_t dense_groups(int64_t B, int64_t C, int64_t HW, int64_t s, bool dice, bool backward);
+int64_t dense_groups(int64_t L, int64_t B, int64_t C, int64_t HW, int64_t s, bool f32, bool dice, bool backward);
 size_t dense_partials_bytes(int64_t L, int64_t B, int64_t C, int64_t HW, int64_t groups, bool dice);
 int launch_zero_fill(void* p, size_t bytes, hipStream_t st);
 

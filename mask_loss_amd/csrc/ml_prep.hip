@@ -310,9 +310,11 @@ __global__ __launch_bounds__(256) void prep_labels_kernel(PrepArgs a) {
   }
 }
 
-// s > 1: the count tiles of 256 cells (four blocks), four threads per cell,
-// each taking every fourth target row of the cell's s x s block (S = s for the
-// unrolled forms 2 and 4, else 0).  grid (nblk, B)
+// s > 1: the count tiles of 256 cells (four blocks), four threads per cell
+// (two for s = 2, where the others would idle: 8 maps of 1024 x 1024 with 2
+// rows about 35 -> 15 us), each taking every
+// fourth target row of the cell's s x s block (S = s for the unrolled forms 2
+// and 4, else 0).  grid (nblk, B)
 //
 // Bound by reading the labels (8 s^2 bytes per cell).  The counts of a block
 // are built in LDS (rc rows of 256 cells at a time; every row at once for up
@@ -324,8 +326,10 @@ __global__ __launch_bounds__(256) void prep_labels_kernel(PrepArgs a) {
 // runs at 5.15), against 6.7 + 24.5 us for clearing the counts and adding to
 // them in memory pixel by pixel.
 constexpr size_t kCntLds = 40 * 1024;  // of the rows in LDS: three workgroups per CU
+template <int S>
+constexpr int kCellThreads = S == 2 ? 2 : 4;
 template <int CW, int S>
-__global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, int rc, int vec) {
+__global__ __launch_bounds__(kCellThreads<S> * kCntCells) void prep_counts_kernel(PrepArgs a, int rc, int vec) {
   __shared__ uint32_t pres[kPresWords];
   extern __shared__ __align__(16) unsigned char tile[];  // [4 blocks][rc][64] of CW bytes
   const int64_t b = blockIdx.y;
@@ -336,11 +340,12 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
   const int64_t HW = a.H * a.W;
   const bool mark = a.pbits != nullptr;
   if (mark) pres_clear(pres);
-  const int tid = threadIdx.x, cl = tid >> 2;
+  constexpr int T = kCellThreads<S>, threads = T * kCntCells;
+  const int tid = threadIdx.x, cl = tid / T;
   auto clear = [&]() {
-    for (int i = tid; i < rc * (kCntCells * CW / 16); i += kCntThreads) ((uint4*)tile)[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = tid; i < rc * (kCntCells * CW / 16); i += threads) ((uint4*)tile)[i] = make_uint4(0u, 0u, 0u, 0u);
   };
-  CellLabels<S> px;
+  CellLabels<S, T> px;
   px.load(a.targets, b, a.Ht, a.Wt, a.W, HW, a.s, (int64_t)blockIdx.x * kCntCells + cl, vec != 0);
   clear();  // while the labels are on their way
   px.settle();
@@ -368,7 +373,7 @@ __global__ __launch_bounds__(kCntThreads) void prep_counts_kernel(PrepArgs a, in
     const uint32_t words = per * (uint32_t)min((int64_t)(kCntCells / kCountCells), a.counts.nb - blk0);
     uint4* dst = (uint4*)(out0 + ((b * a.counts.nb + blk0) * a.counts.rows + r0) * kCountCells * CW);
     const uint32_t skip = (uint32_t)(a.counts.rows - nr) * (kCountCells * CW / 16);  // the other rows of a block
-    for (uint32_t i = tid; i < words; i += kCntThreads) dst[i + (skip ? i / per * skip : 0u)] = ((const uint4*)tile)[i];
+    for (uint32_t i = tid; i < words; i += threads) dst[i + (skip ? i / per * skip : 0u)] = ((const uint4*)tile)[i];
     __syncthreads();
   }
   if (mark) pres_store(a, pres, b);
@@ -408,10 +413,10 @@ int launch_prep(const PrepArgs& a, const Dims& d, hipStream_t st) {
     // pairs of labels by one 16-byte load: even s keeps every row 16-byte aligned
     const int vec = ((uintptr_t)a.targets & 15) == 0 ? 1 : 0;
     const int S = d.s == 4 ? 4 : d.s == 2 ? 2 : 0;
-    if (d.cw == 2) hipLaunchKernelGGL((prep_counts_kernel<2, 0>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
-    else if (S == 4) hipLaunchKernelGGL((prep_counts_kernel<1, 4>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
-    else if (S == 2) hipLaunchKernelGGL((prep_counts_kernel<1, 2>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
-    else hipLaunchKernelGGL((prep_counts_kernel<1, 0>), grid, dim3(kCntThreads), lds, st, a, rows, vec);
+    if (d.cw == 2) hipLaunchKernelGGL((prep_counts_kernel<2, 0>), grid, dim3(kCellThreads<0> * kCntCells), lds, st, a, rows, vec);
+    else if (S == 4) hipLaunchKernelGGL((prep_counts_kernel<1, 4>), grid, dim3(kCellThreads<4> * kCntCells), lds, st, a, rows, vec);
+    else if (S == 2) hipLaunchKernelGGL((prep_counts_kernel<1, 2>), grid, dim3(kCellThreads<2> * kCntCells), lds, st, a, rows, vec);
+    else hipLaunchKernelGGL((prep_counts_kernel<1, 0>), grid, dim3(kCellThreads<0> * kCntCells), lds, st, a, rows, vec);
   }
   if ((rc = check_launch("prep"))) return rc;
   if (a.pbits) {

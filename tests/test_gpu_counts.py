@@ -130,8 +130,8 @@ def test_dense(ml, shape):
                                    (4, 16, 16, 161, False), (15, 5, 13, 330, False), (15, 4, 4, 3, True)],
                          ids=lambda v: "s%d_%dx%d_C%d_%d" % v)
 def test_dense_groups(ml, shape, dtype):
-    """The kernels that count for themselves: class groups of 1, 16 and 17
-    rows, two groups by LDS (161), the counts in memory (330 classes at s = 15)."""
+    """The kernels that count for themselves: 16 and 17 classes, two groups by
+    LDS (161); the counts in memory below 16 classes and for 330 at s = 15."""
     s, H, W, C, shifted = shape
     rng = np.random.default_rng(s * H + C)
     L, B = 2, 2
