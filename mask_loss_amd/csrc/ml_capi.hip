@@ -411,8 +411,10 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   const SavedLayout SL = saved_layout(d);
   unsigned char* sv = (unsigned char*)saved;
   float* stats = saved ? (float*)(sv + SL.stats) : nullptr;
-  const bool tab = mask_dtype == ML_BF16 && g_use_lut && !force_masks;
-  CostPlan plan = make_cost_plan(d, mask_dtype, tab);
+  const ElemParams mask_ep = make_elem_params(p->mask_gamma, p->mask_alpha,
+                                              p->uncertainty_gamma, p->uncertainty_gamma_min);
+  const CostForm form = cost_form(d, mask_dtype, mask_ep, force_masks);
+  CostPlan plan = make_cost_plan(d, mask_dtype, form);
   if (packed) fit_cost_plan(plan, d, force_masks, ws_bytes / 2);
   const Layout L = packed ? make_layout(d, force_masks, plan) : make_layout(d, force_masks);
   // point-sampling front end: presence records of the full label map after the layout
@@ -483,8 +485,6 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   if (void_ready && hipEventRecord(void_ready, st) != hipSuccess)
     return fail(ML_ELAUNCH, "cannot record the void-check event");
 
-  const ElemParams mask_ep = make_elem_params(p->mask_gamma, p->mask_alpha,
-                                              p->uncertainty_gamma, p->uncertainty_gamma_min);
   CostArgs ca;
   ca.logits = mask_logits;
   ca.lab16 = pa.lab16;
@@ -498,7 +498,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   ca.L = d.L; ca.B = d.B; ca.Q = d.Q; ca.HW = d.HW; ca.HWp = d.HWp;
   ca.rtiles = d.rtiles; ca.GT_total = d.GT_total; ca.bg = d.bg; ca.rows = d.rows;
   ca.nslot = d.nslot; ca.N2 = (float)d.N2; ca.ep = mask_ep;
-  ca.use_lut = g_use_lut;
+  ca.form = form;
   // Two image subsets when the widest class (more than 111 non-empty GTs:
   // the longest solver chains) is the first and the polled counts show
   // another non-empty class: the widest class's finalize runs right after
@@ -512,7 +512,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
   SideStream side;
   if (d.LB > 0 && d.rtiles > 0) {
     if (!poll_classes) {
-      if ((rc = launch_cost(ca, d, mask_dtype, force_masks, st))) return rc;
+      if ((rc = launch_cost(ca, d, mask_dtype, st))) return rc;
     } else {
       // one class first, unconditionally: class 0 when the shape allows two
       // classes, else the widest; while it runs, the column pass's counts
@@ -521,7 +521,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
       // before the first class would leave the GPU idle instead)
       ProfScope ps_("pair_cost", st);
       const int first = plan.nclass > 2 ? plan.nclass - 1 : 0;
-      if ((rc = launch_cost(ca, d, mask_dtype, force_masks, st, 1u << first, false))) return rc;
+      if ((rc = launch_cost(ca, d, mask_dtype, st, 1u << first, false))) return rc;
       int32_t n[kClasses];
       if ((rc = wait_class_counts(cc_host, plan.nclass, first, st, n))) return rc;
       unsigned rest = 0;
@@ -532,7 +532,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
       if (rest && !costs_only && first == kClasses - 1 && cc_host[first] > 0) {
         phase_first = first;
         rest_classes = rest;  // launched after the first class's finalize
-      } else if (rest && (rc = launch_cost(ca, d, mask_dtype, force_masks, st, rest, false))) {
+      } else if (rest && (rc = launch_cost(ca, d, mask_dtype, st, rest, false))) {
         return rc;
       }
     }
@@ -645,7 +645,7 @@ int forward_impl(const ml_shape* s, const ml_params* p, int mask_dtype,
     if (!rc1) rc1 = launch_assign(a1, d, side.s, "assign_early");
     {
       ProfScope ps_("cost_rest", st);
-      rc2 = launch_cost(ca, d, mask_dtype, force_masks, st, rest_classes, false);
+      rc2 = launch_cost(ca, d, mask_dtype, st, rest_classes, false);
     }
     if (!rc2) rc2 = launch_finalize(a2, d, st);
     if (!rc2) rc2 = launch_assign(a2, d, st);
@@ -685,8 +685,9 @@ int forward_packed_bytes(const ml_shape* s, const ml_params* p, int mask_dtype, 
   if (!make_dims(s, p->background_index, mask_dtype, d, err)) return fail(ML_EINVAL, err);
   if (!check_assign_dims(d, err)) return fail(ML_EUNSUPPORTED, err);
   const bool force_masks = p->force_unmatched_masks_to_empty != 0;
-  const bool tab = mask_dtype == ML_BF16 && g_use_lut && !force_masks;
-  CostPlan plan = make_cost_plan(d, mask_dtype, tab);
+  const ElemParams ep = make_elem_params(p->mask_gamma, p->mask_alpha, p->uncertainty_gamma,
+                                         p->uncertainty_gamma_min);
+  CostPlan plan = make_cost_plan(d, mask_dtype, cost_form(d, mask_dtype, ep, force_masks));
   fit_cost_plan(plan, d, force_masks, budget / 2);
   bytes = make_layout(d, force_masks, plan).total;
   return ML_OK;

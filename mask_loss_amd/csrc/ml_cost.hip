@@ -15,27 +15,35 @@
 // slots: their right operands are zero outside the tiles that a K-step's cells
 // touch, so those tiles' MFMAs are skipped.
 //
-// Operands are float16.  The planes are scaled by 2^9, split into two float16
-// terms for float32 and float16 logits (22 bits) and one for bf16 ones (11
-// bits).  The right operand is made of 16-bit integer ops: label codes of two
-// labels differ by at least 0x100 under xor, so a saturating subtraction of the
-// xor from 0x100 gives 0x100 (as a float16: 2^-16) where they agree and 0 elsewhere;
-// times 0x3C it is 1.0, which the two-term operands take (the matrix cores align a
-// subnormal factor's product without normalising it: with 2^-24, ten places
-// down, float32 sums were 1e-5 off; 2^-16 costs two places of a bf16 logit's
-// plane).  A u8 count n becomes 0x6400 + n = 1024 + n by one byte permute, then n.
-// The sums leave with all scales undone (powers of two).  A plane above
-// 127 (|z| > 127, or > 2558 at the smallest weight), inf or nan makes the wave's
-// sums non-finite; such a wave redoes its K-range with bf16 operands (3, 2 or 1
-// terms), which hold any float32.
+// Operands are float16 where that loses nothing, else bf16.  A float16 plane is
+// scaled by 2^lg (cost_form: the largest scale that keeps it finite) and split into
+// two terms for float32 and float16 logits (22 bits), one for bf16 ones (11
+// bits).  Below 2^-14 a scaled plane has absolute steps of 2^-24 instead: a plane is
+// then up to 2^-25-lg off, 2e-12 at the operator's default weights and 3e-11 without
+// weights.  The formulas are 6e-8 w off there themselves (1 + e^-|z| rounded to
+// float32), but only as long as no factor makes the planes small: where a focal
+// power does, or an uncertainty weight with a floor below 2^-6 (CostForm::wide), and
+// where a range holds |z| > 60, the operands are bf16 terms (3, 2 or 1), which
+// keep 24, 16 or 8 bits of any float32.
 //
-// Bounds and measurements (MI355X; before: bf16 operands, 3 terms for float32
-// and 2 for float16, counts evaluated by formula from planes of u8 counts).  The
-// float32 kernels are bound by vector-ALU issue (~25 ops and 3 transcendental per
-// logit, a third of them the split): 10 M logits in 32 columns 28.1 -> 21.8 us, 33.6 M
-// against 4x targets 96 -> 58.6 us, the 16- and 7-tile launches of 39 M logits
-// 113 + 49 -> 88 + 39 us.  float32 sums are as far from 64 bits as before (4e-8 to
-// 1e-7), float16 and bf16 ones 3 to 10 times closer.
+// The right operand is made of 16-bit integer ops: label codes of two
+// labels differ by at least 0x100 under xor, so a saturating subtraction of the
+// xor from 0x100 gives 0x100 (as a float16: 2^-16) where they agree and 0
+// elsewhere; times a constant it is 2^-lg or a bf16 one.  The table kernels take
+// the 2^-16 itself (the matrix cores align a subnormal factor's product without
+// normalising it: that costs two of the plane's 11 bits).  A u8 count n under a
+// float16 exponent whose last place is 2^-lg becomes 2^(10-lg) + 2^-lg n by one byte
+// permute, then 2^-lg n.  Scales are powers of two, so no result depends on them
+// but for the steps above.
+//
+// The kernels by formula are bound by vector-ALU issue (~25 ops and 3 transcendental
+// per logit, a third of them the split), the widest class by latency at one wave per
+// SIMD.  Float32 logits, bf16 operands throughout / float16 where they fit: 10 M in 32
+// columns 28.1 / 22.2 us (focal gamma 2, bf16 operands by its rule: 29.8), 33.6 M
+// against 4x targets 96 / 59, the 16- and 7-tile launches of 39 M 113 + 49 / 97 +
+// 40.  A range that is redone costs its formula pass again: 40% of 10 M logits
+// filled with -10^4, whole cost call 40.3 / 41.7 us (bf16 logits, in the table's
+// kernels: 54 / 56, against 4x targets 50 / 60).
 //
 // Work decomposition: one wave = 16 query rows of one image over a
 // contiguous range of 32-cell K-steps; each image is handled by the kernel
@@ -63,22 +71,20 @@ typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u16x2_t as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2_t, v); }
 __device__ __forceinline__ uint32_t as_u32(u16x2_t v) { return __builtin_bit_cast(uint32_t, v); }
 
-constexpr float kPlaneScale = 512.f;  // of the float16 planes
-
-// terms per plane: float16 operands, and the bf16 operands of a redone range
+// terms per plane: float16 operands, and bf16 ones
 template <int DT>
 struct InTraits;
 template <>
 struct InTraits<ML_F32> {
-  static constexpr int kTerms = 2, kRedo = 3;
+  static constexpr int kTerms = 2, kWide = 3;
 };
 template <>
 struct InTraits<ML_BF16> {
-  static constexpr int kTerms = 1, kRedo = 1;
+  static constexpr int kTerms = 1, kWide = 1;
 };
 template <>
 struct InTraits<ML_F16> {
-  static constexpr int kTerms = 2, kRedo = 2;
+  static constexpr int kTerms = 2, kWide = 2;
 };
 
 // ---- LUT geometry (bytes): positive block at 0, negative block at 32768 ----
@@ -89,6 +95,7 @@ constexpr uint32_t kLutSub = kLutBase - 1;       // idx = sat(m - kLutSub): 0 = 
 constexpr uint32_t kLutBlock = kLutN + 2;        // tiny + regular + overflow slot
 constexpr uint32_t kLutNegOff = 32768;
 constexpr uint32_t kLutBytes = kLutNegOff + kLutBlock * 8;
+constexpr float kNarrowMax = 60.f;               // of |z|: float16 operands by formula (see the top)
 constexpr int kDepth = 4;  // K-steps of logits in flight per wave
 
 __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
@@ -108,78 +115,93 @@ __device__ __forceinline__ float rem_hi(float v, uint32_t w) {
 }
 
 // ---- planes of one logit ---------------------------------------------------
-// The four planes from the float32 formulas, unscaled, and the unweighted terms
-// of the unmatched-mask penalty.
-__device__ __forceinline__ void planes_formula(float z, const ElemParams& ep, float& neg, float& pos,
-                                               float& wp, float& w, float& negu, float& pu) {
-  const Sig s = sig_terms(z);
-  w = unc_weight(s, ep);
-  float mn, mp;
-  focal_mods(s, ep, mn, mp);
-  negu = ep.an * mn * s.cn;
-  pu = s.p;
-  neg = w * negu;
-  pos = w * (ep.ap * mp * s.cp);
-  wp = w * s.p;
-}
-
 // Which of the per-logit forms a call takes (chosen once per 8 logits, wave-uniform):
 // 0 general; 1 no focal terms, weight H^1 (the operator's defaults); 2 no
 // focal terms, no weights; 3 focal gamma 2 with or without weights H^1.
 __device__ __forceinline__ int elem_mode(const ElemParams& ep) {
   const bool plain = ep.gamma_mode == 0 && ep.an == 1.f && ep.ap == 1.f;
   if (plain && ep.ug_mode == 1) return 1;
-  if (plain && ep.ug_mode == 0 && ep.ug_min <= 1.f) return 2;
+  if (plain && ep.ug_mode == 0) return 2;
   if (ep.gamma_mode == 2 && ep.ug_mode != 2) return 3;
   return 0;
 }
 
-// The planes scaled by kPlaneScale.  With t = -|z| log2 e, e = 2^t, d = 1 + e:
+// The planes of logit z scaled by sc (ug_sc: the scaled weight floor) and the
+// unweighted terms of the unmatched-mask penalty.  With t = -|z| log2 e, e = 2^t, d = 1 + e:
 // the entropy -(p ln p + q ln q) / ln 2 is log2 d + (e / d) |t| (both terms
 // non-negative) and softplus(+-z) = ln 2 log2 d + max(+-z, 0), so the default
 // form takes 3 transcendental and 15 other ops per logit.
 template <int EM>
-__device__ __forceinline__ void planes_scaled(float z, const ElemParams& ep, float& neg, float& pos, float& wp,
-                                              float& w, float& negu, float& pu) {
+__device__ __forceinline__ void planes_of(float z, const ElemParams& ep, float sc, float ug_sc, float& neg,
+                                          float& pos, float& wp, float& w, float& negu, float& pu) {
   if constexpr (EM == 0) {
-    planes_formula(z, ep, neg, pos, wp, w, negu, pu);
-    neg *= kPlaneScale;
-    pos *= kPlaneScale;
-    wp *= kPlaneScale;
-    w *= kPlaneScale;
-    return;
-  }
-  const float t = -fabsf(z) * kLog2e;
-  const float e = __builtin_amdgcn_exp2f(t);
-  const float d = 1.f + e;
-  const float r = __builtin_amdgcn_rcpf(d);
-  const float l2 = __builtin_amdgcn_logf(d);  // log2
-  const float er = e * r;
-  const bool up = z >= 0.f;
-  const float p = up ? r : er;
-  float cn = __builtin_fmaf(l2, kLn2, fmaxf(z, 0.f)), cp = __builtin_fmaf(l2, kLn2, fmaxf(-z, 0.f));
-  if constexpr (EM == 3) {
-    const float q = up ? er : r;
-    cn *= ep.an * (p * p);
-    cp *= ep.ap * (q * q);
-  }
-  if (EM == 1 || (EM == 3 && ep.ug_mode == 1)) {
-    const float h = __builtin_fmaf(-er, t, l2);
-    w = __builtin_amdgcn_fmed3f(h * kPlaneScale, ep.ug_min * kPlaneScale, kPlaneScale);
+    const Sig s = sig_terms(z);
+    float mn, mp;
+    focal_mods(s, ep, mn, mp);
+    w = unc_weight(s, ep) * sc;
+    negu = ep.an * mn * s.cn;
+    pu = s.p;
+    pos = w * (ep.ap * mp * s.cp);
   } else {
-    w = kPlaneScale;
+    const float t = -fabsf(z) * kLog2e;
+    const float e = __builtin_amdgcn_exp2f(t);
+    const float d = 1.f + e;
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float l2 = __builtin_amdgcn_logf(d);  // log2
+    const float er = e * r;
+    const bool up = z >= 0.f;
+    const float p = up ? r : er;
+    float cn = __builtin_fmaf(l2, kLn2, fmaxf(z, 0.f)), cp = __builtin_fmaf(l2, kLn2, fmaxf(-z, 0.f));
+    if constexpr (EM == 3) {
+      const float q = up ? er : r;
+      cn *= ep.an * (p * p);
+      cp *= ep.ap * (q * q);
+    }
+    if (EM == 1 || (EM == 3 && ep.ug_mode == 1)) {
+      // (|z| beyond 2^127 / 1.44: 0 x inf here, and a NaN leaves the floor)
+      const float h = __builtin_fmaf(-er, t, l2);
+      w = __builtin_amdgcn_fmed3f(h * sc, ug_sc, sc);
+    } else {
+      w = sc;
+    }
+    negu = cn;
+    pu = p;
+    pos = w * cp;
   }
-  negu = cn;
-  pu = p;
-  neg = w * cn;
-  pos = w * cp;
-  wp = w * p;
+  neg = w * negu;
+  wp = w * pu;
 }
 
-// Build the LUT in LDS (all threads of the workgroup).  The overflow slot
-// holds NaN so that a wave whose sums come out NaN knows it met |z| >= 64,
-// inf or nan (finite table entries stay below 2^15 and cannot produce NaN).
-__device__ void build_lut(unsigned char* lut, const ElemParams& ep) {
+// Operand types of the matrix instructions: float16, or bf16 (WIDE).
+template <bool WIDE>
+struct Ops {
+  using v8 = f16x8_t;
+  static __device__ __forceinline__ uint32_t pack(float a, float b) { return pack_f16x2(a, b); }
+  static __device__ __forceinline__ f32x4_t mma16(v8 a, v8 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x16_t mma32(v8 a, v8 b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Ops<true> {
+  using v8 = bf16x8_t;
+  static __device__ __forceinline__ uint32_t pack(float a, float b) { return pack_bf16x2(a, b); }
+  static __device__ __forceinline__ f32x4_t mma16(v8 a, v8 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x16_t mma32(v8 a, v8 b, f32x16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+};
+
+// Build the LUT in LDS (all threads of the workgroup): float16 planes scaled by
+// 2^lg, or bf16 planes (WIDE).  The overflow slot holds NaN so that a wave whose
+// sums come out NaN knows it met |z| >= 64, inf or nan (every other entry is finite).
+template <bool WIDE>
+__device__ void build_lut(unsigned char* lut, const ElemParams& ep, int lg) {
+  const float sc = WIDE ? 1.f : __builtin_ldexpf(1.f, lg);
   for (uint32_t e = threadIdx.x; e < 2 * kLutBlock; e += blockDim.x) {
     const uint32_t sgn = e >= kLutBlock ? 1u : 0u;
     const uint32_t j = e - sgn * kLutBlock;
@@ -188,12 +210,12 @@ __device__ void build_lut(unsigned char* lut, const ElemParams& ep) {
       const uint32_t mag = j == 0 ? 0u : kLutSub + j;  // j == 0: |z| < 2^-9 -> z = 0
       const float z = __uint_as_float(((sgn << 15) | mag) << 16);
       float neg, pos, wp, w, nu, pu;
-      planes_scaled<0>(z, ep, neg, pos, wp, w, nu, pu);
-      v.x = pack_f16x2(neg, pos);
-      v.y = pack_f16x2(wp, w);
+      planes_of<0>(z, ep, sc, 0.f, neg, pos, wp, w, nu, pu);
+      v.x = Ops<WIDE>::pack(neg, pos);
+      v.y = Ops<WIDE>::pack(wp, w);
     } else {
-      v.x = 0x7E007E00u;  // NaN marker
-      v.y = 0x7E007E00u;
+      v.x = WIDE ? 0x7FC07FC0u : 0x7E007E00u;  // NaN marker
+      v.y = v.x;
     }
     *(uint2*)(lut + sgn * kLutNegOff + j * 8) = v;
   }
@@ -266,7 +288,7 @@ __device__ __forceinline__ void split_f16(const float v[8], f16x8_t out[NT]) {
     out[1] = __builtin_bit_cast(f16x8_t, lo);
   }
 }
-// ... and as NS bf16 terms (redone ranges).
+// ... and as NS bf16 terms.
 template <int NS>
 __device__ __forceinline__ void split_bf16(const float v[8], bf16x8_t out[NS]) {
   float rem[8];
@@ -288,19 +310,17 @@ __device__ __forceinline__ void split_bf16(const float v[8], bf16x8_t out[NS]) {
   }
 }
 
-// A planes of one row's 8 cells by formula, float16 terms; with MASK, cells >=
-// nvalid are zero.  ub, up: sums of the unweighted terms (unw).
-template <int DT, int NT, bool MASK>
-__device__ __forceinline__ void planes8_formula(const Raw8<DT>& r, const ElemParams& ep, int64_t nvalid, bool unw,
-                                                f16x8_t A[4][NT], float& ub, float& up) {
-  float z[8];
-  raw_to_f32<DT>(r, z);
-  float v[4][8];
+// The planes of one row's 8 cells, scaled by sc; with MASK, cells >= nvalid are
+// zero.  ub, up: sums of the unweighted terms (unw).
+template <bool MASK>
+__device__ __forceinline__ void planes8(const float (&z)[8], const ElemParams& ep, float sc,
+                                        int64_t nvalid, bool unw, float (&v)[4][8], float& ub, float& up) {
+  const float ug_sc = ep.ug_min * sc;
   auto cells = [&](auto em) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       float neg, pos, wp, w, nu, pu;
-      planes_scaled<decltype(em)::value>(z[k], ep, neg, pos, wp, w, nu, pu);
+      planes_of<decltype(em)::value>(z[k], ep, sc, ug_sc, neg, pos, wp, w, nu, pu);
       const bool ok = !MASK || k < nvalid;
       v[0][k] = ok ? neg : 0.f;
       v[1][k] = ok ? pos : 0.f;
@@ -318,28 +338,17 @@ __device__ __forceinline__ void planes8_formula(const Raw8<DT>& r, const ElemPar
     case 3: cells(std::integral_constant<int, 3>()); break;
     default: cells(std::integral_constant<int, 0>()); break;
   }
-#pragma unroll
-  for (int pl = 0; pl < 4; ++pl) split_f16<NT>(v[pl], A[pl]);
 }
-// The same as unscaled bf16 terms, for a redone range.
-template <int DT>
-__device__ __forceinline__ void planes8_redo(const Raw8<DT>& r, const ElemParams& ep, int64_t nvalid,
-                                             bf16x8_t A[4][InTraits<DT>::kRedo]) {
-  float z[8];
-  raw_to_f32<DT>(r, z);
-  float v[4][8];
+// max(|a|, |b|, |c|), NaNs aside (written out: the compiler would quiet each operand first)
+__device__ __forceinline__ float max_abs3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float max_abs8(const float (&z)[8], float m) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    float neg, pos, wp, w, nu, pu;
-    planes_formula(z[k], ep, neg, pos, wp, w, nu, pu);
-    const bool ok = k < nvalid;
-    v[0][k] = ok ? neg : 0.f;
-    v[1][k] = ok ? pos : 0.f;
-    v[2][k] = ok ? wp : 0.f;
-    v[3][k] = ok ? w : 0.f;
-  }
-#pragma unroll
-  for (int pl = 0; pl < 4; ++pl) split_bf16<InTraits<DT>::kRedo>(v[pl], A[pl]);
+  for (int k = 0; k < 8; k += 2) m = max_abs3(z[k], z[k + 1], m);
+  return m;
 }
 
 // Table byte offsets (sign block included) of the two bf16 logits packed in
@@ -357,6 +366,14 @@ __device__ __forceinline__ uint32_t lut_addr_pair(uint32_t u) {
   return addr;
 }
 
+// Any of 8 bf16 logits beyond the table (|z| >= 64, inf, nan).
+__device__ __forceinline__ bool lut_over8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  const u16x2_t m = __builtin_elementwise_max(
+      __builtin_elementwise_max(as_u16x2(a & 0x7FFF7FFFu), as_u16x2(b & 0x7FFF7FFFu)),
+      __builtin_elementwise_max(as_u16x2(c & 0x7FFF7FFFu), as_u16x2(d & 0x7FFF7FFFu)));
+  return m[0] >= kLutOver || m[1] >= kLutOver;
+}
+
 // Table entries of one row's 8 bf16 cells (LDS reads only; see lut_planes).
 __device__ __forceinline__ void lut_lookup8(const uint4& x, const unsigned char* lut, uint2 E[8]) {
   const uint32_t u[4] = {x.x, x.y, x.z, x.w};
@@ -370,20 +387,19 @@ __device__ __forceinline__ void lut_lookup8(const uint4& x, const unsigned char*
 
 // The four A planes from the entries of 8 cells: (neg, pos) and (wp, w) of
 // each cell regrouped into per-plane pairs of consecutive cells.
-__device__ __forceinline__ void lut_planes(const uint2 E[8], f16x8_t A[4]) {
-  u32x4_t a0, a1, a2, a3;
+template <class V>
+__device__ __forceinline__ void lut_planes(const uint2 E[8], V A[4]) {
+  u32x4_t a[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint2 e0 = E[2 * i], e1 = E[2 * i + 1];
-    a0[i] = __builtin_amdgcn_perm(e1.x, e0.x, 0x05040100u);
-    a1[i] = __builtin_amdgcn_perm(e1.x, e0.x, 0x07060302u);
-    a2[i] = __builtin_amdgcn_perm(e1.y, e0.y, 0x05040100u);
-    a3[i] = __builtin_amdgcn_perm(e1.y, e0.y, 0x07060302u);
+    a[0][i] = __builtin_amdgcn_perm(e1.x, e0.x, 0x05040100u);
+    a[1][i] = __builtin_amdgcn_perm(e1.x, e0.x, 0x07060302u);
+    a[2][i] = __builtin_amdgcn_perm(e1.y, e0.y, 0x05040100u);
+    a[3][i] = __builtin_amdgcn_perm(e1.y, e0.y, 0x07060302u);
   }
-  A[0] = __builtin_bit_cast(f16x8_t, a0);
-  A[1] = __builtin_bit_cast(f16x8_t, a1);
-  A[2] = __builtin_bit_cast(f16x8_t, a2);
-  A[3] = __builtin_bit_cast(f16x8_t, a3);
+#pragma unroll
+  for (int pl = 0; pl < 4; ++pl) A[pl] = __builtin_bit_cast(V, a[pl]);
 }
 
 // ---- right operands ---------------------------------------------------------
@@ -412,16 +428,14 @@ __device__ __forceinline__ u32x4_t imul8(const u32x4_t& n, unsigned short c) {
   for (int i = 0; i < 4; ++i) b[i] = as_u32(as_u16x2(n[i]) * (u16x2_t){c, c});
   return b;
 }
-// 8 u8 counts with `hi` as every high byte: 0 for integers, 0x64 for 1024 + n in float16.
-template <uint32_t HI>
-__device__ __forceinline__ u32x4_t widen8(uint32_t x, uint32_t y) {
-  constexpr uint32_t h = HI * 0x01010101u;
-  constexpr uint32_t s0 = HI ? 0x04010400u : 0x0C010C00u, s1 = HI ? 0x04030402u : 0x0C030C02u;
-  return u32x4_t{__builtin_amdgcn_perm(h, x, s0), __builtin_amdgcn_perm(h, x, s1), __builtin_amdgcn_perm(h, y, s0),
-                 __builtin_amdgcn_perm(h, y, s1)};
+// 8 u8 counts as 16-bit words with a byte of hi4 above each.
+__device__ __forceinline__ u32x4_t widen8(uint32_t hi4, uint32_t x, uint32_t y) {
+  constexpr uint32_t s0 = 0x04010400u, s1 = 0x04030402u;
+  return u32x4_t{__builtin_amdgcn_perm(hi4, x, s0), __builtin_amdgcn_perm(hi4, x, s1),
+                 __builtin_amdgcn_perm(hi4, y, s0), __builtin_amdgcn_perm(hi4, y, s1)};
 }
-// c + t and c - t for 8 float16 values, two per op (exact here: integers below
-// 2048); c: the value twice.
+// c + t and c - t for 8 float16 values, two per op (exact here: both are multiples
+// of the same last place below 2^11 of them); c: the value twice.
 template <bool NEG>
 __device__ __forceinline__ u32x4_t hadd8(uint32_t c, const u32x4_t& t) {
   u32x4_t b;
@@ -432,46 +446,77 @@ __device__ __forceinline__ u32x4_t hadd8(uint32_t c, const u32x4_t& t) {
   }
   return b;
 }
-// The operands n and N2 - n of one column tile.
+// Operands n and N2 - n of one column tile.
 struct Opnd {
-  f16x8_t n, rest;
+  u32x4_t n, rest;
 };
-// u8 counts; top: 1024 + N2 as a float16 pair (wave-uniform).
+// float16 counts times 2^-lg (lg <= 14, N2 < 1024): wave-uniform constants.
+struct RightF16 {
+  uint32_t mul, one2;       // label compare: the factor of kHot, and the result twice
+  uint32_t hi4, base, top;  // u8: bytes above a count, minus their value, their value + 2^-lg N2 (pairs)
+  float inv;                // 2^-lg
+};
+__device__ __forceinline__ RightF16 right_f16(int lg, float N2) {
+  const uint32_t one = (uint32_t)(15 - lg) << 10, e = (uint32_t)(25 - lg) << 10;
+  return RightF16{one / kHot, one * 0x10001u, (e >> 8) * 0x01010101u, (e | 0x8000u) * 0x10001u,
+                  (e + (uint32_t)N2) * 0x10001u, __builtin_ldexpf(1.f, -lg)};
+}
 template <bool REST>
-__device__ __forceinline__ Opnd opnd_u8(uint32_t x, uint32_t y, uint32_t top) {
-  const u32x4_t t = widen8<0x64>(x, y);  // 1024 + n
+__device__ __forceinline__ Opnd opnd_u8(uint32_t x, uint32_t y, const RightF16& c) {
+  const u32x4_t t = widen8(c.hi4, x, y);
   Opnd o;
-  o.n = __builtin_bit_cast(f16x8_t, hadd8<false>(0xE400E400u, t));  // -1024
-  if (REST) o.rest = __builtin_bit_cast(f16x8_t, hadd8<true>(top, t));
+  o.n = hadd8<false>(c.base, t);
+  if (REST) o.rest = hadd8<true>(c.top, t);
   return o;
 }
-__device__ __forceinline__ uint32_t opnd_top(float N2) { return (0x6400u + (uint32_t)N2) * 0x10001u; }
-// Label compare: ONE is the value of a hit, kHot (2^-16) or 0x3C00 (1.0).
-template <uint32_t ONE, bool REST>
-__device__ __forceinline__ Opnd opnd_hot(const u32x4_t& hot) {
-  const u32x4_t v = ONE == kHot ? hot : imul8(hot, (unsigned short)(ONE / kHot));
+// Label compare: `mul` times kHot is the value of a hit, one2 that value twice.
+template <bool REST>
+__device__ __forceinline__ Opnd opnd_hot(const u32x4_t& hot, uint32_t mul, uint32_t one2) {
   Opnd o;
-  o.n = __builtin_bit_cast(f16x8_t, v);
-  if (REST) o.rest = __builtin_bit_cast(f16x8_t, isub8(ONE * 0x10001u, v));
+  o.n = mul == 1u ? hot : imul8(hot, (unsigned short)mul);
+  if (REST) o.rest = isub8(one2, o.n);
   return o;
 }
-// Bits 0..10 (HIGH = 0) or 11..15 of 8 16-bit integers as float16.
+// ... as the table kernels take it: 2^-16, or a bf16 0.5 (WIDE).
+template <bool WIDE>
+__device__ __forceinline__ Opnd opnd_tab(const u32x4_t& hot) {
+  return WIDE ? opnd_hot<true>(hot, 0x3Fu, 0x3F003F00u) : opnd_hot<true>(hot, 1u, kHot * 0x10001u);
+}
+// Bits 0..10 (HIGH = 0) or 11..15 of 8 16-bit integers as float16, times inv.
 template <bool HIGH>
-__device__ __forceinline__ f16x8_t part8(const u32x4_t& w) {
+__device__ __forceinline__ u32x4_t part8(const u32x4_t& w, float inv) {
   constexpr uint32_t m = HIGH ? 0xF800u : 0x07FFu;
   u32x4_t b;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) b[i] = pack_f16x2((float)(w[i] & m), (float)((w[i] >> 16) & m));
-  return __builtin_bit_cast(f16x8_t, b);
+  for (int i = 0; i < 4; ++i) b[i] = pack_f16x2((float)(w[i] & m) * inv, (float)((w[i] >> 16) & m) * inv);
+  return b;
 }
-// bf16 operands of a redone range from 16-bit integers: the bits of `mask`,
-// shifted down.
-__device__ __forceinline__ bf16x8_t redo8(const u32x4_t& w, uint32_t mask, int shift = 0) {
+// bf16 operands: a label hit as 1.0; a u8 count; and one byte of 16-bit integers,
+// exact in 8 bits.
+__device__ __forceinline__ u32x4_t wide_hot8(const u32x4_t& hot) {
+  u32x4_t b = imul8(hot, 0x7Fu);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = as_u32(as_u16x2(b[i]) >> (u16x2_t){1, 1});
+  return b;
+}
+__device__ __forceinline__ Opnd wide_u8(uint32_t x, uint32_t y, float N2) {
+  Opnd o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w = i < 2 ? x : y;
+    const float a = (float)((w >> (16 * (i & 1))) & 0xFFu), b = (float)((w >> (16 * (i & 1) + 8)) & 0xFFu);
+    o.n[i] = pack_bf16x2(a, b);
+    o.rest[i] = pack_bf16x2(N2 - a, N2 - b);
+  }
+  return o;
+}
+template <bool HIGH>
+__device__ __forceinline__ u32x4_t wide_byte8(const u32x4_t& w) {
+  constexpr uint32_t m = HIGH ? 0xFF00u : 0xFFu;
   u32x4_t b;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    b[i] = pack_bf16x2((float)((w[i] & mask) >> shift), (float)(((w[i] >> 16) & mask) >> shift));
-  return __builtin_bit_cast(bf16x8_t, b);
+  for (int i = 0; i < 4; ++i) b[i] = pack_bf16x2((float)(w[i] & m), (float)((w[i] >> 16) & m));
+  return b;
 }
 
 // Pacing of the waves of one workgroup that share a CU: the SIMD arbiter
@@ -515,9 +560,9 @@ constexpr int kRedBarriers = 4;  // per level of the tree
 // One wave's work: 16 query rows of task (lb, rtile) over the K-steps of
 // split ks of KS; writes the partial sums to `out` ([NP][16][16*NT]) and,
 // for unweighted penalties, the row sums to `rs` ([16][2]).  TAB:
-// per-cell planes from the LDS table (bf16 only).  If the sums come out
-// non-finite (the table's marker, or a plane beyond float16), the wave redoes
-// the range with bf16 operands before writing.  `setup` (the
+// per-cell planes from the LDS table (bf16 only; WIDE: a table of bf16, label
+// maps only).  If a table wave's sums come out non-finite (the marker), it redoes
+// the range with the formulas and bf16 operands before writing.  `setup` (the
 // workgroup's table build and barrier) is called exactly once on every path,
 // after the first D K-steps of loads are issued, so their latency overlaps it.
 // With red.buf, the R waves of the group add their sums in a fixed tree order
@@ -526,19 +571,19 @@ constexpr int kRedBarriers = 4;  // per level of the tree
 // CNT: 0 label map, 1 u8 counts, 2 u16 counts.  In the wide classes (NT >= 7) a
 // K-step's MFMAs run only for the column tiles its 32 cells touch (a coherent
 // label map touches few of them).
-template <int DT, int NT, int CNT, bool TAB, class Setup>
+template <int DT, int NT, int CNT, bool TAB, bool WIDE, class Setup>
 __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t rtile, int64_t ks, int64_t KS,
                                           const unsigned char* lut, float* out, float* rs_out, int* prog,
                                           Setup&& setup, const SplitRed& red = SplitRed(),
                                           uint32_t* klut = nullptr) {
-  constexpr int NS = TAB ? 1 : InTraits<DT>::kTerms;
+  constexpr int NS = TAB ? 1 : InTraits<DT>::kTerms, NW = InTraits<DT>::kWide;
+  using V = typename Ops<TAB && WIDE>::v8;  // the table's or the float16 operands
   // label maps in the wide classes: the label -> (slot | tile bit << 16) table
   // klut (this wave's, in LDS) gives each K-step's slots and touched tiles
   constexpr bool KEYS = CNT == 0 && NT >= 7;
   constexpr bool SUMS = NT >= 7;  // slot sums
   constexpr int NP = class_planes(SUMS ? 1 : 0);
   constexpr int D = TAB ? kDepth : 2;  // K-steps of logits and labels in flight
-  constexpr uint32_t kOne = TAB ? kHot : 0x3C00u;  // a label hit's operand
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g4 = lane >> 4;
   const ElemParams ep = a.ep;
@@ -672,36 +717,61 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
     }
   };
   const uint32_t n2pair = (uint32_t)a.N2 * 0x10001u;
-  auto mma_step = [&](f16x8_t (&A)[4][NS], const BRaw& x, const uint32_t (&kp)[4], uint32_t tmask) {
+  // table sums carry the planes' scale, the others none
+  const RightF16 rf = right_f16(TAB ? 0 : a.form.lg, a.N2);
+  auto mul_tile = [&](auto ops, int nt, const auto& A, const Opnd& o) {
+    using O = decltype(ops);
+    constexpr int T = sizeof(A[0]) / sizeof(A[0][0]);
+    auto mul = [&](int i, int pl, const u32x4_t& v) {
+#pragma unroll
+      for (int sp = 0; sp < T; ++sp)
+        acc[i][nt] = O::mma16(A[pl][sp], __builtin_bit_cast(typename O::v8, v), acc[i][nt]);
+    };
+    if constexpr (SUMS) {
+#pragma unroll
+      for (int pl = 0; pl < 4; ++pl) mul(pl, pl, o.n);
+    } else {
+      mul(0, 0, o.rest);
+      mul(1, 2, o.n);
+      mul(2, 3, o.n);
+      mul(0, 1, o.n);
+    }
+  };
+  auto mma_step = [&](const V (&A)[4][NS], const BRaw& x, const uint32_t (&kp)[4], uint32_t tmask) {
     for_tiles(x, kp, tmask, [&](int nt, const u32x4_t& raw) {
-      auto mul = [&](int i, int pl, const f16x8_t& v) {
-#pragma unroll
-        for (int sp = 0; sp < NS; ++sp)
-          acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[pl][sp], v, acc[i][nt], 0, 0, 0);
-      };
-      auto mul_all = [&](const Opnd& o) {
-        if constexpr (SUMS) {
-#pragma unroll
-          for (int pl = 0; pl < 4; ++pl) mul(pl, pl, o.n);
-        } else {
-          mul(0, 0, o.rest);
-          mul(1, 2, o.n);
-          mul(2, 3, o.n);
-          mul(0, 1, o.n);
-        }
-      };
-      if constexpr (CNT == 0) {
-        mul_all(opnd_hot<kOne, !SUMS>(raw));
+      auto mul = [&](const Opnd& o) { mul_tile(Ops<TAB && WIDE>(), nt, A, o); };
+      if constexpr (CNT == 0 && TAB) {
+        mul(opnd_tab<WIDE>(raw));
+      } else if constexpr (CNT == 0) {
+        mul(opnd_hot<!SUMS>(raw, rf.mul, rf.one2));
       } else if constexpr (CNT == 1) {
-        mul_all(opnd_u8<!SUMS>(raw[0], raw[1], opnd_top(a.N2)));
+        mul(opnd_u8<!SUMS>(raw[0], raw[1], rf));
       } else {  // integers up to 65025 as two exact float16 parts
         const u32x4_t rest = isub8(n2pair, raw);
-        mul_all(Opnd{part8<false>(raw), part8<false>(rest)});
-        mul_all(Opnd{part8<true>(raw), part8<true>(rest)});
+        mul(Opnd{part8<false>(raw, rf.inv), part8<false>(rest, rf.inv)});
+        mul(Opnd{part8<true>(raw, rf.inv), part8<true>(rest, rf.inv)});
       }
     });
   };
-
+  // the same with bf16 operands from unscaled planes
+  auto mma_wide = [&](const float (&v)[4][8], const BRaw& x, const uint32_t (&kp)[4], uint32_t tmask) {
+    bf16x8_t A[4][NW];
+#pragma unroll
+    for (int pl = 0; pl < 4; ++pl) split_bf16<NW>(v[pl], A[pl]);
+    for_tiles(x, kp, tmask, [&](int nt, const u32x4_t& raw) {
+      auto mul = [&](const Opnd& o) { mul_tile(Ops<true>(), nt, A, o); };
+      if constexpr (CNT == 0) {
+        const u32x4_t n = wide_hot8(raw);
+        mul(Opnd{n, isub8(0x3F803F80u, n)});
+      } else if constexpr (CNT == 1) {
+        mul(wide_u8(raw[0], raw[1], a.N2));
+      } else {
+        const u32x4_t rest = isub8(n2pair, raw);
+        mul(Opnd{wide_byte8<false>(raw), wide_byte8<false>(rest)});
+        mul(Opnd{wide_byte8<true>(raw), wide_byte8<true>(rest)});
+      }
+    });
+  };
   // Software pipeline over this wave's nst steps: D steps of logits (and
   // labels) in flight, the count operands one step ahead.  Slot j holds step
   // k + j; it is turned into A operands first and then refilled with step
@@ -710,6 +780,10 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
   // step counters in 32 bits: their compares stay scalar (a wave has at most
   // HW / 32 < 2^31 steps)
   const int nst = (int)(s1 - s0);
+  // steps summed; the bf16 loop below takes the rest.  A range that opens with
+  // logits these operands do not take (a filled region) goes there whole, at once.
+  int done = nst;
+  float most = 0.f;  // of |z|, by formula
   if (nst > 0) {
     constexpr int DB = CNT ? 2 : D;  // right operands in flight
     Raw8<DT> buf[D];
@@ -722,21 +796,18 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
     }
     if constexpr (CNT != 0) fetch_b(bb[0], at(0));
     setup();
-    int k = 0;
+    int k = 0, nmain = nst;
     if constexpr (TAB) {
+      const uint4 w = buf[0].w[0];
+      if (__ballot(lut_over8(w.x, w.y, w.z, w.w)) != 0ull) nmain = done = 0;
       // software-pipelined one step deep: the table reads of step k + 1 are
       // issued before the right operands and MFMAs of step k, so their
       // latency hides behind that work
       uint2 E[8];
       lut_lookup8(buf[0].w[0], lut, E);
       auto step = [&](int j, int kj, bool refill) {
-        f16x8_t A[4][1];
-        {
-          f16x8_t T[4];
-          lut_planes(E, T);
-#pragma unroll
-          for (int pl = 0; pl < 4; ++pl) A[pl][0] = T[pl];
-        }
+        V A[4][1];
+        lut_planes(E, &A[0][0]);
         uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
         if constexpr (KEYS) tm = keys_of(bb[j % DB].lab, kp);
         lut_lookup8(buf[(j + 1) % D].w[0], lut, E);
@@ -747,111 +818,110 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
         __builtin_amdgcn_sched_barrier(0);
         if (CNT == 0 && refill) fetch_b(bb[j % DB], at(kj + D));
       };
-      for (; k + D <= nst; k += D) {
+      for (; k + D <= nmain; k += D) {
         if (prog && (k & (2 * D - 1)) == 0) pace(prog, k);
 #pragma unroll
         for (int j = 0; j < D; ++j) step(j, k + j, true);
       }
 #pragma unroll
       for (int j = 0; j < D - 1; ++j)  // the last nst % D steps
-        if (k + j < nst) step(j, k + j, false);
+        if (k + j < nmain) step(j, k + j, false);
     } else {
+      const float sc = WIDE ? 1.f : __builtin_ldexpf(1.f, a.form.lg);
+      if constexpr (!WIDE) {
+        float z[8];
+        raw_to_f32<DT>(buf[0], z);
+        if (__ballot(max_abs8(z, 0.f) > kNarrowMax) != 0ull) nmain = done = 0;
+      }
       auto step = [&](int j, int kj, bool refill) {
         // the key table reads go out before the plane work
         uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
         if constexpr (KEYS) tm = keys_of(bb[j % DB].lab, kp);
         if constexpr (CNT != 0) fetch_b(bb[(j + 1) % DB], at(kj + 1));
-        f16x8_t A[4][NS];
-        planes8_formula<DT, NS, false>(buf[j], ep, 8, unw, A, ub, up);
+        float z[8], v[4][8];
+        raw_to_f32<DT>(buf[j], z);
+        if constexpr (!WIDE) most = max_abs8(z, most);
+        planes8<false>(z, ep, sc, 8, unw, v, ub, up);
         // keep each refill below the last read of its slot, so that it reuses
         // the slot's registers instead of rotating the whole pipeline
         __builtin_amdgcn_sched_barrier(0);
         if (refill) load_raw8<DT>(a.logits, rowoff + at(kj + D) * kStep, buf[j]);
-        mma_step(A, bb[j % DB], kp, tm);
+        if constexpr (WIDE) {
+          mma_wide(v, bb[j % DB], kp, tm);
+        } else {
+          V A[4][NS];
+#pragma unroll
+          for (int pl = 0; pl < 4; ++pl) split_f16<NS>(v[pl], A[pl]);
+          mma_step(A, bb[j % DB], kp, tm);
+        }
         __builtin_amdgcn_sched_barrier(0);
         if (CNT == 0 && refill) fetch_b(bb[j % DB], at(kj + D));
       };
-      for (; k + D <= nst; k += D) {
+      for (; k + D <= nmain; k += D) {
         if (prog && (k & (2 * D - 1)) == 0) pace(prog, k);
 #pragma unroll
         for (int j = 0; j < D; ++j) step(j, k + j, true);
       }
 #pragma unroll
       for (int j = 0; j < D - 1; ++j)  // the last nst % D steps
-        if (k + j < nst) step(j, k + j, false);
+        if (k + j < nmain) step(j, k + j, false);
     }
   } else {
     setup();
   }
 
-  const int64_t tail0 = full * kStep + g4 * 8;  // the tail step's first cell of this lane
-  if (has_tail) {  // last partial step: guarded loads, masked planes
-    Raw8<DT> raw;
-    load_raw8_part<DT>(a.logits, rowoff + full * kStep, a.HW - tail0, raw);
-    f16x8_t A[4][NS];
-    planes8_formula<DT, NS, true>(raw, ep, a.HW - tail0, unw, A, ub, up);
-    BRaw x;
-    fetch_b(x, full);
-    uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
-    if constexpr (KEYS) tm = keys_of(x.lab, kp);
-    mma_step(A, x, kp, tm);
-  }
-
-  // every non-finite or oversized plane shows in the sums of A_neg and A_pos
-  bool bad = false;
+  if constexpr (TAB) {
+    // the marker shows in the sums of A_neg and A_pos
+    bool bad = false;
 #pragma unroll
-  for (int i = 0; i < (SUMS ? 2 : 1); ++i)
+    for (int i = 0; i < (SUMS ? 2 : 1); ++i)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bad |= !(fabsf(acc[i][nt][e]) < INFINITY);
-  bad = __ballot(bad) != 0;
-  if (bad) {  // bf16 operands, one step at a time
-    constexpr int NR = InTraits<DT>::kRedo;
-    clear();
-    const int64_t last = has_tail ? full + 1 : s1;
-    for (int64_t st = s0; st < last; ++st) {
-      if (st >= s1 && st < full) continue;
-      Raw8<DT> raw;
-      const int64_t nv = a.HW - (st * kStep + g4 * 8);
-      load_raw8_part<DT>(a.logits, rowoff + st * kStep, nv, raw);
-      bf16x8_t A[4][NR];
-      planes8_redo<DT>(raw, ep, nv, A);
-      BRaw x;
-      fetch_b(x, st);
-      uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
-      if constexpr (KEYS) tm = keys_of(x.lab, kp);
-      for_tiles(x, kp, tm, [&](int nt, const u32x4_t& raw) {
-        const u32x4_t n = CNT == 1 ? widen8<0>(raw[0], raw[1]) : raw;
-        auto mul = [&](int i, int pl, const u32x4_t& v) {
-          // counts up to 255 are exact in bf16; larger ones as high and low byte
-          const bf16x8_t lo = CNT == 0 ? redo8(v, 0xFFFFu, 8) : redo8(v, 0xFFu), hi = redo8(v, 0xFF00u);
-#pragma unroll
-          for (int sp = 0; sp < NR; ++sp) {
-            acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[pl][sp], lo, acc[i][nt], 0, 0, 0);
-            if constexpr (CNT == 2)
-              acc[i][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[pl][sp], hi, acc[i][nt], 0, 0, 0);
-          }
-        };
-        const uint32_t all = CNT == 0 ? kHot * 0x10001u : n2pair;
-        if constexpr (SUMS) {
-  #pragma unroll
-        for (int pl = 0; pl < 4; ++pl) mul(pl, pl, n);
-        } else {
-          mul(0, 0, isub8(all, n));
-          mul(0, 1, n);
-          mul(1, 2, n);
-          mul(2, 3, n);
-        }
-      });
-    }
-  }
-  {
-    const float sc = bad ? 1.f : (CNT == 0 && TAB ? 65536.f : 1.f) / kPlaneScale;
+        for (int e = 0; e < 4; ++e) bad |= !(fabsf(acc[i][nt][e]) < INFINITY);
+    const float undo = WIDE ? 2.f : __builtin_ldexpf(1.f, (CNT == 0 ? 16 : 0) - a.form.lg);
 #pragma unroll
     for (int i = 0; i < NP; ++i)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[i][nt] *= sc;
+      for (int nt = 0; nt < NT; ++nt) acc[i][nt] *= undo;
+    if (__builtin_expect(__ballot(bad) != 0ull, 0)) {
+      clear();
+      done = 0;
+    }
+  } else if constexpr (!WIDE) {
+    if (__builtin_expect(__ballot(most > kNarrowMax) != 0ull, 0)) {
+      clear();
+      ub = up = 0.f;
+      done = 0;
+    }
+  }
+
+  // Steps by the formulas with bf16 operands, the next one's loads in flight: the
+  // last partial step, or a whole range (redone).
+  // (Marked unlikely, so that it takes no registers from the loops above.)
+  const int nall = nst + (has_tail ? 1 : 0);
+  if (__builtin_expect(done < nall, 0)) {
+    const int64_t tailn = a.HW - (full * kStep + g4 * 8);  // valid cells of the partial step
+    Raw8<DT> raw, nraw;
+    BRaw x, nx;
+    auto fetch = [&](int k) {
+      const int64_t st = k < nst ? s0 + k : full;
+      if (k < nst) load_raw8<DT>(a.logits, rowoff + st * kStep, nraw);
+      else load_raw8_part<DT>(a.logits, rowoff + st * kStep, tailn, nraw);
+      fetch_b(nx, st);
+    };
+    fetch(done);
+    for (int k = done; k < nall; ++k) {
+      raw = nraw;
+      x = nx;
+      if (k + 1 < nall) fetch(k + 1);
+      uint32_t kp[4] = {0u, 0u, 0u, 0u}, tm = 0;
+      if constexpr (KEYS) tm = keys_of(x.lab, kp);
+      float z[8], v[4][8];
+      raw_to_f32<DT>(raw, z);
+      planes8<true>(z, ep, 1.f, k < nst ? 8 : tailn, unw, v, ub, up);
+      mma_wide(v, x, kp, tm);
+    }
   }
 
   if constexpr (SUMS) if (red.buf) {
@@ -922,7 +992,7 @@ constexpr int kClassOf = NT == 2 ? 0 : NT == 7 ? 1 : 2;
 // grid's groups is task u % n at partial u / n, its R waves take R
 // consecutive splits of the R * KS-way split and add their sums in LDS
 // (n * KS * R <= slots, so the groups fit the grid).
-template <int DT, int NT, int CNT, bool TAB>
+template <int DT, int NT, int CNT, bool TAB, bool WIDE>
 __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs a) {
   constexpr int CI = kClassOf<NT>;
   constexpr int WV = cost_waves(NT, TAB);
@@ -940,7 +1010,7 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
   const int64_t total = n * KS;
   // table build + barrier: once per wave, after its first loads are in flight
   auto setup = [&]() {
-    if constexpr (TAB) build_lut(lut_s, a.ep);
+    if constexpr (TAB) build_lut<WIDE>(lut_s, a.ep, a.form.lg);
     __syncthreads();
   };
   constexpr int64_t tile = class_planes(CI) * 16 * 16 * NT;
@@ -968,7 +1038,7 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
     red.R = R;
     red.r = r;
     red.grp = grp;
-    cost_wave<DT, NT, CNT, TAB>(a, lb, rtile, kp * R + r, KS * R, lut_s, out, rs, nullptr, setup, red, klut);
+    cost_wave<DT, NT, CNT, TAB, WIDE>(a, lb, rtile, kp * R + r, KS * R, lut_s, out, rs, nullptr, setup, red, klut);
     return;
   }
   const int64_t w0 = (int64_t)blockIdx.x * WV;
@@ -985,7 +1055,7 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
   float* out = a.partials + a.plan.float_base[CI] + w * tile;
   float* rs = a.rowsum ? a.rowsum + (a.plan.slot_base[CI] + w) * 16 * 2 : nullptr;
   // pace the waves only where many share the workgroup's CU
-  cost_wave<DT, NT, CNT, TAB>(a, lb, rtile, ks, KS, lut_s, out, rs, WV >= 16 ? prog_s : nullptr, setup,
+  cost_wave<DT, NT, CNT, TAB, WIDE>(a, lb, rtile, ks, KS, lut_s, out, rs, WV >= 16 ? prog_s : nullptr, setup,
                               SplitRed(), klut);
 }
 
@@ -1100,7 +1170,8 @@ __device__ __forceinline__ u32x4_t ring_read_async(uint32_t addr) {
   asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
   return v;
 }
-__device__ __forceinline__ void lut_planes64(const uint64_t E64[8], f16x8_t A[4]) {
+template <class V>
+__device__ __forceinline__ void lut_planes64(const uint64_t E64[8], V A[4]) {
   uint2 E[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) E[i] = make_uint2((uint32_t)E64[i], (uint32_t)(E64[i] >> 32));
@@ -1143,8 +1214,8 @@ constexpr int64_t kPairTile = 3 * 32 * 32;            // partial tile (floats)
 static_assert(kPairGroupCells * 32 * 2 == (int)kGroupBytes, "a pair group fills one ring slot");
 static_assert(kPairGroupCells == kCountCells, "a group's counts are one block");
 
-// CNT: 0 label map, 1 u8 counts
-template <int CNT, class Setup>
+// CNT: 0 label map, 1 u8 counts; WIDE: a table of bf16 (label maps only)
+template <int CNT, bool WIDE, class Setup>
 __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, int64_t q0, int64_t ks,
                                                int64_t KS, const unsigned char* lut, uint32_t ring,
                                                f32x16_t (&acc)[3], Setup&& setup) {
@@ -1173,7 +1244,9 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
   };
   clear();
 
-  const uint32_t top = (uint32_t)__builtin_amdgcn_readfirstlane((int)opnd_top(a.N2));
+  using V = typename Ops<WIDE>::v8;
+  RightF16 rf = right_f16(0, a.N2);
+  rf.top = (uint32_t)__builtin_amdgcn_readfirstlane((int)rf.top);
   // full K-steps of this split (whole groups with counts), then the tail
   const int64_t full = CNT ? a.HW / kPairGroupCells * kGroupSteps : a.HW / kPairStep;
   const int64_t ngr = ceil_div(full, kGroupSteps);
@@ -1223,12 +1296,15 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
     lbuf[j] = j ? label_load<16>(p, crow + 32u * h) : label_load<0>(p, crow + 32u * h);
   };
 
-  auto mma = [&](const f16x8_t (&A)[4], const Opnd& o) {
-    acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], o.rest, acc[0], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[2], o.n, acc[1], 0, 0, 0);
-    acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[3], o.n, acc[2], 0, 0, 0);
-    acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], o.n, acc[0], 0, 0, 0);
+  auto mma_ops = [&](auto ops, const auto& A, const Opnd& o) {
+    using O = decltype(ops);
+    const auto n = __builtin_bit_cast(typename O::v8, o.n), rest = __builtin_bit_cast(typename O::v8, o.rest);
+    acc[0] = O::mma32(A[0], rest, acc[0]);
+    acc[1] = O::mma32(A[2], n, acc[1]);
+    acc[2] = O::mma32(A[3], n, acc[2]);
+    acc[0] = O::mma32(A[1], n, acc[0]);
   };
+  auto mma = [&](const V (&A)[4], const Opnd& o) { mma_ops(Ops<WIDE>(), A, o); };
 
   // Every load of the pipeline is issued in a fixed order, so the vmcnt waits
   // below are exact.
@@ -1244,6 +1320,7 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
   // LDS reads run two steps ahead for the ring and one for the table: step t waits
   // for both (lds_wait), then issues the table reads of step t + 1 and the ring
   // read of step t + 2.
+  int k = nst;  // steps summed by the table
   if (nst > 0) {
     const int ngl = (int)(g1 - g0);
     const uint32_t lut_base = (uint32_t)(size_t)(lds_void_t*)lut;
@@ -1262,9 +1339,11 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
     else __builtin_amdgcn_s_waitcnt(0x0F74);                // vmcnt(4)
     uint64_t E[8];
     u32x4_t xr[2];  // ring words of steps t + 1 (xr[(t + 1) & 1]) and t + 2
-    lut_lookup8_asm(ring_read(step_addr(0)), lut_base, E);
+    const u32x4_t x0 = ring_read(step_addr(0));
+    if (__ballot(lut_over8(x0[0], x0[1], x0[2], x0[3])) != 0ull) k = 0;  // a filled region: redone at once
+    lut_lookup8_asm(x0, lut_base, E);
     xr[1] = nst > 1 ? ring_read_async(step_addr(1)) : u32x4_t{0u, 0u, 0u, 0u};
-    for (int t0 = 0; t0 < nst; t0 += kGroupSteps) {
+    for (int t0 = 0; t0 < k; t0 += kGroupSteps) {
 #pragma unroll
       for (int s = 0; s < kGroupSteps; ++s) {  // s compile-time: lbuf and xr stay in registers
         const int t = t0 + s;
@@ -1272,7 +1351,7 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
           u32x4_t& xn = xr[(s + 1) & 1];  // step t + 1
           u32x4_t& xnn = xr[s & 1];       // step t + 2
           lds_wait(E, xn);
-          f16x8_t A[4];
+          V A[4];
           lut_planes64(E, A);
           // E is consumed above the next lookups, which then reuse its
           // registers.  Past the last step the lookups and ring reads still
@@ -1287,17 +1366,17 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
           }
           xnn = ring_read_async(step_addr(t + 2));
           if (s == kGroupSteps - 1) {  // every step of this slot is read: refill it two groups on
-            const int k = t0 / kGroupSteps;
-            fetch_group(k & (kRingGroups - 1), g0 + min(k + kRingGroups, ngl - 1));
+            const int gk = t0 / kGroupSteps;
+            fetch_group(gk & (kRingGroups - 1), g0 + min(gk + kRingGroups, ngl - 1));
           }
           Opnd o;
           if constexpr (CNT) {
             if (s == 0) label_wait<5>(lbuf[0]);
-            o = opnd_u8<true>(lbuf[s >> 1][2 * (s & 1)], lbuf[s >> 1][2 * (s & 1) + 1], top);
+            o = opnd_u8<true>(lbuf[s >> 1][2 * (s & 1)], lbuf[s >> 1][2 * (s & 1) + 1], rf);
           } else {
             label_wait<7>(lbuf[s]);
             const uint32_t L2[4] = {lbuf[s][0], lbuf[s][1], lbuf[s][2], lbuf[s][3]};
-            o = opnd_hot<kHot, true>(hot8(L2, colL, colM));
+            o = opnd_tab<WIDE>(hot8(L2, colL, colM));
           }
           __builtin_amdgcn_sched_barrier(0);
           mma(A, o);
@@ -1319,59 +1398,63 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
   // steps at natural cell order (16 st + 8 h + (0 .. 7)), guarded: the tail, and a redone range
   const ElemParams ep = a.ep;
   const int64_t rowoff = (lb * a.Q + min(q0 + r, a.Q - 1)) * a.HW + h * 8;
-  // the 16-bit integers of step st (compare results or counts)
+  // raw right operand of step st: compare results, or counts in the first two words
   auto counts_of = [&](int64_t st) -> u32x4_t {
     if constexpr (CNT) {
       const int64_t cell = st * kPairStep + h * 8;
       const uint2 c = *(const uint2*)(cimg + (cell >> 6) * cstep + crow + (cell & 63));
-      return widen8<0>(c.x, c.y);
+      return u32x4_t{c.x, c.y, 0u, 0u};
     } else {
       const uint4 lv = *(const uint4*)(labp + st * kPairStep + h * 8);
       const uint32_t L2[4] = {lv.x, lv.y, lv.z, lv.w};
       return hot8(L2, colL, colM);
     }
   };
-  const uint32_t all = CNT ? (uint32_t)a.N2 * 0x10001u : kHot * 0x10001u;
-  for (int64_t st = full; st < steps; ++st) {
-    const int64_t nv = a.HW - (st * kPairStep + h * 8);
-    Raw8<ML_BF16> raw;
-    load_raw8_part<ML_BF16>(a.logits, rowoff + st * kPairStep, nv, raw);
-    f16x8_t T[4][1];
-    float ub = 0.f, up = 0.f;
-    planes8_formula<ML_BF16, 1, true>(raw, ep, nv, false, T, ub, up);
-    const f16x8_t A[4] = {T[0][0], T[1][0], T[2][0], T[3][0]};
-    const u32x4_t n = counts_of(st);
-    if constexpr (CNT) mma(A, Opnd{part8<false>(n), part8<false>(isub8(all, n))});
-    else mma(A, opnd_hot<kHot, true>(n));
-  }
-  // |z| >= 64, inf or nan somewhere in the range: bf16 operands, one step at a time
+  // |z| >= 64, inf or nan somewhere in the range (the table's marker): redone
   bool bad = false;
 #pragma unroll
   for (int e = 0; e < 16; ++e) bad |= !(fabsf(acc[0][e]) < INFINITY);
-  bad = __ballot(bad) != 0;
-  if (bad) {
-    clear();
-    for (int64_t st = s0; st < steps; ++st) {
-      if (st >= s0 + nst && st < full) st = full;
-      if (st >= steps) break;
-      const int64_t nv = a.HW - (st * kPairStep + h * 8);
-      Raw8<ML_BF16> raw;
-      load_raw8_part<ML_BF16>(a.logits, rowoff + st * kPairStep, nv, raw);
-      bf16x8_t A[4][1];
-      planes8_redo<ML_BF16>(raw, ep, nv, A);
-      const u32x4_t n = counts_of(st);
-      const bf16x8_t Bp = redo8(isub8(all, n), 0xFFFFu, CNT ? 0 : 8), Bv = redo8(n, 0xFFFFu, CNT ? 0 : 8);
-      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0][0], Bp, acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[2][0], Bv, acc[1], 0, 0, 0);
-      acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[3][0], Bv, acc[2], 0, 0, 0);
-      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[1][0], Bv, acc[0], 0, 0, 0);
-    }
-  }
-  const float sc = bad ? 1.f : (CNT ? 1.f : 65536.f) / kPlaneScale;
+  const float undo = WIDE ? 2.f : __builtin_ldexpf(1.f, (CNT ? 0 : 16) - a.form.lg);
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[i][e] *= sc;
+    for (int e = 0; e < 16; ++e) acc[i][e] *= undo;
+  if (__builtin_expect(__ballot(bad) != 0ull, 0)) {
+    clear();
+    k = 0;
+  }
+  // the tail and a redone range: the formulas and bf16 operands, the next step's
+  // loads in flight
+  const int nall = nst + (int)(steps - full);
+  if (__builtin_expect(k < nall, 0)) {
+    auto nv_of = [&](int64_t st) { return a.HW - (st * kPairStep + h * 8); };
+    Raw8<ML_BF16> raw, nraw;
+    u32x4_t n, nn;
+    auto fetch = [&](int k) {
+      const int64_t st = k < nst ? s0 + k : full + (k - nst);
+      if (k < nst) load_raw8<ML_BF16>(a.logits, rowoff + st * kPairStep, nraw);
+      else load_raw8_part<ML_BF16>(a.logits, rowoff + st * kPairStep, nv_of(st), nraw);
+      nn = counts_of(st);
+    };
+    fetch(k);
+    for (; k < nall; ++k) {
+      raw = nraw;
+      n = nn;
+      if (k + 1 < nall) fetch(k + 1);
+      float z[8], v[4][8], ub = 0.f, up = 0.f;
+      raw_to_f32<ML_BF16>(raw, z);
+      planes8<true>(z, ep, 1.f, k < nst ? 8 : nv_of(full + (k - nst)), false, v, ub, up);
+      bf16x8_t A[4];
+#pragma unroll
+      for (int pl = 0; pl < 4; ++pl) split_bf16<1>(v[pl], &A[pl]);
+      if constexpr (CNT) {
+        mma_ops(Ops<true>(), A, wide_u8(n[0], n[1], a.N2));
+      } else {
+        const u32x4_t one = wide_hot8(n);
+        mma_ops(Ops<true>(), A, Opnd{one, isub8(0x3F803F80u, one)});
+      }
+    }
+  }
 }
 
 // One wave's accumulators in LDS (12 KB): 4 consecutive registers per lane
@@ -1395,7 +1478,7 @@ __device__ __forceinline__ void acc_add_lds(f32x16_t (&acc)[3], const float* buf
     }
 }
 
-template <int CNT>
+template <int CNT, bool WIDE>
 __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
   __shared__ __align__(16) unsigned char lds[kDmaLds];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1412,7 +1495,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
   const int64_t pq = g / KSq, ksq = g - pq * KSq, p = 4 * pq + (wave >> 2);
   const int kq = wave & 3;
   auto setup = [&]() {
-    build_lut(lds, a.ep);
+    build_lut<WIDE>(lds, a.ep, a.form.lg);
     __syncthreads();
   };
   f32x16_t acc[3];
@@ -1424,7 +1507,7 @@ __global__ __launch_bounds__(64 * kDmaWaves) void cost_pair_kernel(CostArgs a) {
     const int64_t task = __builtin_amdgcn_readfirstlane(a.sched[kSchedList + j * rt + 2 * rp]);
     lb = task / rt;
     const uint32_t ring = (uint32_t)(size_t)(lds_void_t*)lds + ring_base(wave);
-    cost_wave_pair<CNT>(a, lb, 32 * rp, 4 * ksq + kq, 4 * KSq, lds, ring, acc, setup);
+    cost_wave_pair<CNT, WIDE>(a, lb, 32 * rp, 4 * ksq + kq, 4 * KSq, lds, ring, acc, setup);
   } else {
     setup();
   }
@@ -1478,28 +1561,33 @@ static int occ_slots(std::atomic<int> (&cache)[64], const void* kernel, int wave
   }
   return v;
 }
-template <int DT, int NT, int CNT, bool TAB>
+template <int DT, int NT, int CNT, bool TAB, bool WIDE>
 static int occ_slots_of() {
   static std::atomic<int> cache[64];
-  return occ_slots(cache, (const void*)cost_kernel<DT, NT, CNT, TAB>, cost_waves(NT, TAB));
+  return occ_slots(cache, (const void*)cost_kernel<DT, NT, CNT, TAB, WIDE>, cost_waves(NT, TAB));
 }
-template <int CNT>
+template <int CNT, bool WIDE>
 static int occ_slots_pair() {
   static std::atomic<int> cache[64];
-  return occ_slots(cache, (const void*)cost_pair_kernel<CNT>, (int)kDmaWaves);
+  return occ_slots(cache, (const void*)cost_pair_kernel<CNT, WIDE>, (int)kDmaWaves);
 }
 
 // cnt: 0 label map, 1 u8 counts, 2 u16 counts
 template <int DT, int NT>
-static int occ_slots_for(int cnt, bool tab) {
+static int occ_slots_for(int cnt, bool tab, bool wide) {
   constexpr bool kTab = DT == ML_BF16;
   if (kTab && tab)
-    return cnt == 1   ? occ_slots_of<DT, NT, 1, kTab>()
-           : cnt == 2 ? occ_slots_of<DT, NT, 2, kTab>()
-                      : occ_slots_of<DT, NT, 0, kTab>();
-  return cnt == 1   ? occ_slots_of<DT, NT, 1, false>()
-         : cnt == 2 ? occ_slots_of<DT, NT, 2, false>()
-                    : occ_slots_of<DT, NT, 0, false>();
+    return cnt == 1   ? occ_slots_of<DT, NT, 1, kTab, false>()
+           : cnt == 2 ? occ_slots_of<DT, NT, 2, kTab, false>()
+           : wide     ? occ_slots_of<DT, NT, 0, kTab, true>()
+                      : occ_slots_of<DT, NT, 0, kTab, false>();
+  if (wide)
+    return cnt == 1   ? occ_slots_of<DT, NT, 1, false, true>()
+           : cnt == 2 ? occ_slots_of<DT, NT, 2, false, true>()
+                      : occ_slots_of<DT, NT, 0, false, true>();
+  return cnt == 1   ? occ_slots_of<DT, NT, 1, false, false>()
+         : cnt == 2 ? occ_slots_of<DT, NT, 2, false, false>()
+                    : occ_slots_of<DT, NT, 0, false, false>();
 }
 
 static int cu_count() {
@@ -1518,32 +1606,53 @@ static int cu_count() {
 // their launches may run beside the widest class's assignment (one
 // workgroup per image on the forward's side stream).
 template <int DT>
-static void plan_slots(CostPlan& p, int cnt, bool tab, int64_t side) {
+static void plan_slots(CostPlan& p, int cnt, bool tab, bool wide, int64_t side) {
   const int cus = cu_count();
   side = std::min<int64_t>(side, cus / 8);
   for (int ci = 0; ci < p.nclass; ++ci) {
     int v = 0;
     switch (ci) {
       case 0:
-        v = !p.pair0 ? occ_slots_for<DT, 2>(cnt, tab) : cnt ? occ_slots_pair<1>() : occ_slots_pair<0>();
+        v = !p.pair0 ? occ_slots_for<DT, 2>(cnt, tab, wide)
+            : cnt    ? occ_slots_pair<1, false>()
+            : wide   ? occ_slots_pair<0, true>()
+                     : occ_slots_pair<0, false>();
         break;
-      case 1: v = occ_slots_for<DT, 7>(cnt, tab); break;
-      default: v = occ_slots_for<DT, 16>(cnt, tab); break;
+      case 1: v = occ_slots_for<DT, 7>(cnt, tab, wide); break;
+      default: v = occ_slots_for<DT, 16>(cnt, tab, wide); break;
     }
     if (p.nclass == kClasses && ci < kClasses - 1) v -= (int)((int64_t)v * side / cus);
     p.slots[ci] = (int)std::min<int64_t>(std::max(v, 8), kCostSlots);
   }
 }
 
-CostPlan make_cost_plan(const Dims& d, int dtype, bool tab) {
+// Operands of the contraction for the call's per-logit terms (see the top).
+CostForm cost_form(const Dims& d, int dtype, const ElemParams& ep, bool force_masks) {
+  CostForm f;
+  // focal powers, and weights below 2^-6, leave planes of any size
+  f.wide = ep.gamma_mode != 0 || (ep.ug_mode != 0 && ep.ug_min < 0.015625f);
+  // bf16 table: a wide one holds label maps only, float16 counts being its right operand
+  f.tab = dtype == ML_BF16 && g_use_lut && !force_masks && !(f.wide && d.counts_mode);
+  // the largest power of two that keeps the planes of |z| <= zmax below 65504:
+  // w softplus(|z|) <= zmax without weights, and H softplus(|z|) < 1.2 where the
+  // weight is H^ug, ug >= 1, above its floor
+  const float zmax = f.tab ? 63.75f : kNarrowMax;
+  float most = zmax * 1.0001f;
+  if (ep.ug_mode != 0 && ep.ug >= 1.f) most = std::max(1.2f, ep.ug_min * (zmax + 1.f));
+  f.lg = 0;
+  while (f.lg < 14 && std::max(most, 1.f) * (float)(2 << f.lg) <= 65504.f) ++f.lg;
+  return f;
+}
+
+CostPlan make_cost_plan(const Dims& d, int dtype, const CostForm& f) {
   CostPlan p = bound_cost_plan(d);
   const int cnt = d.counts_mode ? d.cw : 0;
-  p.pair0 = dtype == ML_BF16 && tab && d.pair_ok ? 1 : 0;
+  p.pair0 = f.tab && d.pair_ok ? 1 : 0;
   const int64_t side = std::min<int64_t>(d.LB, kSideCUs);
   switch (dtype) {
-    case ML_F32: plan_slots<ML_F32>(p, cnt, false, side); break;
-    case ML_BF16: plan_slots<ML_BF16>(p, cnt, tab, side); break;
-    case ML_F16: plan_slots<ML_F16>(p, cnt, false, side); break;
+    case ML_F32: plan_slots<ML_F32>(p, cnt, false, f.wide, side); break;
+    case ML_BF16: plan_slots<ML_BF16>(p, cnt, f.tab, f.wide, side); break;
+    case ML_F16: plan_slots<ML_F16>(p, cnt, false, f.wide, side); break;
   }
   return p;
 }
@@ -1552,17 +1661,22 @@ template <int DT, int NT, bool TAB>
 static void launch_cnt(const CostArgs& a, const Dims& d, hipStream_t st) {
   const int WV = cost_waves(NT, TAB);
   const dim3 grid((unsigned)ceil_div(std::max<int64_t>(a.plan.slots[kClassOf<NT>], a.plan.ntasks), WV)), blk(64 * WV);
-  if (!d.counts_mode) hipLaunchKernelGGL((cost_kernel<DT, NT, 0, TAB>), grid, blk, 0, st, a);
-  else if (d.cw == 1) hipLaunchKernelGGL((cost_kernel<DT, NT, 1, TAB>), grid, blk, 0, st, a);
-  else hipLaunchKernelGGL((cost_kernel<DT, NT, 2, TAB>), grid, blk, 0, st, a);
+  auto launch = [&](auto wide) {
+    constexpr bool WIDE = decltype(wide)::value, COUNTS = !(TAB && WIDE);
+    if (!COUNTS || !d.counts_mode) hipLaunchKernelGGL((cost_kernel<DT, NT, 0, TAB, WIDE>), grid, blk, 0, st, a);
+    else if (d.cw == 1) hipLaunchKernelGGL((cost_kernel<DT, NT, COUNTS ? 1 : 0, TAB, WIDE>), grid, blk, 0, st, a);
+    else hipLaunchKernelGGL((cost_kernel<DT, NT, COUNTS ? 2 : 0, TAB, WIDE>), grid, blk, 0, st, a);
+  };
+  if (a.form.wide) launch(std::true_type());
+  else launch(std::false_type());
 }
 
 template <int DT, int NT>
-static int launch_one(const CostArgs& a, const Dims& d, bool tab, hipStream_t st) {
+static int launch_one(const CostArgs& a, const Dims& d, hipStream_t st) {
   constexpr int CI = kClassOf<NT>;
   if (NT == 2 && a.plan.pair0) {
     // the schedule's K-split was chosen for row-tile pairs
-    if (DT != ML_BF16 || !tab || !d.pair_ok || d.rows != 16)
+    if (DT != ML_BF16 || !a.form.tab || !d.pair_ok || d.rows != 16)
       return fail(ML_EINVAL, "internal: row-tile pair plan without the bf16 table path");
     // workgroups: ceil(np / 4) pair quads x KSq split quads, where np * 4 KSq
     // <= max(slots, np) unless KSq = 1 (then np <= L B ceil(rtiles / 2)), and
@@ -1570,11 +1684,12 @@ static int launch_one(const CostArgs& a, const Dims& d, bool tab, hipStream_t st
     const int64_t np_max = d.LB * ((d.rtiles + 1) / 2);
     const int64_t wgs = ceil_div(a.plan.slots[CI], 16) + ceil_div(np_max, 4) + d.ks_max / 4 + 1;
     const dim3 grid((unsigned)wgs), blk(64 * kDmaWaves);
-    if (d.counts_mode) hipLaunchKernelGGL(cost_pair_kernel<1>, grid, blk, 0, st, a);
-    else hipLaunchKernelGGL(cost_pair_kernel<0>, grid, blk, 0, st, a);
+    if (d.counts_mode) hipLaunchKernelGGL((cost_pair_kernel<1, false>), grid, blk, 0, st, a);
+    else if (a.form.wide) hipLaunchKernelGGL((cost_pair_kernel<0, true>), grid, blk, 0, st, a);
+    else hipLaunchKernelGGL((cost_pair_kernel<0, false>), grid, blk, 0, st, a);
     return check_launch("pair_cost");
   }
-  if (DT == ML_BF16 && tab) launch_cnt<DT, NT, DT == ML_BF16>(a, d, st);
+  if (DT == ML_BF16 && a.form.tab) launch_cnt<DT, NT, DT == ML_BF16>(a, d, st);
   else launch_cnt<DT, NT, false>(a, d, st);
   return check_launch("pair_cost");
 }
@@ -1582,23 +1697,20 @@ static int launch_one(const CostArgs& a, const Dims& d, bool tab, hipStream_t st
 // One launch per column-tile class up to the padded width; each image is
 // processed by exactly one of them.
 template <int DT>
-static int launch_classes(const CostArgs& a, const Dims& d, bool tab, unsigned classes, hipStream_t st) {
+static int launch_classes(const CostArgs& a, const Dims& d, unsigned classes, hipStream_t st) {
   int rc = 0;
-  if (classes & 1u) rc = launch_one<DT, 2>(a, d, tab, st);
-  if (!rc && a.plan.nclass > 1 && (classes & 2u)) rc = launch_one<DT, 7>(a, d, tab, st);
-  if (!rc && a.plan.nclass > 2 && (classes & 4u)) rc = launch_one<DT, 16>(a, d, tab, st);
+  if (classes & 1u) rc = launch_one<DT, 2>(a, d, st);
+  if (!rc && a.plan.nclass > 1 && (classes & 2u)) rc = launch_one<DT, 7>(a, d, st);
+  if (!rc && a.plan.nclass > 2 && (classes & 4u)) rc = launch_one<DT, 16>(a, d, st);
   return rc;
 }
 
-int launch_cost(const CostArgs& a, const Dims& d, int dtype, bool, hipStream_t st, unsigned classes,
-                bool prof) {
+int launch_cost(const CostArgs& a, const Dims& d, int dtype, hipStream_t st, unsigned classes, bool prof) {
   ProfScope ps_(prof ? "pair_cost" : nullptr, st);
-  // bf16 without unweighted row sums: table path
-  const bool tab = dtype == ML_BF16 && a.use_lut && a.rowsum == nullptr;
   switch (dtype) {
-    case ML_F32: return launch_classes<ML_F32>(a, d, false, classes, st);
-    case ML_BF16: return launch_classes<ML_BF16>(a, d, tab, classes, st);
-    case ML_F16: return launch_classes<ML_F16>(a, d, false, classes, st);
+    case ML_F32: return launch_classes<ML_F32>(a, d, classes, st);
+    case ML_BF16: return launch_classes<ML_BF16>(a, d, classes, st);
+    case ML_F16: return launch_classes<ML_F16>(a, d, classes, st);
   }
   return fail(ML_EINVAL, "unsupported mask logits dtype");
 }

@@ -241,7 +241,14 @@ Layout make_layout(const Dims& d, bool force_masks, const CostPlan& pl);
 Layout make_layout(const Dims& d, bool force_masks);  // with bound_cost_plan(d)
 // Plan slots / offsets of the cost launches (queries kernel occupancy on the
 // current device; the workspace bound uses kCostSlots only).
-CostPlan make_cost_plan(const Dims& d, int dtype, bool tab);
+// How a call's contraction forms its operands (see ml_cost.hip).
+struct CostForm {
+  bool tab;   // bf16 logits: per-cell planes from the LDS table
+  bool wide;  // bf16 operands throughout: the planes may get small at any logit
+  int lg;     // float16 planes are scaled by 2^lg
+};
+CostForm cost_form(const Dims& d, int dtype, const ElemParams& ep, bool force_masks);
+CostPlan make_cost_plan(const Dims& d, int dtype, const CostForm& f);
 CostPlan bound_cost_plan(const Dims& d);
 // Region offsets re-packed for the plan's own slot counts (class c holds
 // max(slots[c], ntasks) work items): the smallest layout that gives the same
@@ -309,7 +316,7 @@ struct CostArgs {
   int nslot;
   float N2;
   ElemParams ep;
-  int use_lut;       // bf16 logits: per-cell planes from the LDS table
+  CostForm form;
 };
 
 struct LayerArgs {
@@ -488,8 +495,8 @@ struct ProfScope {
 int launch_prep(const PrepArgs& a, const Dims& d, hipStream_t st);
 // classes: bit c launches column-tile class c (all by default); prof: bracket
 // the launches with the profiling events
-int launch_cost(const CostArgs& a, const Dims& d, int dtype, bool force_masks, hipStream_t st,
-                unsigned classes = ~0u, bool prof = true);
+int launch_cost(const CostArgs& a, const Dims& d, int dtype, hipStream_t st, unsigned classes = 7u,
+                bool prof = true);
 int launch_finalize(const AssignArgs& a, const Dims& d, hipStream_t st,
                     const char* prof = "finalize");
 int launch_assign(const AssignArgs& a, const Dims& d, hipStream_t st, const char* prof = "assign");
