@@ -1076,9 +1076,10 @@ bool dense_plan(const ml_dense_shape* s, int dtype, bool dice, bool backward, De
   d.cw = d.s >= 16 ? 2 : 1;
   d.crows = d.C;
   P.groups = dense_groups(d.L, d.B, d.C, d.HW, d.s, dtype == ML_F32, dice, backward);
-  P.tgt_bytes = align256(target_bytes(d));  // kept in the size where no counts are stored: one rule for callers
+  P.tgt_bytes = P.groups ? 0 : align256(target_bytes(d));  // groups: no counts are stored
   P.partial_off = P.tgt_bytes;
   P.total = P.tgt_bytes + (backward ? 0 : align256(dense_partials_bytes(d.L, d.B, d.C, d.HW, P.groups, dice)));
+  if (P.groups) P.total = std::max<size_t>(P.total, 256);  // a size of 0 stands for a refused shape
   return true;
 }
 

@@ -121,6 +121,26 @@ def test_dense_workspace_query():
     assert lib.ml_dense_loss_workspace_size(ctypes.byref(DShape(1, 2, 4, 1, 1, 256, 256)), 1, 0, 0) == 0
 
 
+def test_dense_workspace_without_counts():
+    """Where the kernels count in LDS (s in 2..15, 16 or more classes, not the dice
+    forward) no counts are stored, and the size asks for none."""
+    import torch  # noqa: F401
+    if not os.path.exists(LIB):
+        pytest.skip("library not built")
+    lib = ctypes.CDLL(LIB)
+
+    class DShape(ctypes.Structure):
+        _fields_ = [(k, ctypes.c_int64) for k in ["L", "B", "C", "H", "W", "Ht", "Wt"]]
+
+    lib.ml_dense_loss_workspace_size.restype = ctypes.c_size_t
+    shape = ctypes.byref(DShape(1, 4, 150, 128, 128, 512, 512))
+    counts = 4 * 150 * 128 * 128
+    for dtype in range(3):
+        for dice, bwd in ((0, 0), (0, 1), (1, 1)):
+            assert 0 < lib.ml_dense_loss_workspace_size(shape, dtype, dice, bwd) < counts // 64
+        assert lib.ml_dense_loss_workspace_size(shape, dtype, 1, 0) >= counts
+
+
 def test_point_sampling_queries_and_host_tensors_rejected():
     """The front end's size queries accept only the (L,B,C,1,P) sampled shape
     and valid planes; its operators reject host tensors (no CPU path)."""
