@@ -151,3 +151,39 @@ def test_dense_groups(ml, shape, dtype):
     ref = O.dice_loss_backward(go.cpu().numpy(), z64, t, *sums, 1.0, nm, 1.5)
     close_extra(ml.backward_dice_loss(go, zt, tt, I, P, T, 1.0, nm, 1.5).float().cpu().numpy(), ref, RTOL[dtype],
                 1e-2 * np.abs(ref).max(), sub + dice_grad_cancellation(go.cpu().numpy(), z64, t, *sums, 1.0, nm, 1.5))
+
+
+@pytest.mark.parametrize("shape", [(2, 40, 40, 300), (2, 24, 40, 300), (4, 24, 25, 500), (2, 64, 72, 2),
+                                   (4, 128, 136, 20), (3, 40, 57, 60)], ids=lambda v: "s%d_%dx%d_L%d" % v)
+def test_pair_groups(ml, shape):
+    """The pair kernel on u8 counts with more 64-cell groups per wave than its two
+    ring slots: with 4,096 waves resident the shapes give 7, 4, 3, 2, 6 and 3
+    groups, the third and the last a tail that is no whole group.  Every layer
+    holds the same logits, so one layer's oracle serves the waves of all.
+
+    Each group has labels of its own, and the logits' size changes from group to
+    group, so a group's logits or counts taken for another's show at once.  Planes
+    of 11 bits and counts that are exact put each sum within 2^-12 of itself (all
+    terms are non-negative), a quotient within 2^-11; the entry for |z| < 2^-9 and
+    the float32 sums are far below the rest of the 2^-10 allowed."""
+    s, H, W, L = shape
+    rng = np.random.default_rng(s * 1000 + W)
+    B, Q, C, G = 2, 37, 6, 24
+    group = (np.arange(H * W) // 64).reshape(H, W)
+    own = 1 + (5 * group + rng.integers(0, 2, size=(B, H, W))) % G
+    t = np.repeat(np.repeat(own, s, 1), s, 2)
+    mixed = rng.random(t.shape) < 0.2
+    t[mixed] = rng.integers(-1, G + 2, size=int(mixed.sum()))
+    size = 0.25 + (7 * group) % 11 * 0.5
+    zt, z64 = rounded(rng.normal(size=(1, B, Q, H, W)) * size, "bfloat16")
+    zc = rng.normal(size=(1, B, Q, C)).astype(np.float32)
+    ct = rng.integers(0, C, size=(B, G + 1))
+    zg, zcg = zt.cuda().expand(L, -1, -1, -1, -1).contiguous(), torch.from_numpy(zc).cuda().expand(L, -1, -1, -1).contiguous()
+    got = ml.pairwise_mask_loss_forward(zg, on_gpu(t, False), zcg, torch.from_numpy(ct).cuda(), 1.0, 1.0, 1.0, 1.0, 0,
+                                        1.0, 0.05, 0.0, -1.0, 0.0, -1.0, True, True)
+    ref = O.pairwise_mask_loss_forward(z64, t, zc.astype(np.float64), ct, background_index=0, use_softmax=True)
+    for k in range(2):
+        want = torch.from_numpy(np.asarray(ref[k])).cuda().expand(L, -1, -1, -1)
+        there = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got[k]), there)
+        assert (got[k].double() - want)[there].abs().max().item() <= 2.0 ** -10 * max(1.0, want[there].abs().max().item())
