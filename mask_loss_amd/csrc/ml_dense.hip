@@ -289,9 +289,9 @@ __global__ __launch_bounds__(256) void dense_bwd_kernel(DenseArgs a, int64_t nch
 // Bound by the logits (and the gradient).  Counting in a launch of its own
 // costs another pass: at 4 images, 150 classes, 128 x 128, s = 4 that launch
 // took 7.9 us and wrote 9.8 MB which this one reads back beside 39 MB of
-// logits.Figures there, launch of the counts included: CE
-// forward 17.5 + 7.9 -> 16.0 us, CE gradient 23.4 + 7.9 -> 20.6 us (87 MB,
-// 4.2 TB/s), dice gradient 18.4 + 7.9 -> 18.8 us.
+// logits.  Figures there, launch of the counts included: CE forward 17.5 + 7.9 ->
+// 16.0 us, CE gradient 23.4 + 7.9 -> 20.6 us (87 MB, 4.2 TB/s), dice gradient
+// 18.4 + 7.9 -> 18.8 us.
 enum { kDenseCe = 0, kDenseCeGrad = 1, kDenseDiceGrad = 2 };
 constexpr int kFuseU = 4;  // class rows in flight per wave
 
@@ -460,18 +460,28 @@ constexpr int64_t kFuseLeast = 16;
 // float16: 12.5 M 29, 26 and 22 against 31, 34 and 26; 16 M 40, 49 and 40
 // against 29, 33 and 23; 84 M 126, 163 and 170 against 90, 133 and 91.
 constexpr int64_t kFuseElems = 3 << 22;
-// More groups than that only where the cells alone would leave CUs without a
-// workgroup: with 256 workgroups of 150 classes the three kernels below take
-// 16.0, 20.6 and 18.8 us, with 512 of 75 classes 16.6, 24.9 and 23.3, with
-// 1024 of 38 classes 21.6, 30.8 and 28.2.
+// More groups than that only where the cells alone leave whole multiples of CUs (256
+// on this card) without a workgroup: with 256 workgroups of 150 classes the three
+// kernels below take 16.0, 20.6 and 18.8 us, with 512 of 75 classes 16.6, 24.9 and
+// 23.3, with 1024 of 38 classes 21.6, 30.8 and 28.2; s = 8, 40 classes of one 200 x 200
+// map in 157 workgroups 16, 15 and 14, in 314 27, 26 and 26 (23, 21 and 19 with the
+// counts in memory).
 constexpr int64_t kFuseBlocks = 256;
+// ... and not where the groups' label reads add up: s = 12, 100 classes of one 128 x 128
+// map in 4 groups (76 MB) 33, 32 and 31 us, in 2 (38 MB) 29, 28 and 27, with the
+// counts in memory 30, 30 and 27; s = 10 in 4 groups (52 MB) 22, 21 and 20 against 25,
+// 24 and 21.  Over 16 to 160 classes and 4,096 to 147,456 cells at s = 2, 4, 5, 8, 10, 12 and
+// 15 the sum of the three is 1.65, 1.61, 1.50, 1.33, 1.23, 1.18 and 1.09 times as fast as with the
+// counts in memory (the least 0.85: s = 15, 100 and more classes of one 64 x 64 map).
+constexpr int64_t kFuseLabelBytes = (int64_t)56 << 20;
 int64_t dense_groups(int64_t L, int64_t B, int64_t C, int64_t HW, int64_t s, bool f32, bool dice, bool backward) {
   if (s < 2 || s > 15 || (dice && !backward) || B < 1 || C < kFuseLeast || B > 65535) return 0;
   if (L * B * C * HW > kFuseElems * (f32 ? 2 : 1)) return 0;
   const int64_t least = ceil_div(C, kFuseRows);
   if ((least - 1) * 8 * s * s > 2 * C) return 0;
-  const int64_t fill = std::min(ceil_div(kFuseBlocks, ceil_div(HW, kCntCells) * B), ceil_div(C, 16));
-  const int64_t g = std::max(least, fill);
+  const int64_t fill = std::min({kFuseBlocks / (ceil_div(HW, kCntCells) * B), kFuseLabelBytes / (8 * s * s * HW * B),
+                                 ceil_div(C, 16)});
+  const int64_t g = std::max({least, fill, (int64_t)1});
   return ceil_div(C, ceil_div(C, g));
 }
 

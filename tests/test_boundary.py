@@ -139,6 +139,14 @@ def test_dense_workspace_without_counts():
         for dice, bwd in ((0, 0), (0, 1), (1, 1)):
             assert 0 < lib.ml_dense_loss_workspace_size(shape, dtype, dice, bwd) < counts // 64
         assert lib.ml_dense_loss_workspace_size(shape, dtype, 1, 0) >= counts
+    # one partial sum per 256 cells and class group: groups only as far as the
+    # cells leave CUs without a workgroup (157 of 256 here), and as their label reads allow
+    def groups(s, B, C, H):
+        size = lib.ml_dense_loss_workspace_size(ctypes.byref(DShape(1, B, C, H, H, s * H, s * H)), 0, 0, 0)
+        return size / (8 * B * (-(-H * H // 256)))
+
+    assert 1 <= groups(8, 1, 40, 200) < 2 and 1 <= groups(8, 4, 100, 96) < 2 and 1 <= groups(15, 1, 100, 128) < 2
+    assert groups(4, 1, 150, 128) == 4 and groups(4, 4, 150, 128) == 1 and groups(4, 1, 161, 256) == 2
 
 
 def test_point_sampling_queries_and_host_tensors_rejected():
