@@ -117,13 +117,14 @@ __device__ __forceinline__ float rem_hi(float v, uint32_t w) {
 // ---- planes of one logit ---------------------------------------------------
 // Which of the per-logit forms a call takes (chosen once per 8 logits, wave-uniform):
 // 0 general; 1 no focal terms, weight H^1 (the operator's defaults); 2 no
-// focal terms, no weights; 3 focal gamma 2 with or without weights H^1.
+// focal terms, no weights; 3 focal gamma 2 with or without weights H^1; 4 no focal
+// terms, weight H^ug.
 __device__ __forceinline__ int elem_mode(const ElemParams& ep) {
   const bool plain = ep.gamma_mode == 0 && ep.an == 1.f && ep.ap == 1.f;
   if (plain && ep.ug_mode == 1) return 1;
   if (plain && ep.ug_mode == 0) return 2;
   if (ep.gamma_mode == 2 && ep.ug_mode != 2) return 3;
-  return 0;
+  return plain ? 4 : 0;
 }
 
 // The planes of logit z scaled by sc (ug_sc: the scaled weight floor) and the
@@ -157,9 +158,10 @@ __device__ __forceinline__ void planes_of(float z, const ElemParams& ep, float s
       cn *= ep.an * (p * p);
       cp *= ep.ap * (q * q);
     }
-    if (EM == 1 || (EM == 3 && ep.ug_mode == 1)) {
+    if (EM == 1 || EM == 4 || (EM == 3 && ep.ug_mode == 1)) {
       // (|z| beyond 2^127 / 1.44: 0 x inf here, and a NaN leaves the floor)
-      const float h = __builtin_fmaf(-er, t, l2);
+      float h = __builtin_fmaf(-er, t, l2);
+      if constexpr (EM == 4) h = __builtin_amdgcn_exp2f(ep.ug * __builtin_amdgcn_logf(h));
       w = __builtin_amdgcn_fmed3f(h * sc, ug_sc, sc);
     } else {
       w = sc;
@@ -336,6 +338,7 @@ __device__ __forceinline__ void planes8(const float (&z)[8], const ElemParams& e
     case 1: cells(std::integral_constant<int, 1>()); break;
     case 2: cells(std::integral_constant<int, 2>()); break;
     case 3: cells(std::integral_constant<int, 3>()); break;
+    case 4: cells(std::integral_constant<int, 4>()); break;
     default: cells(std::integral_constant<int, 0>()); break;
   }
 }
