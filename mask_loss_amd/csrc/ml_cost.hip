@@ -42,8 +42,9 @@
 // columns 28.1 / 22.2 us (focal gamma 2, bf16 operands by its rule: 29.8), 33.6 M
 // against 4x targets 96 / 59, the 16- and 7-tile launches of 39 M 113 + 49 / 97 +
 // 40.  A range that is redone costs its formula pass again: 40% of 10 M logits
-// filled with -10^4, whole cost call 40.3 / 41.7 us (bf16 logits, in the table's
-// kernels: 54 / 56, against 4x targets 50 / 60).
+// filled with -10^4, whole cost call 41.4 / 42.9 us (float16 logits 40.0 / 39.5; bf16
+// ones, in the table's kernels, 45.0 / 43.4, against 4x targets 49.5 / 50.2).  Some logit
+// beyond 60 in every K-step (20 M of sigma 24): 76.6 / 86.3 us, 66.8 / 77.6 and 76.5 / 74.0.
 //
 // Work decomposition: one wave = 16 query rows of one image over a
 // contiguous range of 32-cell K-steps; each image is handled by the kernel
@@ -922,7 +923,8 @@ __device__ __forceinline__ void cost_wave(const CostArgs& a, int64_t lb, int64_t
       if constexpr (KEYS) tm = keys_of(x.lab, kp);
       float z[8], v[4][8];
       raw_to_f32<DT>(raw, z);
-      planes8<true>(z, ep, 1.f, k < nst ? 8 : tailn, unw, v, ub, up);
+      if ((TAB || !WIDE) && k < nst) planes8<false>(z, ep, 1.f, 8, unw, v, ub, up);
+      else planes8<true>(z, ep, 1.f, k < nst ? 8 : tailn, unw, v, ub, up);
       mma_wide(v, x, kp, tm);
     }
   }
@@ -1446,7 +1448,8 @@ __device__ __forceinline__ void cost_wave_pair(const CostArgs& a, int64_t lb, in
       if (k + 1 < nall) fetch(k + 1);
       float z[8], v[4][8], ub = 0.f, up = 0.f;
       raw_to_f32<ML_BF16>(raw, z);
-      planes8<true>(z, ep, 1.f, k < nst ? 8 : nv_of(full + (k - nst)), false, v, ub, up);
+      if (k < nst) planes8<false>(z, ep, 1.f, 8, false, v, ub, up);
+      else planes8<true>(z, ep, 1.f, nv_of(full + (k - nst)), false, v, ub, up);
       bf16x8_t A[4];
 #pragma unroll
       for (int pl = 0; pl < 4; ++pl) split_bf16<1>(v[pl], &A[pl]);
