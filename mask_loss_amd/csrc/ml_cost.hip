@@ -1096,9 +1096,9 @@ __global__ __launch_bounds__(64 * cost_waves(NT, TAB)) void cost_kernel(CostArgs
 // quads, KSq; the kernel runs 4 KSq K-ranges.
 //
 // Bound by vector-ALU issue (59 ops per K-step of 512 logits), LDS table reads and
-// load latency at 4 waves per SIMD: 210 M logits against label maps 102 -> 97 us
-// (bf16 operands took 65 ops per K-step), 671 M against u8 counts of 4x targets 314 us
-// (with the 7-tile class's 94 us; 886 + 208 us on the formula path).
+// load latency at 4 waves per SIMD: 210 M logits against label maps 106 -> 100 us
+// (traced; bf16 operands took 65 ops per K-step), 671 M against u8 counts of 4x targets
+// 314 - 333 us (with the 7-tile class's 94 us; 886 + 208 us on the formula path).
 //
 // LDS map of the 16-wave workgroup: positive table block [0, 8 kLutBlock), the
 // rings of waves 0 and 1 in the gap before the negative block at kLutNegOff,

@@ -324,8 +324,11 @@ __global__ __launch_bounds__(256) void prep_labels_kernel(PrepArgs a) {
 // store; other cells add their runs with LDS atomics.  8 maps of 1024 x 1024
 // at s = 4 with 61 rows: 22.6 us (67 MB read, 32 MB written, 4.4 TB/s; a copy
 // runs at 5.15), against 6.7 + 24.5 us for clearing the counts and adding to
-// them in memory pixel by pixel.
-constexpr size_t kCntLds = 40 * 1024;  // of the rows in LDS: three workgroups per CU
+// them in memory pixel by pixel; 38 us where the labels come from HBM (in a step
+// whose other kernels push them out of the last-level cache).
+// Rows in LDS: the 16 waves of a 1024-thread workgroup let two share a CU (the
+// 8 of the s = 2 form four, by waves and by this limit).
+constexpr size_t kCntLds = 40 * 1024;
 template <int S>
 constexpr int kCellThreads = S == 2 ? 2 : 4;
 template <int CW, int S>
