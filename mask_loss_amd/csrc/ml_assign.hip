@@ -1065,7 +1065,9 @@ __global__ __launch_bounds__(256) void assign_kernel(AssignArgs a) {
             const int c = t < nv ? vcols[t] : 0;
             const bool open = t < nv && cap[c] > 0;
             const uint64_t m = __ballot(open);
-            if (open) hrows[M + __popcll(m & ((1ull << lane) - 1ull))] = c;
+            // the first nrem open columns are this round's rows (hrows holds Q of them)
+            const int at = M + __popcll(m & ((1ull << lane) - 1ull));
+            if (open && at < nrem) hrows[at] = c;
             M += __popcll(m);
           }
           if (M == 0 || nrem == 0) break;

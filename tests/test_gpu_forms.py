@@ -50,6 +50,14 @@ def test_upstream_gradient_strides(ml, dtype, form):
 
 
 @pytest.mark.parametrize("strategy", [0, 1, 2, 3])
+@pytest.mark.parametrize("K,G,Q", [(1, 7, 5), (1, 70, 5), (2, 130, 33), (4, 100, 64), (2, 250, 17), (1, 31, 1)])
+def test_strategies_with_more_columns_than_queries(ml, strategy, K, G, Q):
+    """Only the first Q open columns are rows of an assignment; the lists in LDS
+    hold no more."""
+    test_strategies_with_many_columns(ml, strategy, K, G, Q)
+
+
+@pytest.mark.parametrize("strategy", [0, 1, 2, 3])
 @pytest.mark.parametrize("K,G,Q", [(1, 70, 200), (2, 70, 100), (3, 130, 150), (2, 3, 40)])
 def test_strategies_with_many_columns(ml, strategy, K, G, Q):
     z, t, zc, ct = inputs(2, 1, 2, Q, 24, 24, G, 6)
