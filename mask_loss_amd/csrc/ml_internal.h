@@ -71,7 +71,7 @@ constexpr int64_t kCostSlots = 4096;
 // the widest class's assignment (at most one per image, at most 1/8 of them)
 constexpr int kSideCUs = 16;
 
-// Planes of class ci's partial tile (see ml_cost.hip): bce numerator, I, T of
+// Planes of class ci's partial tile (see ml_cost.h): bce numerator, I, T of
 // every column slot, slot G of an image with G non-empty columns being the ones
 // column (class 0); or the slot sums N, Pos, I, T, slot G holding the pixels of
 // no column.
@@ -241,7 +241,7 @@ Layout make_layout(const Dims& d, bool force_masks, const CostPlan& pl);
 Layout make_layout(const Dims& d, bool force_masks);  // with bound_cost_plan(d)
 // Plan slots / offsets of the cost launches (queries kernel occupancy on the
 // current device; the workspace bound uses kCostSlots only).
-// How a call's contraction forms its operands (see ml_cost.hip).
+// How a call's contraction forms its operands (see ml_cost.h).
 struct CostForm {
   bool tab;   // bf16 logits: per-cell planes from the LDS table
   bool wide;  // bf16 operands throughout: the planes may get small at any logit
